@@ -7,6 +7,7 @@
 namespace llz {
 
 typedef float llz_f4v __attribute__((ext_vector_type(4)));  // four floats as one 16-byte access
+typedef float llz_f4u __attribute__((ext_vector_type(4), aligned(4)));  // the same from any 4-byte aligned address
 
 constexpr int kCandCap = 2048;  // candidate list capacity per row (power of two)
 constexpr int kPenMax = 64;     // fused repetition penalty: window entries at most (one per lane)

@@ -49,24 +49,93 @@ __global__ __launch_bounds__(kMaxNT) void k_penalty(const float* __restrict__ lo
 }
 
 // ---------------------------------------------------------------------------
-// k_argmax: one workgroup per row.
+// k_argmax: sampleArgmax (sampler.zig:31-41) of the post-processed rows, each
+// row cut into `chunks` runs of consecutive logits, one workgroup each.
+//
+// The reference's scan keeps the first strict maximum; a NaN never wins,
+// except at index 0, where it is never replaced.  That is the largest key
+// under (value, lower index first) with NaN below everything and index 0's
+// NaN above it, so chunks combine in any order.  They combine through the
+// row's token word itself, with no scratch memory: a workgroup reads the
+// word, and while its own best beats the element the word names it swaps its
+// index in.  The word needs no initialisation: what an earlier call left
+// there is either not an index of the row (any element beats it) or names a
+// real element of it, which the row's best beats or equals.
+//
+// Bound by HBM latency and launch: a workgroup per row with one 4-byte load
+// in flight per thread took 19.9 us for 32 x 50021 (0.32 TB/s); chunks of at
+// least kArgChunk logits over up to kArgGroups workgroups, four 16-byte loads
+// in flight per thread, take 10.5 us of kernel where that took 21.3 (traced).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kNT) void k_argmax(const float* __restrict__ logits, int64_t stride,
-                                                int n, uint32_t xf, float cap, float inv_scale,
-                                                uint32_t* __restrict__ tokens,
-                                                uint8_t* __restrict__ consumed,
-                                                uint32_t* __restrict__ kept_count,
-                                                uint32_t* __restrict__ path) {
-  __shared__ WgScratch<kNT> sh;
-  int bank = 0;
-  const int row = blockIdx.x;
-  const RowSrc x{logits + (int64_t)row * stride, xf & ~kXfPen, cap, inv_scale, 1.0f, nullptr};
-  const uint32_t tok = wg_argmax_row<kNT>(x, n, sh, bank);
+constexpr int kArgNT = 256;
+constexpr int kArgUnroll = 4;                            // float4 loads in flight per thread
+constexpr int kArgStep = kArgNT * 4 * kArgUnroll;        // logits per loop step of a workgroup
+constexpr int kArgChunk = kArgStep;                      // logits per chunk at least
+constexpr int kArgGroups = 1024;                         // workgroups aimed at (four per CU)
+
+// The order of sampleArgmax as an unsigned key (larger wins).
+__device__ __forceinline__ uint64_t amax_key(float v, uint32_t i) {
+  const uint32_t b = __float_as_uint(v + 0.0f);  // -0 and +0 are one value
+  const uint32_t o = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
+  const uint32_t k = v != v ? (i == 0u ? 0xffffffffu : 0u) : o;
+  return ((uint64_t)k << 32) | (uint32_t)~i;
+}
+
+__global__ __launch_bounds__(kArgNT) void k_argmax(const float* __restrict__ logits, int64_t stride,
+                                                   int n, int chunks, int per_chunk, uint32_t xf, float cap,
+                                                   float inv_scale, uint32_t* __restrict__ tokens,
+                                                   uint8_t* __restrict__ consumed, uint32_t* __restrict__ kept_count,
+                                                   uint32_t* __restrict__ path) {
+  __shared__ uint64_t best[kArgNT / kWave];
+  const int row = (int)(blockIdx.x / (unsigned)chunks), c = (int)(blockIdx.x % (unsigned)chunks);
+  const float* x = logits + (int64_t)row * stride;
+  const int p0 = c * per_chunk, p1 = min(n, p0 + per_chunk);  // chunks divide the row: p0 < n
+  uint64_t bk = 0ull;  // below every element's key
+  if (p1 - p0 >= 4) {
+    // starts past the chunk's last four logits are moved back to them: an
+    // element read twice changes no maximum, and no load needs a branch
+    for (int base = p0; base < p1; base += kArgStep) {
+      llz_f4u v[kArgUnroll];
+      uint32_t pos[kArgUnroll];
+#pragma unroll
+      for (int u = 0; u < kArgUnroll; ++u) {
+        pos[u] = (uint32_t)min(base + (u * kArgNT + (int)threadIdx.x) * 4, p1 - 4);
+        v[u] = *reinterpret_cast<const llz_f4u*>(x + pos[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kArgUnroll; ++u)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) bk = max(bk, amax_key(logit_post(v[u][k], xf, cap, inv_scale), pos[u] + (uint32_t)k));
+    }
+  } else {
+    for (int i = p0 + (int)threadIdx.x; i < p1; i += kArgNT)
+      bk = max(bk, amax_key(logit_post(x[i], xf, cap, inv_scale), (uint32_t)i));
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) bk = max(bk, (uint64_t)__shfl_xor((unsigned long long)bk, m, kWave));
+  if (lane_id() == 0) best[wave_id()] = bk;
+  __syncthreads();
   if (threadIdx.x == 0) {
-    tokens[row] = tok;
-    if (consumed) consumed[row] = 0;
-    if (kept_count) kept_count[row] = 0;
-    if (path) path[row] = 0;
+#pragma unroll
+    for (int w = 1; w < kArgNT / kWave; ++w) bk = max(bk, best[w]);
+    const uint32_t mine = ~(uint32_t)bk;
+    if (chunks == 1) {
+      tokens[row] = mine;
+    } else {
+      uint32_t cur = __hip_atomic_load(&tokens[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // each failed exchange means another chunk's better or worse index
+      // came in between: at most one per chunk
+      while (cur >= (uint32_t)n || bk > amax_key(logit_post(x[cur], xf, cap, inv_scale), cur)) {
+        if (__hip_atomic_compare_exchange_strong(&tokens[row], &cur, mine, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+          break;
+      }
+    }
+    if (c == 0) {
+      if (consumed) consumed[row] = 0;
+      if (kept_count) kept_count[row] = 0;
+      if (path) path[row] = 0;
+    }
   }
 }
 
@@ -151,8 +220,13 @@ hipError_t launch_penalty(const float* logits, int64_t stride, int rows, int n, 
 hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, uint32_t xf, float cap,
                          float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
                          uint32_t* path, hipStream_t st) {
-  hipLaunchKernelGGL(k_argmax, dim3(rows), dim3(kNT), 0, st, logits, stride, n, xf, cap, inv_scale, tokens,
-                     consumed, kept_count, path);
+  // chunks per row: as many as fill kArgGroups workgroups, none below kArgChunk logits
+  const int most = std::max(1, (n + kArgChunk - 1) / kArgChunk);
+  const int want = std::min(most, std::max(1, kArgGroups / rows));
+  const int per = ((n + want - 1) / want + 3) & ~3;
+  const int chunks = (n + per - 1) / per;
+  hipLaunchKernelGGL(k_argmax, dim3((unsigned)rows * (unsigned)chunks), dim3(kArgNT), 0, st, logits, stride, n, chunks,
+                     per, xf, cap, inv_scale, tokens, consumed, kept_count, path);
   return hipGetLastError();
 }
 
