@@ -751,7 +751,7 @@ __device__ __noinline__ NormResult select_norm_fallback(const KArgs* A, int row,
 
 template <class Src>
 __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenShared* pen, SampleShared& sh,
-                                             int bank, float m, float S, uint32_t path);
+                                             int bank, float m, float S, uint32_t path, int wslot);
 
 constexpr int kShortMax = 256;  // longest candidate list of the short path
 
@@ -1031,7 +1031,7 @@ template <class Src, class OSrc>
 __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q, SampleShared& sh, float m,
                                            float S, uint32_t cc_in, bool uncertified, float u_row, bool pre_ok,
                                            uint64_t cand_pre, uint32_t cand_n0, const Src& X, const OSrc& O,
-                                           const PenShared* pen, const KArgs* A, int row) {
+                                           const PenShared* pen, const KArgs* A, int row, int wslot) {
   int bank = 0;
   const int t = (int)threadIdx.x;
   const int n = P.n;
@@ -1129,7 +1129,7 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
   const bool ovf = cc > (uint32_t)kCap;
   const int c = ovf ? kCap : (int)cc;
   if (!ovf && c <= kShortMax && !(P.typical_p > 0.0f && P.typical_p < 1.0f)) {
-    if (!select_short(Pl, Q, row, sh, c, m, S, path, u_row)) select_full_row<Src>(A, row, pen, sh, bank, m, S, path);
+    if (!select_short(Pl, Q, row, sh, c, m, S, path, u_row)) select_full_row<Src>(A, row, pen, sh, bank, m, S, path, wslot);
     return;
   }
   const int csort = next_pow2(c);
@@ -1238,7 +1238,7 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
   }
 
   // ---- full-row fallback: every probability, stable radix sort, filters
-  select_full_row<Src>(A, row, pen, sh, bank, m, S, path);
+  select_full_row<Src>(A, row, pen, sh, bank, m, S, path, wslot);
 }
 
 // The full-row fallback of k_select: every probability, stable radix sort of
@@ -1322,7 +1322,6 @@ __device__ TypicalHead typical_head(const Src& X, int n, float m, float S, float
       const uint32_t gpk = wg_min_u32<kNT>(bpk, sh.wg, bank);
       r.first = wg_min_u32<kNT>(bpk == gpk ? bid : 0xffffffffu, sh.wg, bank);
     }
-    __threadfence();
     __syncthreads();
     // ---- 2. the head's last bucket (wave 0: 32 buckets per lane)
     if (wave_id() == 0) {
@@ -1371,11 +1370,9 @@ __device__ TypicalHead typical_head(const Src& X, int n, float m, float S, float
       }
       C += (int)wg_sum_sat<kNT>(cnt, 0x7fffffffu, sh.wg, bank);
     }
-    __threadfence();
     __syncthreads();
     // ---- 4. sorted by key, then the exact cumulative sum
     wg_radix_sort_pairs<kNT>(Ck, Cv, Bk, Bv, C, sh.u.post.radix);
-    __threadfence();
     __syncthreads();
     int st;
     list_accumulate<kNT, 2, false>(
@@ -1460,7 +1457,6 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   const uint32_t gk = wg_min_u32<kNT>(fk, sh.wg, bank);
   const uint32_t first = wg_min_u32<kNT>(fk == gk ? fid : 0xffffffffu, sh.wg, bank);  // indices[0]
   const uint32_t Lw = min(Kk, km);  // positions top-k and min-p keep
-  __threadfence();
   __syncthreads();
   for (int b = t; b < kNB; b += kNT) hist_unpack(bs.hist[bix(b)], coarse_Etop(b), bs.cnt[bix(b)], bs.mass[bix(b)]);
   __syncthreads();
@@ -1595,7 +1591,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
 
 template <class Src>
 __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenShared* pen, SampleShared& sh,
-                                             int bank, float m, float S, uint32_t path) {
+                                             int bank, float m, float S, uint32_t path, int wslot) {
   const RowParams& P = A->P;
   const RowPtrs& Q = A->Q;
   const Src X = make_src<Src>(P, Q, row, pen);
@@ -1617,35 +1613,44 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
     }
     return;
   }
-  // one of the call's fb_slots buffer sets, claimed for this row: a slot is
+  // The row's buffer set.  With a set per workgroup of the grid, workgroup
+  // wslot keeps set wslot for all its rows: nothing is handed between
+  // workgroups, so nothing is claimed, and the buffers' writes need ordering
+  // within the workgroup only (__syncthreads).  (The claim and its agent-scope
+  // fences, which write back the XCD's L2, took 12-44 us per row.)
+  // With fewer sets (P.fb_slots < P.grid) a row claims one: a slot is
   // free for this call when its owner word holds anything but this call's
   // epoch.  At most fb_slots rows hold one at a time; a row that finds none
   // waits for a holder (a running workgroup that needs nothing else) to
   // release one.  The fences make the previous holder's writes, possibly
   // from another XCD's L2, land before this row touches the buffers.
-  if (t == 0) {
-    const unsigned long long E = P.epoch;
-    int got = -1;
-    for (uint32_t spin = 0; got < 0 && spin < (1u << 20); ++spin) {
-      for (int k = 0; k < P.fb_slots && got < 0; ++k) {
-        const int s = (row + k) % P.fb_slots;
-        const unsigned long long old = __hip_atomic_load(&Q.fb_owner[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (old != E && atomicCAS(&Q.fb_owner[s], old, E) == old) got = s;
-      }
-      if (got < 0) __builtin_amdgcn_s_sleep(127);
-    }
-    __threadfence();
-    sh.misc[1] = (uint32_t)got;
-  }
-  __syncthreads();
-  const int slot = (int)sh.misc[1];
-  if (slot < 0 || slot >= P.fb_slots) {  // no slot within the wait bound
+  const bool own_set = P.fb_slots >= P.grid;
+  int slot = wslot;
+  if (!own_set) {
     if (t == 0) {
-      Q.tokens[row] = 0xffffffffu;
-      if (Q.consumed) Q.consumed[row] = 0;
-      if (Q.status) Q.status[row] = path | kPathError;
+      const unsigned long long E = P.epoch;
+      int got = -1;
+      for (uint32_t spin = 0; got < 0 && spin < (1u << 20); ++spin) {
+        for (int k = 0; k < P.fb_slots && got < 0; ++k) {
+          const int s = (row + k) % P.fb_slots;
+          const unsigned long long old = __hip_atomic_load(&Q.fb_owner[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (old != E && atomicCAS(&Q.fb_owner[s], old, E) == old) got = s;
+        }
+        if (got < 0) __builtin_amdgcn_s_sleep(127);
+      }
+      __threadfence();
+      sh.misc[1] = (uint32_t)got;
     }
-    return;
+    __syncthreads();
+    slot = (int)sh.misc[1];
+    if (slot < 0 || slot >= P.fb_slots) {  // no slot within the wait bound
+      if (t == 0) {
+        Q.tokens[row] = 0xffffffffu;
+        if (Q.consumed) Q.consumed[row] = 0;
+        if (Q.status) Q.status[row] = path | kPathError;
+      }
+      return;
+    }
   }
   LLZ_STAMP(row, 8);
   const int64_t fo = (int64_t)slot * n;
@@ -1666,10 +1671,10 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
   // release the slot once every thread is done with it (a value no later
   // call's epoch takes)
   auto release = [&]() {
-    __threadfence();
+    if (!own_set) __threadfence();
     __syncthreads();
     LLZ_STAMP(row, 14);
-    if (t == 0) atomicExch(&Q.fb_owner[slot], P.epoch ^ (1ull << 63));
+    if (!own_set && t == 0) atomicExch(&Q.fb_owner[slot], P.epoch ^ (1ull << 63));
   };
   // Without typical-p the kept prefix, the total and the draw come from
   // buckets of the p keys (llz_bucket.h), without a sort of the row.  The
@@ -1722,11 +1727,9 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
       }
     }
     kmin = wg_min_u32<kNT>(kmin, sh.wg, bank);
-    __threadfence();
     __syncthreads();
     LLZ_STAMP(row, 9);
     wg_radix_sort_pairs<kNT>(Ak, Av, Bk, Bv, n, sh.u.post.radix, kmin);
-    __threadfence();
     __syncthreads();
     LLZ_STAMP(row, 10);
     K = prefix_filters(GL, n, kInf, n, P, S, sh, bank);  // M = n: never -1
@@ -1789,7 +1792,6 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
         const uint32_t id = GL.id(q);
         mask[q] = (!cut || dk < dkc || (dk == dkc && id < idc)) ? 1 : 0;
       }
-      __threadfence();
       __syncthreads();
       finish(GL, K, [&](int q) { return mask[q] != 0; }, 0xffffffffu);
     } else {
@@ -1818,13 +1820,10 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
           Ak[d] = id;
           Av[d] = ~__float_as_uint(p);
         }
-        __threadfence();
         __syncthreads();
         wg_radix_sort_pairs<kNT>(Ak, Av, Bk, Bv, keep_n, sh.u.post.radix);
-        __threadfence();
         __syncthreads();
         wg_radix_sort_pairs<kNT>(Av, Ak, Bk, Bv, keep_n, sh.u.post.radix);
-        __threadfence();
         __syncthreads();
         finish(GlobalList{Av, Ak}, keep_n, [&](int) { return true; }, th.first);
       }

@@ -1823,7 +1823,8 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // walk's results, lie past F.u): no barrier here
   static_assert(sizeof(SampleShared) <= sizeof(F.u), "the selection's memory must lie inside F.u");
   select_row(P, Q, U.select, m, certified ? S : 0.0f, certified ? cc : 0u, !certified, u_row, certified && pre_ok,
-             cand_pre, cand_n0, X, O, XF ? &pen_sh : nullptr, kernel_args_ptr(), row);
+             cand_pre, cand_n0, X, O, XF ? &pen_sh : nullptr, kernel_args_ptr(), row,
+             wslot);
   LLZ_STAMP(row, 15);
   // the walk's diagnostics join the status thread 0 wrote (F.diag lies past
   // the selection's memory)
