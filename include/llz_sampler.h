@@ -108,8 +108,8 @@ enum {
     LLZ_PATH_TOKEN_ONLY = 128,   /* the token decided without the exact normaliser (calls    */
                                  /*   asking for neither probabilities nor row statistics)  */
     LLZ_PATH_DECLINE_SHIFT = 8,  /* bits 8-15: the bucket path's decline reason (see above)  */
-    LLZ_PATH_RECOLLECT = 1 << 16, /* a flooded candidate list collected again, its largest  */
-                                 /*   terms only, so the selection ran on a list            */
+    LLZ_PATH_RECOLLECT = 1 << 16, /* the candidate list holds the largest terms only: above */
+                                 /*   a raised threshold, or collected again after it flooded */
     LLZ_PATH_SPLIT = 1 << 17,    /* with LLZ_PATH_TOKEN_ONLY: the row was read by several   */
                                  /*   workgroups, one chunk each (calls of few rows)       */
     LLZ_PATH_ERROR = (int)0x80000000u

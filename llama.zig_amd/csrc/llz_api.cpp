@@ -348,14 +348,14 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
     if (cus <= 0) return LLZ_E_HIP;
     P.grid = std::min(std::min(rows, cus), kMaxGrid);
   }
-  // Split rows: a token-only call of at most kSplitRows plain, 16-byte
-  // aligned rows reads each row with S workgroups of one chunk each (the
+  // Split rows: a token-only call of at most kSplitRows plain rows
+  // reads each row with S workgroups of one chunk each (the
   // smallest chunk, 2048 nv logits, whose rows x S workgroups fit the CUs at
   // once), where one workgroup per row would leave most CUs idle.
   // Rows read through post-processing or the fused penalty take chunks of at
   // most 2 float4 per thread: each logit's exact transform is then a few per
   // thread (calls of up to 8 rows at 128k vocab).
-  if (split_room && tok_only && !typical_on && vec && vocab % 4 == 0 && P.tok_theta > 0.0f && P.l2e_t > 0.0f &&
+  if (split_room && tok_only && !typical_on && P.tok_theta > 0.0f && P.l2e_t > 0.0f &&
       P.l2e_t <= 0x1p40f && g_split_mode.load(std::memory_order_relaxed) != 1) {
     const int cus = device_cus(st);
     const int nv_max = (xf_src | xb) != 0u ? 2 : kSplitNV;

@@ -62,7 +62,7 @@
 
 namespace llz {
 namespace fastp {
-constexpr int NT = 512;
+constexpr int NT = kStatsNT;
 constexpr int W = NT / kWave;       // 8 waves
 constexpr int SEG = 256;            // elements per segment: one float4 per lane
 constexpr int KV = 45;              // register-resident segments per wave
@@ -136,8 +136,7 @@ struct FastShared {
   float cw[fastp::W];
   float bw[fastp::W];       // per wave: |aw|, the R_w argument's magnitude (error bound)
   uint32_t nanw[fastp::W];
-  float wtot[fastp::W];     // per wave: sum of its scaled segment sums
-  uint32_t wflag[fastp::W]; //   bit 0: not certifiable, bit 1: candidate flood
+  uint32_t wflag[fastp::W]; // per wave: its estimates above the candidate threshold tried
   int wnex[fastp::W];       //   number of its EXACT segments
   uint32_t ncand;
   int nslot;      // EXACT slots in use this round
@@ -150,7 +149,7 @@ struct FastShared {
   uint32_t diag;  // kPathWalkRounds / kPathResolveGeneric (diagnostics for the row's status)
   float qsum[fastp::W];  // token-only rows: per wave, the sum of its estimates q
   float tx[fastp::W];    // token-only typical-p rows: per wave, sum of q (log2 q + aw)
-  float txa[fastp::W];   //   and of its terms' magnitudes
+  float txa[fastp::W];   //   and of its terms' magnitudes; later its sums in all and above a threshold
   float theta2;          // token-only rows: the threshold of a list collected again
   float qwsum[fastp::W];  // token-only rows: per wave, its segments' sums of q times n - their first position
   uint32_t tcand; // token-only rows: candidates collected
@@ -221,18 +220,6 @@ __device__ __forceinline__ float4 buf_ld4(llz_i4v rsrc, int voffset, int soffset
 __device__ __forceinline__ float4 ld_nt4(const float* p) {
   const llz_f4v v = __builtin_nontemporal_load(reinterpret_cast<const llz_f4v*>(p));
   return make_float4(v.x, v.y, v.z, v.w);
-}
-
-// Segment load: a full, 16-byte aligned segment as one float4 per lane;
-// otherwise per element, absent positions (>= n) as -inf.
-__device__ __forceinline__ float4 ld_seg(const float* xr, int pos, int n, bool vec) {
-  if (vec && pos + 4 <= n) return ld_nt4(xr + pos);
-  float4 v;
-  v.x = pos + 0 < n ? xr[pos + 0] : -__builtin_inff();
-  v.y = pos + 1 < n ? xr[pos + 1] : -__builtin_inff();
-  v.z = pos + 2 < n ? xr[pos + 2] : -__builtin_inff();
-  v.w = pos + 3 < n ? xr[pos + 3] : -__builtin_inff();
-  return v;
 }
 
 __device__ __forceinline__ float wave_sum_f32(float v) {

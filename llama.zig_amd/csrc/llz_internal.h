@@ -32,7 +32,7 @@ constexpr int kSplitRows = 64;
 
 // RowParams.flags
 constexpr uint32_t kFlagTIsOne = 1u;    // temperature == 1.0f exactly: (v - m) / T == v - m
-constexpr uint32_t kFlagVecSrc = 2u;    // 16-byte loads are legal on the rows the chain reads
+constexpr uint32_t kFlagVecSrc = 2u;    // the rows the chain reads are 16-byte aligned
 constexpr uint32_t kFlagFallback = 4u;  // the full-row fallback buffers are present
 constexpr uint32_t kFlagTokenOnly = 8u;  // no probabilities or row statistics requested: the token alone
 constexpr uint32_t kFlagXfExact = 16u;   // transformed rows the single pass cannot estimate: the exact streaming path
@@ -57,7 +57,8 @@ constexpr uint32_t kPathWalkRounds = 16u;    // diagnostic: the walk took more t
 constexpr uint32_t kPathResolveGeneric = 32u;  // diagnostic: an event beyond a segment's tabulated grids
 constexpr uint32_t kPathTokenOnly = 128u;     // the token certified without the exact normaliser
 constexpr uint32_t kPathBuckets = 64u;        // full row without a sort: kept prefix, total and draw by p-key buckets
-constexpr uint32_t kPathRecollect = 1u << 16;  // a flooded candidate list collected again (its largest terms)
+constexpr uint32_t kPathRecollect = 1u << 16;  // the candidate list holds its largest terms only (raised threshold, or
+                                               //   collected again after it flooded)
 constexpr uint32_t kPathSplit = 1u << 17;      // token-only row finished from chunks read by several workgroups
 constexpr uint32_t kPathError = 0x80000000u;
 
@@ -68,7 +69,7 @@ constexpr uint32_t kPathError = 0x80000000u;
 constexpr int kStampRows = 4096;
 constexpr int kStampSlots = 60;
 #ifdef LLZ_PHASE_STAMPS
-static __device__ unsigned long long llz_phase_stamps[kStampRows * kStampSlots];  // read by llz_stats.hip's copy-out
+static __device__ unsigned long long llz_phase_stamps[kStampRows * kStampSlots];  // read by its object's copy-out
 #define LLZ_STAMP(row, k)                                                                     \
   do {                                                                                        \
     if (threadIdx.x == 0 && (row) < ::llz::kStampRows)                                        \
@@ -161,6 +162,8 @@ struct KArgs {
   RowParams P;
   RowPtrs Q;
 };
+typedef void (*StatsKernel)(KArgs);
+constexpr int kStatsNT = 512;  // threads of its workgroups
 
 hipError_t launch_penalty(const float* logits, int64_t stride, int rows, int n, const uint32_t* prev,
                           int n_prev, int64_t prev_stride, int window, float penalty, uint32_t xf, float cap,

@@ -1,5 +1,5 @@
 // llz_kernels.hip -- MI355X (gfx950) kernels around the fused sampling kernel
-// (llz_stats.hip):
+// (llz_stats.h):
 //   k_penalty     (optional) penalised copy of the rows   sampler.zig:54-75
 //   k_math_probe  the device exp/log/expm1/tanh (parity tests)
 //   k_argmax      greedy rows (temperature <= 0)          sampler.zig:31-41,50

@@ -83,6 +83,28 @@ __device__ uint32_t wg_argmax_row(const Src& x, int n, WgScratch<NT>& sh, int& b
   return ri;
 }
 
+// Four logits from position pos of a row of any length and alignment,
+// without a branch per lane (so that every load of a wave can be in flight at
+// once): a start within the row's last three positions reads the row's last
+// four and shifts them; positions >= n are -inf.
+__device__ __forceinline__ float4 rd4_any(const float* xr, int pos, int n) {
+  float4 v;
+  if (n < 4) {
+    v.x = pos + 0 < n ? xr[pos + 0] : -kInf;
+    v.y = pos + 1 < n ? xr[pos + 1] : -kInf;
+    v.z = pos + 2 < n ? xr[pos + 2] : -kInf;
+    v.w = pos + 3 < n ? xr[pos + 3] : -kInf;
+    return v;
+  }
+  const int pc = min(pos, n - 4), off = pos - pc;
+  const llz_f4u r = __builtin_nontemporal_load(reinterpret_cast<const llz_f4u*>(xr + pc));
+  v.x = off == 0 ? r.x : (off == 1 ? r.y : (off == 2 ? r.z : (off == 3 ? r.w : -kInf)));
+  v.y = off == 0 ? r.y : (off == 1 ? r.z : (off == 2 ? r.w : -kInf));
+  v.z = off == 0 ? r.z : (off == 1 ? r.w : -kInf);
+  v.w = off == 0 ? r.w : -kInf;
+  return v;
+}
+
 // e_i = exp((v_i - max) / T) as sampler.zig:85 evaluates it.
 __device__ __forceinline__ float row_exp(float v, float m, float T, bool t_is_one) {
   float x = v - m;

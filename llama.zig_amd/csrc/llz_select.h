@@ -250,7 +250,6 @@ __device__ float row_normaliser(const Src& X, int n, const RowParams& P, SampleS
   NormShared<kNT>& ns = sh.u.norm;
   const int lane = lane_id(), w = wave_id();
   const bool t1 = (P.flags & kFlagTIsOne) != 0;
-  const bool vec = (P.flags & kFlagVecSrc) != 0;
   const int p0 = min(n, kPrologue);
 
   // independent loads first: the max partials, the prologue's logits and the
@@ -259,7 +258,7 @@ __device__ float row_normaliser(const Src& X, int n, const RowParams& P, SampleS
   const float vp = (w == 0 && lane < p0) ? X.at(lane) : 0.0f;
   float vcur[kSub][kV], vnext[kSub][kV];
 #pragma unroll
-  for (int c = 0; c < kSub; ++c) X.load4(p0 + w * kSlice + c * (kWave * kV) + lane * kV, n, vec, vcur[c]);
+  for (int c = 0; c < kSub; ++c) X.load4(p0 + w * kSlice + c * (kWave * kV) + lane * kV, n, vcur[c]);
   const float m = wg_fmax<kNT>(mp, sh.wg, bank);
   m_out = m;
 
@@ -284,7 +283,7 @@ __device__ float row_normaliser(const Src& X, int n, const RowParams& P, SampleS
     if (gb + GE < n) {
 #pragma unroll
       for (int c = 0; c < kSub; ++c)
-        X.load4(gb + GE + w * kSlice + c * (kWave * kV) + lane * kV, n, vec, vnext[c]);
+        X.load4(gb + GE + w * kSlice + c * (kWave * kV) + lane * kV, n, vnext[c]);
     }
     uint32_t* part = ns.part[pb];
     const int sb = gb + w * kSlice;
@@ -490,8 +489,7 @@ struct RowTilesT {
   int n;
   bool vec8;
   int nlast;
-  __device__ RowTilesT(const float* x, int n_, bool vec) : xs(x), n(n_), vec8(vec && n_ >= V),
-                                                          nlast(vec && n_ >= V ? ((n_ - V) & ~3) : 0) {}
+  __device__ RowTilesT(const float* x, int n_) : xs(x), n(n_), vec8(n_ >= V), nlast(n_ >= V ? ((n_ - V) & ~3) : 0) {}
   // the row through a global-address-space pointer: the callers run out of
   // line, where a generic pointer would make these flat loads, which count
   // on the LDS counter too (every LDS wait would wait for them)
@@ -503,7 +501,7 @@ struct RowTilesT {
       const int pc = min(pos, nlast);
 #pragma unroll
       for (int h = 0; h < V / 4; ++h) {
-        const llz_f4v q = *(const __attribute__((address_space(1))) llz_f4v*)(g() + pc + 4 * h);
+        const llz_f4u q = *(const __attribute__((address_space(1))) llz_f4u*)(g() + pc + 4 * h);
         r[4 * h + 0] = q.x; r[4 * h + 1] = q.y; r[4 * h + 2] = q.z; r[4 * h + 3] = q.w;
       }
     } else {
@@ -574,11 +572,10 @@ __device__ __noinline__ EntropyResult entropy_pass(Src X, int n, float m, float 
   constexpr float LN2 = 6.93147182e-1f;     // RN(ln 2)
   constexpr float EPS = 24.0f * 0x1p-23f;
   const bool t1 = (flags & kFlagTIsOne) != 0;
-  const bool vec = (flags & kFlagVecSrc) != 0;
   const float rS = 1.0f / S;
   const int t = (int)threadIdx.x;
 
-  const RowTilesT<EV> rt(X.x, n, vec);
+  const RowTilesT<EV> rt(X.x, n);
   // sampler.zig:85 and :131 on one argument x; the term is +0 when p == 0
   auto exact_term = [&](float x) {
     const float p = exp_f32(x) / S;
@@ -789,7 +786,6 @@ __device__ __noinline__ float recollect_top(const Src X, int n, float m, float S
   float* hsum = reinterpret_cast<float*>(sh.u.post.radix.stage_v);
   const int t = (int)threadIdx.x;
   const bool t1 = (flags & kFlagTIsOne) != 0;
-  const bool vec = (flags & kFlagVecSrc) != 0;
   // D: T ln(1/theta) from the hardware log2 (within an ulp), with 2^-10 to spare
   const float D = T * (-__builtin_amdgcn_logf(theta)) * 0.693147182f * (1.0f + 0x1p-10f);
   if (!(D > 0.0f) || !(D < 3.0e38f)) return -1.0f;
@@ -799,7 +795,7 @@ __device__ __noinline__ float recollect_top(const Src X, int n, float m, float S
     hsum[b] = 0.0f;
   }
   lds_barrier();
-  const RowTiles8 rt(X.x, n, vec);
+  const RowTiles8 rt(X.x, n);
   float raw[EV];
   // ---- 1. the histogram (d < D: NaN and -inf logits never enter)
   rt.load(t * EV, raw);
@@ -1026,12 +1022,13 @@ __device__ __forceinline__ bool select_short(const RowParams& P, const RowPtrs& 
 // certify, from the streaming normaliser.  Every thread of the workgroup
 // calls it; `sh` may alias the caller's shared memory once all of it is read.
 // pre_ok: thread 64 + i holds candidate i in cand_pre for i < cand_n0, and
-// cc_in <= 448 (the later ones are read here).
+// cc_in <= 448 (the later ones are read here).  theta_c: the threshold k_stats
+// collected the candidates with (cand_theta or above).
 template <class Src, class OSrc>
 __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q, SampleShared& sh, float m,
                                            float S, uint32_t cc_in, bool uncertified, float u_row, bool pre_ok,
                                            uint64_t cand_pre, uint32_t cand_n0, const Src& X, const OSrc& O,
-                                           const PenShared* pen, const KArgs* A, int row, int wslot) {
+                                           const PenShared* pen, const KArgs* A, int row, int wslot, float theta_c) {
   int bank = 0;
   const int t = (int)threadIdx.x;
   const int n = P.n;
@@ -1105,9 +1102,14 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
   // ---- 4. candidates -> probabilities -> (p desc, id asc) (:90-100)
   lds_barrier();
   uint32_t cc = sh.cand_count;
-  // the list's threshold for the certified prefix: cand_theta, or the bound
-  // of a list collected again (recollect_top) after it flooded
+  // the list's threshold for the certified prefix: the one it was collected
+  // with (theta_c; the streaming normaliser collects with cand_theta), or the
+  // bound of a list collected again (recollect_top) after it flooded
   RowParams Pl = P;
+  if (!uncertified) {
+    Pl.cand_theta = theta_c;
+    if (theta_c > P.cand_theta) path |= kPathRecollect;
+  }
   // only where a filter can end the kept prefix inside the list: top-p, or a
   // top-k within three quarters of it (min-p alone keeps every flooded term)
   const bool bounded = (P.top_p > 0.0f && P.top_p < 1.0f) || (P.top_k > 0u && P.top_k <= (uint32_t)(kCap - kCap / 4) / 2u);
@@ -1278,7 +1280,6 @@ __device__ TypicalHead typical_head(const Src& X, int n, float m, float S, float
   constexpr int TV = 8;     // elements per thread per tile
   const int t = (int)threadIdx.x;
   const bool t1 = (P.flags & kFlagTIsOne) != 0;
-  const bool vec = (P.flags & kFlagVecSrc) != 0;
   uint32_t* hcnt = sh.u.post.radix.stage_k;                        // [HB]
   float* hsum = reinterpret_cast<float*>(sh.u.post.radix.stage_v);  // [HB]
   TypicalHead r{0, -1, 0u};
@@ -1295,8 +1296,8 @@ __device__ TypicalHead typical_head(const Src& X, int n, float m, float S, float
     for (int base = 0; base < n; base += kNT * TV) {
       const int pos = base + t * TV;
       float va[kLaneV], vb[kLaneV];
-      X.load4(pos, n, vec, va);
-      X.load4(pos + kLaneV, n, vec, vb);
+      X.load4(pos, n, va);
+      X.load4(pos + kLaneV, n, vb);
 #pragma unroll
       for (int k = 0; k < TV; ++k) {
         const int i = pos + k;
@@ -1395,7 +1396,6 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   BucketShared& bs = sh.u.bkt;
   const int t = (int)threadIdx.x;
   const bool t1 = (P.flags & kFlagTIsOne) != 0;
-  const bool vec = (P.flags & kFlagVecSrc) != 0;
   const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
   if (n >= (1 << 20)) return false;  // histogram counts hold 20 bits
   const uint32_t Kk = (P.top_k > 0 && P.top_k < (uint32_t)n) ? P.top_k : (uint32_t)n;
@@ -1415,7 +1415,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   uint32_t km = 0, fk = 0xffffffffu, fid = 0xffffffffu;
   {
     constexpr int TV = RowTiles8::V;
-    const RowTiles8 rt(X.x, n, vec);
+    const RowTiles8 rt(X.x, n);
     float raw[TV];
     rt.load(t * TV, raw);
     for (int base = 0; base < n; base += kNT * TV) {
@@ -1598,7 +1598,6 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
   const int t = (int)threadIdx.x;
   const int n = P.n;
   const bool t1 = (P.flags & kFlagTIsOne) != 0;
-  const bool vec = (P.flags & kFlagVecSrc) != 0;
   const bool typical = P.typical_p > 0.0f && P.typical_p < 1.0f;
   const float u = Q.uniforms[row];
   int K = 0;
@@ -1705,7 +1704,7 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
     // (~p bits, id) in index order, the next tile's loads in flight; the
     // smallest key lets the sort skip the digits every key shares
     constexpr int TV = RowTiles8::V;
-    const RowTiles8 rt(X.x, n, vec);
+    const RowTiles8 rt(X.x, n);
     float raw[TV];
     rt.load(t * TV, raw);
     uint32_t kmin = 0xffffffffu;

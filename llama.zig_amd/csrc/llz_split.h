@@ -102,13 +102,6 @@ __device__ __forceinline__ unsigned long long pack2(float lo, float hi) {
 __device__ __forceinline__ float lo_f(unsigned long long w) { return __uint_as_float((uint32_t)w); }
 __device__ __forceinline__ float hi_f(unsigned long long w) { return __uint_as_float((uint32_t)(w >> 32)); }
 
-__device__ __forceinline__ float4 split_ld4(const float* xr, int pos, int n) {
-  const bool in = pos < n;
-  const float4 v = ld_nt4(xr + (in ? pos : 0));
-  const float ni = -__builtin_inff();
-  return in ? v : make_float4(ni, ni, ni, ni);
-}
-
 // Chunk c of row `row` (every thread of the workgroup), NV = split_nv float4
 // per thread (a template parameter: the loads, all issued at once, need no
 // branch between them).  XF: the row is read through the caller's
@@ -132,8 +125,18 @@ __device__ __forceinline__ bool split_chunk(const KArgs& A, int row, int c, Spli
   // every load in flight at once (step j: the workgroup's 2048 logits from
   // base + 2048 j, one float4 per thread)
   float4 v[NV];
+  if ((P.flags & kFlagVecSrc) != 0u && (n & 3) == 0) {  // aligned rows: no shifts of the row's end
 #pragma unroll
-  for (int j = 0; j < NV; ++j) v[j] = split_ld4(xr, base + (j * kSplitNT + t) * 4, n);  // absent: -inf
+    for (int j = 0; j < NV; ++j) {
+      const int pos = base + (j * kSplitNT + t) * 4;
+      const float4 q = ld_nt4(xr + (pos < n ? pos : 0));
+      const float ni = -__builtin_inff();
+      v[j] = pos < n ? q : make_float4(ni, ni, ni, ni);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = rd4_any(xr, base + (j * kSplitNT + t) * 4, n);  // absent: -inf
+  }
   if constexpr (XF) {
     const uint32_t xf = P.xf_src;
     // main.zig:653-666 on each logit of the row (positions past it stay -inf)

@@ -1,9 +1,11 @@
-// llz_stats.hip -- k_stats: the fused per-row sampling kernel.  Phases L .. C
+// llz_stats.h -- k_stats: the fused per-row sampling kernel.  Phases L .. C
 // compute the row statistics (sampler.zig:80-88): the row maximum, the exact
 // sequential f32 normaliser and the candidate list, with one HBM read per
 // logit (method and error bound in llz_fast.h).  The same workgroup then runs
 // the selection stage (llz_select.h, sampler.zig:89-168); a row the fast path
 // cannot certify takes the streaming normaliser there instead.
+#pragma once
+
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -44,38 +46,32 @@ __device__ __forceinline__ llz_f4v to_v4(float4 f) {
 
 __device__ __forceinline__ float4 neg_inf4() { return make_float4(-kInfS, -kInfS, -kInfS, -kInfS); }
 
-// Branch-free segment loads (no per-lane branch, so every load of a wave can
-// be in flight at once).  Absent positions read a valid address and are
-// replaced by -inf.  ld4: 16-byte aligned row with n % 4 == 0.
-__device__ __forceinline__ float4 ld4(const float* xr, int pos, int n) {
-  const bool in = pos < n;
-  const float4 v = ld_nt4(xr + (in ? pos : 0));
-  return in ? v : neg_inf4();
-}
-__device__ __forceinline__ float4 ld1x4(const float* xr, int pos, int n) {
-  float4 v;
-  v.x = xr[pos + 0 < n ? pos + 0 : 0];
-  v.y = xr[pos + 1 < n ? pos + 1 : 0];
-  v.z = xr[pos + 2 < n ? pos + 2 : 0];
-  v.w = xr[pos + 3 < n ? pos + 3 : 0];
-  if (pos + 0 >= n) v.x = -kInfS;
-  if (pos + 1 >= n) v.y = -kInfS;
-  if (pos + 2 >= n) v.z = -kInfS;
-  if (pos + 3 >= n) v.w = -kInfS;
-  return v;
+// Branch-free 16-byte reads of a row (llz_rowops.h's rd4): FASTLD: 16-byte
+// aligned rows with n % 4 == 0, else any row.
+template <bool FASTLD>
+__device__ __forceinline__ float4 rd4(const float* xr, int pos, int n) {
+  if constexpr (FASTLD) {
+    const bool in = pos < n;
+    const float4 v = ld_nt4(xr + (in ? pos : 0));
+    return in ? v : neg_inf4();
+  } else {
+    return rd4_any(xr, pos, n);
+  }
 }
 
 // Copy one segment (1 KB) of the row into an LDS block of 256 floats:
-// straight to LDS when the segment is full and aligned, else through VGPRs.
-__device__ __forceinline__ void seg_to_lds(const float* xr, int seg, int n, bool fastld, float* dst) {
+// straight to LDS when the segment is full (a 16-byte read needs 4-byte
+// alignment only), else through VGPRs.
+template <bool FASTLD>
+__device__ __forceinline__ void seg_to_lds(const float* xr, int seg, int n, float* dst) {
   const int lane = lane_id();
   const int pos = seg * SEG + lane * 4;
-  if (fastld && (seg + 1) * SEG <= n) {
+  if ((seg + 1) * SEG <= n) {
 #if defined(__HIP_DEVICE_COMPILE__)
     __builtin_amdgcn_global_load_lds(xr + pos, dst, 16, 0, 0);
 #endif
   } else {
-    *reinterpret_cast<float4*>(dst + lane * 4) = fastld ? ld4(xr, pos, n) : ld1x4(xr, pos, n);
+    *reinterpret_cast<float4*>(dst + lane * 4) = rd4<FASTLD>(xr, pos, n);
   }
 }
 
@@ -105,7 +101,7 @@ __device__ __forceinline__ int slot_step(int w) { return w == 0 ? DCAP : W - 1; 
 // caller waits for them).
 template <bool FASTLD>
 __device__ __forceinline__ void exact_loads(FastShared& F, const float* xr, int w, int nslot, int n) {
-  for (int slot = w; slot < nslot; slot += slot_step(w)) seg_to_lds(xr, F.slotseg[slot], n, FASTLD, &F.u.x.dump[slot][0]);
+  for (int slot = w; slot < nslot; slot += slot_step(w)) seg_to_lds<FASTLD>(xr, F.slotseg[slot], n, &F.u.x.dump[slot][0]);
 }
 
 // The exact terms of four consecutive positions (sampler.zig:85), without
@@ -535,8 +531,11 @@ __device__ __noinline__ int claim_row(unsigned long long* word, unsigned long lo
   }
 }
 
-// FASTLD: 16-byte aligned rows with n % 4 == 0 (one float4 per lane per
-// segment through buffer loads); otherwise element loads.  XF: the rows are
+// FASTLD: 16-byte aligned rows with n % 4 == 0; otherwise rows of any length
+// and (4-byte) alignment, through the same 16-byte loads, which need 4-byte
+// alignment only, with the last n % 4 logits taken after the loop.  (Element
+// loads for such rows held phase L at 27.6 us for 97 x 32003, @UNAL@.)
+// XF: the rows are
 // read through post-processing and/or the fused repetition penalty
 // (llz_xform.h); otherwise as they are.
 // wslot: the workgroup's block of the special-queue overflow area.
@@ -583,13 +582,12 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // six loads in flight: any code that branches on the penalty inside it
   // costs registers it does not have).
   const float xscale = (XM == kXmLight && (P.xf_src & kXfScale)) ? P.inv_scale : 1.0f;
-  auto seg_in = [&](const int k, float4 v) -> float4 {
+  auto seg_in = [&](const int, float4 v) -> float4 {
     if constexpr (XM == kXmLight) {
-      const int pos = (w + W * k) * SEG + lane * 4;
-      v.x = (FASTLD || pos + 0 < n) ? v.x * xscale : v.x;
-      v.y = (FASTLD || pos + 1 < n) ? v.y * xscale : v.y;
-      v.z = (FASTLD || pos + 2 < n) ? v.z * xscale : v.z;
-      v.w = (FASTLD || pos + 3 < n) ? v.w * xscale : v.w;
+      v.x = v.x * xscale;
+      v.y = v.y * xscale;
+      v.z = v.z * xscale;
+      v.w = v.w * xscale;
     }
     return v;
   };
@@ -609,7 +607,6 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // wave w owns segments w, w + W, w + 2W, ...: its k-th is segment w + W k
   // (interleaved, so the costly start of the row is shared by every wave)
   const int nseg_w = fits ? max(0, (G - w + W - 1) / W) : 0;
-  const int base_w = w * SEG + lane * 4;
   const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
 
   // ---- phase L: per segment as it lands: running maximum, the estimate q
@@ -618,7 +615,10 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   float mx = -kInfS, cw = 0.0f;
   uint32_t nanf = 0;
   const int lane4 = lane * 4;
-  const int lim_w = nseg_w > 0 ? n - w * SEG : 0;  // segment k holds positions lane4 < lim_w - k W SEG
+  // The loop takes whole float4 of the row: the row's last n % 4 logits (!FASTLD)
+  // follow it, like the penalised elements.
+  const int nv = FASTLD ? n : n & ~3;
+  const int lim_w = nseg_w > 0 ? nv - w * SEG : 0;  // segment k holds positions lane4 < lim_w - k W SEG
   // bounds as (lane offset, VGPR) < (scalar limit of the segment); the
   // limits are recomputed in place (an empty asm keeps the compiler from
   // hoisting them all into live registers)
@@ -643,13 +643,6 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       v.y = est_of(v.y);
       v.z = est_of(v.z);
       v.w = est_of(v.w);
-      if constexpr (!FASTLD) {  // single positions past the row: no estimate (q = 0)
-        const int pos = (w + W * k) * SEG + lane4;
-        v.x = pos + 0 < n ? v.x : -kInfS;
-        v.y = pos + 1 < n ? v.y : -kInfS;
-        v.z = pos + 2 < n ? v.z : -kInfS;
-        v.w = pos + 3 < n ? v.w : -kInfS;
-      }
     }
     return q_of(v, l2e_t, ck);
   };
@@ -664,7 +657,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     if (!(fabsf(mr) <= 3.0e38f)) mr = 0.0f;
     cw = mr * l2e_t;
   };
-  if constexpr (FASTLD) {
+  {
     // A window of kLoadWindow loads in flight per wave, one issued as each
     // segment is done: each CU's share of HBM arrives spread over the whole
     // read, and each segment's work overlaps the loads behind it (with every
@@ -673,7 +666,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     // KV .. SPWMAX - 1 first (straight to LDS), then the register segments
     // 0 .. KV - 1.  Every slot issues exactly one load (reads past the row
     // return zeros), so the wait for slot i counts the loads behind it.
-    const llz_i4v rs = row_rsrc(xr, (uint32_t)n * 4u);
+    const llz_i4v rs = row_rsrc(xr, (uint32_t)nv * 4u);
     const int soff = __builtin_amdgcn_readfirstlane(w * SEG * 4);
     const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)&F.u.data[w][0][0]);
     auto issue = [&](const int i) {
@@ -713,30 +706,45 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       // loads are issued; the last kLoadWindow may interleave)
       if (i + kLoadWindow < SPWMAX) issue(i + kLoadWindow);
     }
-  } else {
-    // element loads, all in flight at once (guarded loads are waited for
-    // where they are read)
+  }
+  if constexpr (!FASTLD) {
+    // The row's last n % 4 logits: the wave that holds their segment (its
+    // kt-th) takes them in the lane they belong to, with the estimates the
+    // loop would have computed, and folds the segment's sum again.
+    const int gt = nv >> 8;
+    if (nv != n && fits && (gt & (W - 1)) == w) {
+      const int kt = gt >> 3;
+      const bool own = lane == ((nv >> 2) & (kWave - 1));
+      float4 v = own ? rd4<FASTLD>(xr, nv, n) : neg_inf4();
+      v = seg_in(kt, v);  // a scale keeps no -inf in place: absent positions are cut below
+      const bool a1 = nv + 1 < n, a2 = nv + 2 < n;
+      if constexpr (XM == kXmCap) {
+        v.x = est_of(v.x);
+        v.y = est_of(v.y);
+        v.z = est_of(v.z);
+      }
+      v.x = own ? v.x : -kInfS;
+      v.y = own && a1 ? v.y : -kInfS;
+      v.z = own && a2 ? v.z : -kInfS;
+      v.w = -kInfS;
+      if (nv <= w * SEG) set_cw(wave_max_f32(max4(v)));  // the wave holds no other logit
+      if constexpr (XM != kXmCap) mx = max3_raw(max3_raw(mx, v.x, v.y), v.z, v.w);
+      const float4 q = q_of(v, l2e_t, cw);
+      if (kt >= KV && own) *reinterpret_cast<float4*>(&F.u.data[w][kt - KV][lane4]) = q;
 #pragma unroll
-    for (int k = 0; k < KV; ++k) d[k] = ld1x4(xr, base_w + k * (W * SEG), k < nseg_w ? n : 0);
-    for (int k = KV; k < nseg_w; ++k) seg_to_lds(xr, w + W * k, n, false, &F.u.data[w][k - KV][0]);
-    __builtin_amdgcn_sched_barrier(0);
-    const float4 v0 = seg_in(0, d[0]);
-    set_cw(wave_max_f32(lane4 < seg_lim(0) ? est_of(max4(v0)) : -kInfS));
-#pragma unroll
-    for (int k = 0; k < KV; ++k) {
-      float4 v = v0;
-      if (k > 0) v = seg_in(k, d[k]);
-      float4 q = seg_q(k, v);
-      asm volatile("" : "+v"(q.x), "+v"(q.y), "+v"(q.z), "+v"(q.w));
-      d[k] = q;
-      seg_sum(k, q);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int k = KV; k < nseg_w; ++k) {
-      float4* p = reinterpret_cast<float4*>(&F.u.data[w][k - KV][lane * 4]);
-      const float4 q = seg_q(k, seg_in(k, *p));
-      *p = q;
-      seg_sum(k, q);
+      for (int k = 0; k < KV; ++k) {
+        if (k == kt) {
+          d[k].x = own ? q.x : d[k].x;
+          d[k].y = own ? q.y : d[k].y;
+          d[k].z = own ? q.z : d[k].z;
+          d[k].w = own ? q.w : d[k].w;
+          seg_sum(k, d[k]);
+        }
+      }
+      if (kt >= KV) {
+        __builtin_amdgcn_wave_barrier();  // this wave's own LDS writes: LDS order suffices
+        seg_sum(kt, *reinterpret_cast<const float4*>(&F.u.data[w][kt - KV][lane4]));
+      }
     }
   }
   // ---- the penalty (sampler.zig:54-75) on this wave's penalised elements,
@@ -848,25 +856,19 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     }
   }
   if (!fits) {  // rows the fast path does not take: maximum and NaN scan only
-    if constexpr (FASTLD) {
+    {
       // kScanDepth float4 loads per thread in flight (64 KB per workgroup)
       constexpr int U = kScanDepth;
       for (int b = t * 4; b < n; b += NT * 4 * U) {
         float4 v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = ld4(xr, b + u * (NT * 4), n);  // absent: -inf
+        for (int u = 0; u < U; ++u) v[u] = rd4<FASTLD>(xr, b + u * (NT * 4), n);  // absent: -inf
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const float4 f = X.fix4(b + u * (NT * 4), v[u], n);
           mx = fmaxf(mx, max4(f));  // fmaxf skips NaN, as the scalar loop did
           nanf |= (uint32_t)((f.x != f.x) | (f.y != f.y) | (f.z != f.z) | (f.w != f.w));
         }
-      }
-    } else {
-      for (int i = t; i < n; i += NT) {
-        const float v = X.at(i);
-        mx = fmaxf(mx, v);
-        nanf |= (uint32_t)(v != v);
       }
     }
   }
@@ -962,7 +964,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       for (int h = 0; h < QCAP / kWave; ++h) {
         const int i = h * kWave + lane;
         const int pos = i < nq ? (int)F.qpos[w][i] : 0;
-        tv[h] = FASTLD ? ld4(xr, pos, n) : ld1x4(xr, pos, n);  // raw: transformed where they are read
+        tv[h] = rd4<FASTLD>(xr, pos, n);  // raw: transformed where they are read
       }
     } else {
 #pragma unroll
@@ -1002,14 +1004,10 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     F.tcand = 0u;  // the token-only list (ordered before its atomics by the barrier below)
     F.tfail = 0u;
   }
-  if constexpr (FASTLD) {
-    // every load of the row has landed (the register segments, issued after
-    // the LDS-resident ones, were consumed): the barrier orders LDS only, and
-    // a token-only row's re-reads stay in flight across it
-    lds_barrier();
-  } else {
-    __syncthreads();
-  }
+  // every load of the row has landed (the register segments, issued after
+  // the LDS-resident ones, were consumed): the barrier orders LDS only, and
+  // a token-only row's re-reads stay in flight across it
+  lds_barrier();
   LLZ_STAMP(row, 1);
 
   // ---- phase M: row maximum, scale factors, binade prediction, first slots
@@ -1262,6 +1260,69 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       lds_barrier();
     }
   }
+  // ---- The candidates' threshold of the exact phases.  cand_theta without
+  // min-p (2^-16) floods the list on most rows of a model's usual shape, and
+  // a flooded list costs two more reads of the row (recollect_top, 48 us at
+  // 128256 logits) and thousands of candidates that phase S must leave to the
+  // exact exp.  Where the terms above 2^-10 or 2^-13 already hold the mass
+  // top-p can keep (with 2^-7 to spare: the estimates are within 2^-10 of the
+  // terms, the sequential S within 2^-7 of the real sum), or more terms than
+  // top-k keeps, that threshold is taken: the kept prefix then ends inside
+  // the list, and the selection's certified prefix checks that it does.  A
+  // threshold whose terms do not fit the list means no lower one's do: the
+  // row floods at once.  One pass over the resident estimates per threshold
+  // (3.4 us).
+  float theta_c = P.cand_theta;
+  bool flood_c = false;
+  {
+    const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
+    const bool topk = P.top_k > 0u && P.top_k <= (uint32_t)kCandCap / 2u;
+    if (fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f) {
+      const float Rw = __builtin_amdgcn_exp2f(fmaf(m, -l2e_t, cw));
+      const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
+      for (int pass = 0; pass < 2; ++pass) {
+        const float th = pass == 0 ? 0x1p-10f : 0x1p-13f;
+        if (!(th > P.cand_theta)) break;
+        const float tq_lo = th * (1.0f + 0x1p-9f) / Rw;
+        float ms = 0.0f;
+        uint32_t cn = 0u;
+        auto acc = [&](const float4 q) {
+          const bool b0 = q.x >= tq_lo, b1 = q.y >= tq_lo, b2 = q.z >= tq_lo, b3 = q.w >= tq_lo;
+          ms += ((b0 ? q.x : 0.0f) + (b1 ? q.y : 0.0f)) + ((b2 ? q.z : 0.0f) + (b3 ? q.w : 0.0f));
+          cn += (uint32_t)b0 + (uint32_t)b1 + (uint32_t)b2 + (uint32_t)b3;
+        };
+#pragma unroll
+        for (int k = 0; k < KV; ++k) acc(d[k]);
+        for (int k = KV; k < nseg_w; ++k) acc(*reinterpret_cast<const float4*>(&F.u.data[w][k - KV][lane4]));
+        const float wm = wave_fold_f32(ms) * Rw;
+        const uint32_t wc = wave_sum_u32(cn);
+        if (lane == kWave - 1) {
+          F.tx[w] = tot;
+          F.txa[w] = wm;
+          F.wflag[w] = wc;
+        }
+        lds_barrier();
+        float st = 0.0f, sm = 0.0f;
+        uint32_t sc = 0u;
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          st += F.tx[i];
+          sm += F.txa[i];
+          sc += F.wflag[i];
+        }
+        lds_barrier();  // read by every wave before the next pass writes them
+        const bool holds = (topp && sm >= P.top_p * st * (1.0f + 0x1p-7f)) || (topk && sc > P.top_k);
+        if (sc > (uint32_t)(kCandCap - kCandCap / 16)) {
+          flood_c = true;
+          break;
+        }
+        if (holds) {
+          theta_c = th;
+          break;
+        }
+      }
+    }
+  }
   // the segment sums of q of round `lane` (segments W lane .. W lane + W - 1,
   // one per wave), all read at once; absent ones are 0 (selects, not
   // branches: each branch here would wait out an LDS read of its own)
@@ -1350,7 +1411,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
         const int elo = (int)(__float_as_uint(lo) >> 23) - 127;
         const int ehi = (int)(__float_as_uint(hi) >> 23) - 127;
         const bool plain = lo >= 0x1p-64f && hi <= 3.0e38f && elo == ehi;
-        fl = plain && ldexpf(P.cand_theta, 23 - elo) < 2.0f;
+        fl = plain && ldexpf(theta_c, 23 - elo) < 2.0f;
         // EXACT: tabulate the binades from the one the segment starts in to
         // the one it ends in (the row's first segment starts at 0: its NG
         // highest, below them it is summed term by term)
@@ -1370,7 +1431,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       if (lane == 0) {
         if (exm != 0ull) base = (int)atomicAdd((uint32_t*)&F.nslot, (uint32_t)__popcll(exm));
         if (bad) atomicOr(&F.fail, 1u);
-        if (bal64(fl) != 0ull) atomicOr(&F.flood, 1u);
+        if (flood_c || bal64(fl) != 0ull) atomicOr(&F.flood, 1u);
       }
       base = __builtin_amdgcn_readfirstlane(base);
       if (have) {
@@ -1383,7 +1444,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     __syncthreads();
     LLZ_STAMP(row, 2);
     const bool flood = F.flood != 0u;
-    const float theta = flood ? kInfS : P.cand_theta;
+    const float theta = flood ? kInfS : theta_c;
 
     // ---- phase S: integer sums of PLAIN segments, four segments per step.
     // A lane whose roundings a segment cannot certify (its lower and upper
@@ -1398,7 +1459,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       for (int h = 0; h < 2; ++h) {
         const int i = h * kWave + lane;
         const int pos = i < cnt ? (int)(F.qpos[w][i] & 0x7fffffffu) : 0;
-        const float4 r = FASTLD ? ld4(xr, pos, n) : ld1x4(xr, pos, n);
+        const float4 r = rd4<FASTLD>(xr, pos, n);
         v4q[h] = XM == kXmCap ? r : X.fix4(pos, r, n);  // kXmCap: raw (settle_specials transforms them)
       }
     };
@@ -1824,7 +1885,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   static_assert(sizeof(SampleShared) <= sizeof(F.u), "the selection's memory must lie inside F.u");
   select_row(P, Q, U.select, m, certified ? S : 0.0f, certified ? cc : 0u, !certified, u_row, certified && pre_ok,
              cand_pre, cand_n0, X, O, XF ? &pen_sh : nullptr, kernel_args_ptr(), row,
-             wslot);
+             wslot, theta_c);
   LLZ_STAMP(row, 15);
   // the walk's diagnostics join the status thread 0 wrote (F.diag lies past
   // the selection's memory)
@@ -1867,7 +1928,7 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
   }
 }
 
-// Split rows (token-only calls of few rows, plain 16-byte aligned rows):
+// Split rows (token-only calls of few rows):
 // workgroup b reads chunk b % split_s of row b / split_s (NV float4 per
 // thread); a workgroup that sees the row's chunks published merges it, and
 // the one that takes an uncertified row finishes it with the single-row
@@ -1886,87 +1947,8 @@ __global__ __launch_bounds__(NT) void k_split(KArgs A) {
   if (!split_chunk<NV, XM != kXmNone>(A, row, c, U.split)) return;
   if (split_merge(A, row, U.split)) return;
   if (!split_take(A, row, U.split)) return;  // (its barrier: every wave is done with the merge's shared memory)
-  stats_row<true, XM>(A, row, U.stats, pen_sh, row);
+  stats_row<false, XM>(A, row, U.stats, pen_sh, row);
 }
 
 }  // namespace
-
-// One launch per call: every row's statistics, then its selection.
-hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_begin, hipEvent_t ev_end,
-                         hipStream_t st) {
-  if (ev_begin && hipEventRecord(ev_begin, st) != hipSuccess) return hipErrorUnknown;
-  const bool fastld = (P.flags & kFlagVecSrc) != 0 && (P.n % 4) == 0;
-  // the transform mode: soft-capping (the chain's input) takes the
-  // estimating single pass, the scale and the penalty alone the exact one
-  const int xm = (P.xf_src & kXfCap) ? kXmCap : ((P.xf_src | P.xf_orig) != 0u ? kXmLight : kXmNone);
-  const KArgs A{P, Q};
-  // more rows than workgroups: the grid's workgroups claim rows (the
-  // special-queue overflow area has one block per workgroup of the grid)
-  const bool claim = P.grid < P.rows;
-  // transformed rows split with chunks of at most 2 float4 per thread (each
-  // logit's exact post-processing is then a few per thread)
-  const bool split = P.split_s >= 2 && fastld && P.rows <= kSplitRows && (xm == kXmNone || P.split_nv <= 2);
-  // token-only calls with typical-p (not soft-capped) take the instantiation
-  // that carries typical-p's decisions and the list's second collection
-  // round; the others keep the shorter code
-  const bool ext = (P.flags & kFlagTokenOnly) != 0u && P.typical_p > 0.0f && P.typical_p < 1.0f && xm != kXmCap;
-  const dim3 grid(split ? P.rows * P.split_s : (claim ? P.grid : P.rows)), block(NT);
-  void (*kern)(KArgs) = nullptr;
-  if (split) {
-    if (xm == kXmNone) {
-      switch (P.split_nv) {
-        case 1: kern = k_split<1, kXmNone>; break;
-        case 2: kern = k_split<2, kXmNone>; break;
-        case 4: kern = k_split<4, kXmNone>; break;
-        case 8: kern = k_split<8, kXmNone>; break;
-        default: return hipErrorInvalidValue;
-      }
-    } else if (xm == kXmLight) {
-      kern = P.split_nv == 1 ? k_split<1, kXmLight> : k_split<2, kXmLight>;
-    } else {
-      kern = P.split_nv == 1 ? k_split<1, kXmCap> : k_split<2, kXmCap>;
-    }
-  } else if (claim) {
-    if (ext)
-      kern = fastld ? (xm == kXmNone ? k_stats_rows<true, kXmNone, true> : k_stats_rows<true, kXmLight, true>)
-                    : (xm == kXmNone ? k_stats_rows<false, kXmNone, true> : k_stats_rows<false, kXmLight, true>);
-    else if (fastld)
-      kern = xm == kXmNone ? k_stats_rows<true, kXmNone, false> : xm == kXmLight ? k_stats_rows<true, kXmLight, false>
-                                                                                 : k_stats_rows<true, kXmCap, false>;
-    else
-      kern = xm == kXmNone ? k_stats_rows<false, kXmNone, false> : xm == kXmLight ? k_stats_rows<false, kXmLight, false>
-                                                                                  : k_stats_rows<false, kXmCap, false>;
-  } else {
-    if (ext)
-      kern = fastld ? (xm == kXmNone ? k_stats<true, kXmNone, true> : k_stats<true, kXmLight, true>)
-                    : (xm == kXmNone ? k_stats<false, kXmNone, true> : k_stats<false, kXmLight, true>);
-    else if (fastld)
-      kern = xm == kXmNone ? k_stats<true, kXmNone, false> : xm == kXmLight ? k_stats<true, kXmLight, false>
-                                                                            : k_stats<true, kXmCap, false>;
-    else
-      kern = xm == kXmNone ? k_stats<false, kXmNone, false> : xm == kXmLight ? k_stats<false, kXmLight, false>
-                                                                             : k_stats<false, kXmCap, false>;
-  }
-  void* args[] = {const_cast<KArgs*>(&A)};
-  if (hipLaunchKernel((const void*)kern, grid, block, args, 0, st) != hipSuccess) return hipErrorLaunchFailure;
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  if (ev_end && hipEventRecord(ev_end, st) != hipSuccess) return hipErrorUnknown;
-  return hipSuccess;
-}
-
 }  // namespace llz
-
-#ifdef LLZ_PHASE_STAMPS
-// Measurement builds: the phase timestamps of rows 0 .. rows - 1 (kStampSlots
-// per row, 0 where a row did not reach the boundary) into dst.
-extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int clear) {
-  if (rows <= 0 || rows > llz::kStampRows || !dst) return -1;
-  const size_t bytes = (size_t)rows * llz::kStampSlots * sizeof(unsigned long long);
-  if (clear) {
-    static unsigned long long zeros[llz::kStampRows * llz::kStampSlots];
-    return hipMemcpyToSymbol(HIP_SYMBOL(llz::llz_phase_stamps), zeros, sizeof(zeros)) == hipSuccess ? 0 : -3;
-  }
-  return hipMemcpyFromSymbol(dst, HIP_SYMBOL(llz::llz_phase_stamps), bytes) == hipSuccess ? 0 : -3;
-}
-#endif

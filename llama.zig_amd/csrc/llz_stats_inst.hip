@@ -1,0 +1,47 @@
+// llz_stats_inst.hip -- the instantiations of the sampling kernels
+// (llz_stats.h), one group per object (LLZ_INST), so that they build in
+// parallel:
+//   0-4  k_stats / k_stats_rows: plain, plain with typical-p, light, light
+//        with typical-p, soft-capped (a: 16-byte aligned rows; b: claimed rows)
+//   5    k_split on plain rows (a: float4 per thread)
+//   6    k_split on transformed rows (a: float4 per thread; b: soft-capped)
+#include "llz_stats.h"
+
+#ifndef LLZ_INST
+#error "LLZ_INST selects the group of kernels"
+#endif
+#define LLZ_CAT2(a, b) a##b
+#define LLZ_CAT(a, b) LLZ_CAT2(a, b)
+
+namespace llz {
+
+StatsKernel LLZ_CAT(stats_kernel_, LLZ_INST)(int a, int b) {
+#if LLZ_INST <= 4
+  constexpr int XM = LLZ_INST <= 1 ? kXmNone : LLZ_INST <= 3 ? kXmLight : kXmCap;
+  constexpr bool EXT = LLZ_INST == 1 || LLZ_INST == 3;
+  if (b != 0) return a != 0 ? k_stats_rows<true, XM, EXT> : k_stats_rows<false, XM, EXT>;
+  return a != 0 ? k_stats<true, XM, EXT> : k_stats<false, XM, EXT>;
+#elif LLZ_INST == 5
+  (void)b;
+  return a == 1 ? k_split<1, kXmNone> : a == 2 ? k_split<2, kXmNone> : a == 4 ? k_split<4, kXmNone>
+                                    : a == 8 ? k_split<8, kXmNone> : nullptr;
+#else
+  if (b != 0) return a == 1 ? k_split<1, kXmCap> : k_split<2, kXmCap>;
+  return a == 1 ? k_split<1, kXmLight> : k_split<2, kXmLight>;
+#endif
+}
+
+}  // namespace llz
+
+#ifdef LLZ_PHASE_STAMPS
+// Measurement builds: this object's phase timestamps (each object has its
+// own copy of the array; one call's rows are all in one).
+extern "C" int LLZ_CAT(llz_stamps_, LLZ_INST)(unsigned long long* dst, int rows, int clear) {
+  const size_t bytes = (size_t)rows * llz::kStampSlots * sizeof(unsigned long long);
+  if (clear) {
+    static unsigned long long zeros[llz::kStampRows * llz::kStampSlots];
+    return hipMemcpyToSymbol(HIP_SYMBOL(llz::llz_phase_stamps), zeros, sizeof(zeros)) == hipSuccess ? 0 : -3;
+  }
+  return hipMemcpyFromSymbol(dst, HIP_SYMBOL(llz::llz_phase_stamps), bytes) == hipSuccess ? 0 : -3;
+}
+#endif

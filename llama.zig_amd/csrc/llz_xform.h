@@ -183,9 +183,9 @@ struct RowSrcT {
   __device__ __forceinline__ float4 fix4(int pos, float4 v, int n) const { return pen4(pos, pre4(pos, v, n), n); }
 
   // kLaneV consecutive logits from pos (positions >= n read as 0).
-  __device__ __forceinline__ void load4(int pos, int n, bool vec, float (&v)[kLaneV]) const {
-    if (vec && pos + kLaneV <= n) {
-      const llz_f4v q = *(const __attribute__((address_space(1))) llz_f4v*)(grow(x) + pos);
+  __device__ __forceinline__ void load4(int pos, int n, float (&v)[kLaneV]) const {
+    if (pos + kLaneV <= n) {
+      const llz_f4u q = *(const __attribute__((address_space(1))) llz_f4u*)(grow(x) + pos);
       v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
     } else {
 #pragma unroll
@@ -213,9 +213,9 @@ struct PlainSrc {
   __device__ __forceinline__ float4 pre4(int, float4 v, int) const { return v; }
   __device__ __forceinline__ float4 pen4(int, float4 v, int) const { return v; }
   __device__ __forceinline__ float4 fix4(int, float4 v, int) const { return v; }
-  __device__ __forceinline__ void load4(int pos, int n, bool vec, float (&v)[kLaneV]) const {
-    if (vec && pos + kLaneV <= n) {
-      const llz_f4v q = *(const __attribute__((address_space(1))) llz_f4v*)(grow(x) + pos);
+  __device__ __forceinline__ void load4(int pos, int n, float (&v)[kLaneV]) const {
+    if (pos + kLaneV <= n) {
+      const llz_f4u q = *(const __attribute__((address_space(1))) llz_f4u*)(grow(x) + pos);
       v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
     } else {
 #pragma unroll

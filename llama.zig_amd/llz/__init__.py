@@ -249,7 +249,7 @@ PATH_WALK_ROUNDS, PATH_RESOLVE_GENERIC = 16, 32  # diagnostics of the single pas
 PATH_BUCKETS = 64  # full row without a sort: kept prefix, total and draw from p-key buckets
 PATH_TOKEN_ONLY = 128  # the token decided without the exact normaliser (calls asking for the token alone)
 PATH_DECLINE_SHIFT = 8  # bits 8-15: why the bucket path declined a full-row row (a number, not flags)
-PATH_RECOLLECT = 1 << 16  # a flooded candidate list collected again (its largest terms)
+PATH_RECOLLECT = 1 << 16  # the candidate list holds the largest terms only (raised threshold, or collected again)
 PATH_SPLIT = 1 << 17  # token-only row finished from chunks read by several workgroups (with PATH_TOKEN_ONLY)
 
 
