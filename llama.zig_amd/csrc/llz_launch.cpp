@@ -13,6 +13,8 @@ StatsKernel stats_kernel_3(int, int);
 StatsKernel stats_kernel_4(int, int);
 StatsKernel stats_kernel_5(int, int);
 StatsKernel stats_kernel_6(int, int);
+StatsKernel stats_kernel_7(int, int);
+StatsKernel stats_kernel_8(int, int);
 
 // Every row's statistics, then its selection.
 hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_begin, hipEvent_t ev_end,
@@ -35,7 +37,8 @@ hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_beg
   const bool ext = (P.flags & kFlagTokenOnly) != 0u && P.typical_p > 0.0f && P.typical_p < 1.0f && xm != kXmCap;
   StatsKernel kern = nullptr;
   if (split)
-    kern = xm == kXmNone ? stats_kernel_5(P.split_nv, 0) : stats_kernel_6(P.split_nv, xm == kXmCap);
+    kern = xm == kXmNone ? (fastld ? stats_kernel_5(P.split_nv, 0) : stats_kernel_6(P.split_nv, 0))
+                         : (fastld ? stats_kernel_7 : stats_kernel_8)(P.split_nv, xm == kXmCap);
   else if (xm == kXmCap)
     kern = stats_kernel_4(fastld, claim);
   else if (xm == kXmLight)
@@ -62,13 +65,16 @@ extern "C" int llz_stamps_3(unsigned long long*, int, int);
 extern "C" int llz_stamps_4(unsigned long long*, int, int);
 extern "C" int llz_stamps_5(unsigned long long*, int, int);
 extern "C" int llz_stamps_6(unsigned long long*, int, int);
+extern "C" int llz_stamps_7(unsigned long long*, int, int);
+extern "C" int llz_stamps_8(unsigned long long*, int, int);
 
 // Measurement builds: the phase timestamps of rows 0 .. rows - 1 (kStampSlots
 // per row, 0 where a row did not reach the boundary) into dst.
 extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int clear) {
   if (rows <= 0 || rows > llz::kStampRows || !dst) return -1;
   static int (*const get[])(unsigned long long*, int, int) = {llz_stamps_0, llz_stamps_1, llz_stamps_2, llz_stamps_3,
-                                                              llz_stamps_4, llz_stamps_5, llz_stamps_6};
+                                                              llz_stamps_4, llz_stamps_5, llz_stamps_6, llz_stamps_7,
+                                                              llz_stamps_8};
   static unsigned long long part[llz::kStampRows * llz::kStampSlots];
   const size_t n = (size_t)rows * llz::kStampSlots;
   if (!clear)

@@ -376,7 +376,7 @@ __device__ float row_normaliser(const Src& X, int n, const RowParams& P, SampleS
 
 // Sequential accumulation dispatcher: short lists run the reference's loop
 // on one wave; long ones use the workgroup's exact parallel scan.
-constexpr int kSeqMax = 128;
+constexpr int kSeqMax = 2048;
 
 template <bool SUB, typename TermFn>
 __device__ float seq_accumulate(float s, int len, float thr, int& stop, TermFn term, SampleShared& sh,
@@ -751,6 +751,89 @@ __device__ __noinline__ void select_full_row(const KArgs* A, int row, const PenS
                                              int bank, float m, float S, uint32_t path, int wslot);
 
 constexpr int kShortMax = 256;  // longest candidate list of the short path
+
+// Sort of the candidate list sh.cand[0, c) (c <= kCap distinct keys,
+// ascending).  The keys' upper words span few octaves of p, so equal steps of
+// them make kSortBins bins of a few keys each: counts, an exclusive scan, the
+// keys scattered to their bins, and each bin's few keys put in order by one
+// thread: five barriers, where the bitonic network takes one per stage (66
+// for 2048 keys: 40 us of a row, now @SORTUS@).  Lists with a long bin (many equal or near
+// p) and short lists take the network.
+constexpr int kSortBins = 2048;
+constexpr int kSortBinMax = 24;
+
+__device__ __noinline__ void sort_list(SampleShared& sh_arg, int c, int& bank) {
+  SampleShared& sh = *(SampleShared*)(__attribute__((address_space(3))) SampleShared*)(&sh_arg);
+  const int t = (int)threadIdx.x, lane = lane_id(), w = wave_id();
+  if (c > 128) {
+    constexpr int PT = kSortBins / kNT;
+    uint32_t* cnt = sh.u.post.aux_pos;  // counts, then the bins' next places
+    static_assert(sizeof(sh.u.post.aux_pos) >= kSortBins * sizeof(uint32_t), "bins fit");
+    for (int b = t; b < kSortBins; b += kNT) cnt[b] = 0u;
+    uint32_t lo = 0xffffffffu, hi = 0u;
+    for (int i = t; i < c; i += kNT) {
+      const uint32_t k = (uint32_t)(sh.cand[i] >> 32);
+      lo = min(lo, k);
+      hi = max(hi, k);
+    }
+    lo = wg_min_u32<kNT>(lo, sh.wg, bank);  // (its barrier orders the zeroing too)
+    hi = wg_max_u32<kNT>(hi, sh.wg, bank);
+    const int shift = max(0, 32 - __clz((int)(hi - lo)) - 11);  // (hi - lo) >> shift < 2048
+    for (int i = t; i < c; i += kNT) atomicAdd(&cnt[((uint32_t)(sh.cand[i] >> 32) - lo) >> shift], 1u);
+    lds_barrier();
+    uint32_t v[PT], sum = 0u, longest = 0u;
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+      v[q] = cnt[t * PT + q];
+      sum += v[q];
+      longest = max(longest, v[q]);
+    }
+    const uint32_t incl = wave_incl_scan_op(sum, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+    const uint32_t wl = wave_max_u32(longest);
+    if (lane == kWave - 1) sh.wg.red[bank][w] = incl | (wl > (uint32_t)kSortBinMax ? 0x80000000u : 0u);
+    lds_barrier();
+    uint32_t run = incl - sum;
+    bool too_long = false;
+#pragma unroll
+    for (int i = 0; i < kNT / kWave; ++i) {
+      const uint32_t x = sh.wg.red[bank][i];
+      run += i < w ? x & 0x7fffffffu : 0u;
+      too_long = too_long || (x >> 31) != 0u;
+    }
+    bank ^= 1;
+    if (!too_long) {
+      uint32_t first[PT];
+#pragma unroll
+      for (int q = 0; q < PT; ++q) {
+        first[q] = run;
+        cnt[t * PT + q] = run;
+        run += v[q];
+      }
+      lds_barrier();
+      for (int i = t; i < c; i += kNT) {
+        const uint64_t k = sh.cand[i];
+        sh.u.post.aux[atomicAdd(&cnt[((uint32_t)(k >> 32) - lo) >> shift], 1u)] = k;
+      }
+      lds_barrier();
+      // each key's place in its bin: the bin's smaller keys
+#pragma unroll
+      for (int q = 0; q < PT; ++q) {
+        for (uint32_t i = 0; i < v[q]; ++i) {
+          const uint64_t k = sh.u.post.aux[first[q] + i];
+          uint32_t r = 0u;
+          for (uint32_t j = 0; j < v[q]; ++j) r += sh.u.post.aux[first[q] + j] < k ? 1u : 0u;
+          sh.cand[first[q] + r] = k;
+        }
+      }
+      lds_barrier();
+      return;
+    }
+  }
+  const int n2 = next_pow2(c);
+  for (int i = c + t; i < n2; i += kNT) sh.cand[i] = ~0ull;
+  lds_barrier();
+  lds_bitonic_sort_u64<kNT>(sh.cand, n2);
+}
 
 // A flooded candidate list (more than kCap elements with e >= cand_theta) is
 // collected again from the row, keeping only its largest terms, so that the
@@ -1134,18 +1217,15 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
     if (!select_short(Pl, Q, row, sh, c, m, S, path, u_row)) select_full_row<Src>(A, row, pen, sh, bank, m, S, path, wslot);
     return;
   }
-  const int csort = next_pow2(c);
-  for (int i = t; i < csort; i += kNT) {
-    if (i < c) {
+  if (!ovf) {  // (a list that overflowed decides nothing: M = 0)
+    for (int i = t; i < c; i += kNT) {
       const uint64_t a = sh.cand[i];
       const float p = __uint_as_float((uint32_t)(a >> 32)) / S;
       sh.cand[i] = ((uint64_t)(~__float_as_uint(p)) << 32) | (uint32_t)a;
-    } else {
-      sh.cand[i] = ~0ull;
     }
+    lds_barrier();
+    sort_list(sh, c, bank);
   }
-  lds_barrier();
-  lds_bitonic_sort_u64<kNT>(sh.cand, csort);
 
   // certified prefix: every element outside the list has p <= theta / S
   int M = 0;

@@ -107,9 +107,10 @@ __device__ __forceinline__ float hi_f(unsigned long long w) { return __uint_as_f
 // branch between them).  XF: the row is read through the caller's
 // post-processing and the fused repetition penalty (P.xf_src), applied
 // exactly to every logit of the chunk as it lands (a few per thread).
+// FASTLD: 16-byte aligned rows with n % 4 == 0.
 // Returns true in every thread of a workgroup that saw every chunk of the
 // row published and goes on to merge it.
-template <int NV, bool XF>
+template <int NV, bool XF, bool FASTLD>
 __device__ __forceinline__ bool split_chunk(const KArgs& A, int row, int c, SplitShared& S) {
   const RowParams& P = A.P;
   const RowPtrs& Q = A.Q;
@@ -125,17 +126,16 @@ __device__ __forceinline__ bool split_chunk(const KArgs& A, int row, int c, Spli
   // every load in flight at once (step j: the workgroup's 2048 logits from
   // base + 2048 j, one float4 per thread)
   float4 v[NV];
-  if ((P.flags & kFlagVecSrc) != 0u && (n & 3) == 0) {  // aligned rows: no shifts of the row's end
 #pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int pos = base + (j * kSplitNT + t) * 4;
+  for (int j = 0; j < NV; ++j) {  // absent: -inf
+    const int pos = base + (j * kSplitNT + t) * 4;
+    if constexpr (FASTLD) {
       const float4 q = ld_nt4(xr + (pos < n ? pos : 0));
       const float ni = -__builtin_inff();
       v[j] = pos < n ? q : make_float4(ni, ni, ni, ni);
+    } else {
+      v[j] = rd4_any(xr, pos, n);
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) v[j] = rd4_any(xr, base + (j * kSplitNT + t) * 4, n);  // absent: -inf
   }
   if constexpr (XF) {
     const uint32_t xf = P.xf_src;

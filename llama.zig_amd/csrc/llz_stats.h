@@ -534,7 +534,7 @@ __device__ __noinline__ int claim_row(unsigned long long* word, unsigned long lo
 // FASTLD: 16-byte aligned rows with n % 4 == 0; otherwise rows of any length
 // and (4-byte) alignment, through the same 16-byte loads, which need 4-byte
 // alignment only, with the last n % 4 logits taken after the loop.  (Element
-// loads for such rows held phase L at 27.6 us for 97 x 32003, @UNAL@.)
+// loads for such rows held phase L at 27.6 us for 97 x 32003; 16.9 now.)
 // XF: the rows are
 // read through post-processing and/or the fused repetition penalty
 // (llz_xform.h); otherwise as they are.
@@ -1221,7 +1221,12 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
         collect(theta_t);
       }
       const int tc = (int)F.tcand;
-      if (tc <= kTokCap && F.tfail == 0u) {
+      // top-p alone over a long list: its cut lies among terms of a few 2^-10
+      // of the mass, closer together than the interval of S (8% of such rows
+      // of the default chain were decided); the sort and the decisions (5 us)
+      // are left out
+      const bool open_long = P.tok_theta > P.cand_theta && tc > kTokCap / 4 && !(kk >= 1u && kk <= (uint32_t)(kTokCap / 4));
+      if (tc <= kTokCap && F.tfail == 0u && !open_long) {
         token_sort(tl, tl + kTokCap, reinterpret_cast<uint8_t*>(&F.qpos[0][0]), tc);
         LLZ_STAMP(row, 34);
         if (w == 0) {
@@ -1264,14 +1269,14 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // min-p (2^-16) floods the list on most rows of a model's usual shape, and
   // a flooded list costs two more reads of the row (recollect_top, 48 us at
   // 128256 logits) and thousands of candidates that phase S must leave to the
-  // exact exp.  Where the terms above 2^-10 or 2^-13 already hold the mass
-  // top-p can keep (with 2^-7 to spare: the estimates are within 2^-10 of the
-  // terms, the sequential S within 2^-7 of the real sum), or more terms than
-  // top-k keeps, that threshold is taken: the kept prefix then ends inside
-  // the list, and the selection's certified prefix checks that it does.  A
-  // threshold whose terms do not fit the list means no lower one's do: the
-  // row floods at once.  One pass over the resident estimates per threshold
-  // (3.4 us).
+  // exact exp.  A threshold is taken instead whose terms fit the list and
+  // hold the mass top-p can keep (with 2^-7 to spare: the estimates are within
+  // 2^-10 of the terms, the sequential S within 2^-7 of the real sum), or more
+  // terms than top-k keeps: the kept prefix then ends inside the list, and
+  // the selection's certified prefix checks that it does.  2^-10 serves most
+  // rows; otherwise it is searched from there, one pass over the resident
+  // estimates per threshold (3.4 us).  When some threshold's terms neither
+  // fit nor hold it, none does: the row floods at once.
   float theta_c = P.cand_theta;
   bool flood_c = false;
   {
@@ -1280,9 +1285,12 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     if (fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f) {
       const float Rw = __builtin_amdgcn_exp2f(fmaf(m, -l2e_t, cw));
       const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
-      for (int pass = 0; pass < 2; ++pass) {
-        const float th = pass == 0 ? 0x1p-10f : 0x1p-13f;
-        if (!(th > P.cand_theta)) break;
+      // e: log2 of the threshold tried; below e_lo the terms do not fit the
+      // list, above e_hi they do not hold the prefix
+      float e = -10.0f, e_hi = 0.0f, e_lo = -kInfS;
+      const float e_min = __builtin_amdgcn_logf(P.cand_theta) + 0.5f;
+      for (int pass = 0; pass < 6; ++pass) {
+        const float th = __builtin_amdgcn_exp2f(e);
         const float tq_lo = th * (1.0f + 0x1p-9f) / Rw;
         float ms = 0.0f;
         uint32_t cn = 0u;
@@ -1312,14 +1320,23 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
         }
         lds_barrier();  // read by every wave before the next pass writes them
         const bool holds = (topp && sm >= P.top_p * st * (1.0f + 0x1p-7f)) || (topk && sc > P.top_k);
-        if (sc > (uint32_t)(kCandCap - kCandCap / 16)) {
-          flood_c = true;
-          break;
-        }
-        if (holds) {
+        const bool fit = sc <= (uint32_t)(kCandCap - kCandCap / 16);
+        if (holds && fit) {
           theta_c = th;
           break;
         }
+        if (holds) {
+          e_lo = e;
+          e = 0.5f * (e + e_hi);
+        } else if (!fit) {
+          flood_c = true;
+          break;
+        } else {
+          e_hi = e;
+          e = e_lo > -kInfS ? 0.5f * (e + e_lo) : e - 3.0f;
+          if (e < e_min) break;  // cand_theta's list
+        }
+        flood_c = e_lo > -kInfS && pass == 5;
       }
     }
   }
@@ -1938,16 +1955,16 @@ union SplitLds {
   SplitShared split;
   StatsShared stats;
 };
-template <int NV, int XM>
+template <int NV, int XM, bool FASTLD>
 __global__ __launch_bounds__(NT) void k_split(KArgs A) {
   __shared__ SplitLds U;
   __shared__ PenShared pen_sh;  // the single-row path's penalised positions (kXfPen)
   const int ns = A.P.split_s;
   const int row = (int)blockIdx.x / ns, c = (int)blockIdx.x - row * ns;
-  if (!split_chunk<NV, XM != kXmNone>(A, row, c, U.split)) return;
+  if (!split_chunk<NV, XM != kXmNone, FASTLD>(A, row, c, U.split)) return;
   if (split_merge(A, row, U.split)) return;
   if (!split_take(A, row, U.split)) return;  // (its barrier: every wave is done with the merge's shared memory)
-  stats_row<false, XM>(A, row, U.stats, pen_sh, row);
+  stats_row<FASTLD, XM>(A, row, U.stats, pen_sh, row);
 }
 
 }  // namespace

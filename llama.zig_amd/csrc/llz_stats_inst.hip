@@ -3,8 +3,8 @@
 // parallel:
 //   0-4  k_stats / k_stats_rows: plain, plain with typical-p, light, light
 //        with typical-p, soft-capped (a: 16-byte aligned rows; b: claimed rows)
-//   5    k_split on plain rows (a: float4 per thread)
-//   6    k_split on transformed rows (a: float4 per thread; b: soft-capped)
+//   5, 6 k_split on plain rows: 16-byte aligned, any (a: float4 per thread)
+//   7, 8 k_split on transformed rows, the same (a: float4 per thread; b: soft-capped)
 #include "llz_stats.h"
 
 #ifndef LLZ_INST
@@ -21,13 +21,15 @@ StatsKernel LLZ_CAT(stats_kernel_, LLZ_INST)(int a, int b) {
   constexpr bool EXT = LLZ_INST == 1 || LLZ_INST == 3;
   if (b != 0) return a != 0 ? k_stats_rows<true, XM, EXT> : k_stats_rows<false, XM, EXT>;
   return a != 0 ? k_stats<true, XM, EXT> : k_stats<false, XM, EXT>;
-#elif LLZ_INST == 5
+#elif LLZ_INST <= 6
+  constexpr bool F = LLZ_INST == 5;
   (void)b;
-  return a == 1 ? k_split<1, kXmNone> : a == 2 ? k_split<2, kXmNone> : a == 4 ? k_split<4, kXmNone>
-                                    : a == 8 ? k_split<8, kXmNone> : nullptr;
+  return a == 1 ? k_split<1, kXmNone, F> : a == 2 ? k_split<2, kXmNone, F> : a == 4 ? k_split<4, kXmNone, F>
+                                       : a == 8 ? k_split<8, kXmNone, F> : nullptr;
 #else
-  if (b != 0) return a == 1 ? k_split<1, kXmCap> : k_split<2, kXmCap>;
-  return a == 1 ? k_split<1, kXmLight> : k_split<2, kXmLight>;
+  constexpr bool F = LLZ_INST == 7;
+  if (b != 0) return a == 1 ? k_split<1, kXmCap, F> : k_split<2, kXmCap, F>;
+  return a == 1 ? k_split<1, kXmLight, F> : k_split<2, kXmLight, F>;
 #endif
 }
 
