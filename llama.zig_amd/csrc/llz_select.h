@@ -755,9 +755,9 @@ constexpr int kShortMax = 256;  // longest candidate list of the short path
 // Sort of the candidate list sh.cand[0, c) (c <= kCap distinct keys,
 // ascending).  The keys' upper words span few octaves of p, so equal steps of
 // them make kSortBins bins of a few keys each: counts, an exclusive scan, the
-// keys scattered to their bins, and each bin's few keys put in order by one
-// thread: five barriers, where the bitonic network takes one per stage (66
-// for 2048 keys: 40 us of a row, now @SORTUS@).  Lists with a long bin (many equal or near
+// keys scattered to their bins, and each key's place counted among its bin's:
+// five barriers, where the bitonic network takes one per stage (66
+// for 2048 keys: 37 us of a row, now 4).  Lists with a long bin (many equal or near
 // p) and short lists take the network.
 constexpr int kSortBins = 2048;
 constexpr int kSortBinMax = 24;
@@ -802,10 +802,8 @@ __device__ __noinline__ void sort_list(SampleShared& sh_arg, int c, int& bank) {
     }
     bank ^= 1;
     if (!too_long) {
-      uint32_t first[PT];
 #pragma unroll
       for (int q = 0; q < PT; ++q) {
-        first[q] = run;
         cnt[t * PT + q] = run;
         run += v[q];
       }
@@ -815,15 +813,16 @@ __device__ __noinline__ void sort_list(SampleShared& sh_arg, int c, int& bank) {
         sh.u.post.aux[atomicAdd(&cnt[((uint32_t)(k >> 32) - lo) >> shift], 1u)] = k;
       }
       lds_barrier();
-      // each key's place in its bin: the bin's smaller keys
-#pragma unroll
-      for (int q = 0; q < PT; ++q) {
-        for (uint32_t i = 0; i < v[q]; ++i) {
-          const uint64_t k = sh.u.post.aux[first[q] + i];
-          uint32_t r = 0u;
-          for (uint32_t j = 0; j < v[q]; ++j) r += sh.u.post.aux[first[q] + j] < k ? 1u : 0u;
-          sh.cand[first[q] + r] = k;
-        }
+      // each key's place in its bin (which ends where its next place stands
+      // now, and starts at the end of the bin before): the bin's smaller keys
+      for (int i = t; i < c; i += kNT) {
+        const uint64_t k = sh.u.post.aux[i];
+        const uint32_t b = ((uint32_t)(k >> 32) - lo) >> shift;
+        const uint32_t e = cnt[b], s = b > 0u ? cnt[b - 1u] : 0u;
+        uint32_t r = 0u;
+#pragma unroll 4
+        for (uint32_t j = s; j < e; ++j) r += sh.u.post.aux[j] < k ? 1u : 0u;
+        sh.cand[s + r] = k;
       }
       lds_barrier();
       return;
@@ -1227,6 +1226,7 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
     sort_list(sh, c, bank);
   }
 
+  LLZ_STAMP(row, 56);
   // certified prefix: every element outside the list has p <= theta / S
   int M = 0;
   if (!ovf) {
@@ -1244,18 +1244,34 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
   // a complete list bounds everything outside it: e < theta, p <= theta / S
   const float p_nc = ovf ? kInf : Pl.cand_theta / S;
   K = prefix_filters(LL, M, p_nc, n, P, S, sh, bank);
+  LLZ_STAMP(row, 57);
   const bool typical = P.typical_p > 0.0f && P.typical_p < 1.0f;
   const float u = u_row;
   bool fallback = K < 0;
+  // Typical-p alone (no prefix filter: every element is selected) keeps the
+  // head of the order by dev = |surprise - H| up to where its running sum
+  // passes typical_p.  An element outside the certified prefix has p <=
+  // p_nc, so its surprise is at least that of p_nc (logf within an ulp:
+  // 2^-21) and its dev at least dev_nc when that lies above H: a cut among
+  // the list's terms at a dev below dev_nc is the row's cut, whatever lies
+  // outside the list.  The heavy-tailed rows that typical-p is used on cut
+  // among their largest few dozen terms, and need neither the dev keys of the
+  // whole row nor their sort (626 us of a 151936-logit row).
+  const bool lazy = fallback && typical && !ovf && M >= 1 && M < n && Pl.cand_theta > 0.0f &&
+                    !((P.top_k > 0 && P.top_k < (uint32_t)n) || (P.top_p > 0.0f && P.top_p < 1.0f) || P.min_p > 0.0f);
+  if (lazy) {
+    K = M;
+    fallback = false;
+  }
 
   if (!fallback) {
     // ---- 5. typical-p on the kept prefix (:128-154)
     for (int q = t; q < kCap; q += kNT) sh.u.post.keep[q] = q < K ? 1 : 0;
     lds_barrier();
-    if (typical && K == 1) {
+    if (typical && K == 1 && !lazy) {
       if (t == 0 && LL.p(0) > P.typical_p) sh.u.post.keep[0] = 0;
       lds_barrier();
-    } else if (typical && K >= 2) {
+    } else if (typical && (K >= 2 || lazy)) {
       path |= kPathEntropy;
       {
         const EntropyResult er = entropy_pass<Src>(X, n, m, S, P.temperature, P.flags, sh, bank, row);
@@ -1281,14 +1297,21 @@ __device__ __forceinline__ void select_row(const RowParams& P, const RowPtrs& Q,
       int st;
       seq_accumulate<false>(0.0f, K, P.typical_p, st, [&](int d) { return LL.p((int)sh.u.post.aux_pos[d]); },
                             sh, bank);
+      if (lazy) {
+        const float dev_nc = (-log_f32(p_nc) * (1.0f - 0x1p-21f) - H) * (1.0f - 0x1p-22f);
+        fallback = !(st >= 0 && __uint_as_float((uint32_t)(sh.u.post.aux[max(st, 0)] >> 32)) < dev_nc);
+      }
       if (st >= 0) {
         for (int d = st + t; d < K; d += kNT) sh.u.post.keep[sh.u.post.aux_pos[d]] = 0;
       }
       lds_barrier();
     }
+  }
+  if (!fallback) {
     // ---- 6. total and draw (:156-168)
     total_and_draw(LL, K, [&](int q) { return sh.u.post.keep[q] != 0; }, u, total, token, consumed, sh, bank);
 
+    LLZ_STAMP(row, 58);
     // ---- outputs
     uint32_t kept = 0;
     for (int q = t; q < K; q += kNT) kept += sh.u.post.keep[q];

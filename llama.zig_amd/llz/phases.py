@@ -40,6 +40,7 @@ SLOTS = {
     46: "L: load loop done (wave 0)",
     48: "entropy: first 512 terms", 49: "entropy: tile 0", 50: "entropy: tile 1", 51: "entropy: tile 16",
     52: "entropy: last tile",
+    56: "list: sorted", 57: "list: filters", 58: "list: total and draw",
 }
 # phases as (name, from slot, to slot)
 PHASES = [
@@ -62,6 +63,7 @@ PHASES = [
     ("decisions: draw", 36, 37), ("decisions: outputs + barrier", 37, 15),
     ("recollect: histogram pass", 6, 40), ("recollect: cut", 40, 41), ("recollect: collect pass", 41, 42),
     ("after recollect: sort, filters, draw", 42, 15),
+    ("list: read, sort", 6, 56), ("list: filters", 56, 57), ("list: total, draw", 57, 58), ("list: outputs", 58, 15),
     ("penalty: list -> L end", 43, 1), ("penalty: patch (after loads)", 0, 44), ("penalty: loop end -> patched", 46, 44),
     ("penalty: patched -> list built", 44, 43),
     ("transforms: maximum (from start)", 0, 45), ("transforms: patch -> maximum", 44, 45),
