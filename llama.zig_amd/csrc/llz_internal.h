@@ -10,6 +10,8 @@ typedef float llz_f4v __attribute__((ext_vector_type(4)));  // four floats as on
 typedef float llz_f4u __attribute__((ext_vector_type(4), aligned(4)));  // the same from any 4-byte aligned address
 
 constexpr int kCandCap = 2048;  // candidate list capacity per row (power of two)
+constexpr int kResidentMax = 129024;  // logits of a row the single pass keeps in registers and LDS
+constexpr int kLongMax = 262144;      // logits of a row of k_long at most (128 segments per wave)
 constexpr int kPenMax = 64;     // fused repetition penalty: window entries at most (one per lane)
 constexpr int kQovfWave = 4096;  // k_stats special-queue overflow entries per wave
 constexpr int kQovfRow = 8 * kQovfWave;  // ... per workgroup (eight waves)
@@ -36,6 +38,8 @@ constexpr uint32_t kFlagVecSrc = 2u;    // the rows the chain reads are 16-byte 
 constexpr uint32_t kFlagFallback = 4u;  // the full-row fallback buffers are present
 constexpr uint32_t kFlagTokenOnly = 8u;  // no probabilities or row statistics requested: the token alone
 constexpr uint32_t kFlagXfExact = 16u;   // transformed rows the single pass cannot estimate: the exact streaming path
+
+constexpr uint32_t kFlagLong = 32u;      // rows of k_long: beyond the single pass's residency, up to kLongMax logits
 
 // RowParams.xf_src / xf_orig: transforms applied as a row is read
 constexpr uint32_t kXfCap = 1u;    // v = tanh(v / cap) * cap   (main.zig:653-658)

@@ -15,6 +15,7 @@ StatsKernel stats_kernel_5(int, int);
 StatsKernel stats_kernel_6(int, int);
 StatsKernel stats_kernel_7(int, int);
 StatsKernel stats_kernel_8(int, int);
+StatsKernel stats_kernel_9(int, int);
 
 // Every row's statistics, then its selection.
 hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_begin, hipEvent_t ev_end,
@@ -39,6 +40,8 @@ hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_beg
   if (split)
     kern = xm == kXmNone ? (fastld ? stats_kernel_5(P.split_nv, 0) : stats_kernel_6(P.split_nv, 0))
                          : (fastld ? stats_kernel_7 : stats_kernel_8)(P.split_nv, xm == kXmCap);
+  else if (P.flags & kFlagLong)
+    kern = stats_kernel_9(fastld, xm);
   else if (xm == kXmCap)
     kern = stats_kernel_4(fastld, claim);
   else if (xm == kXmLight)
@@ -67,6 +70,7 @@ extern "C" int llz_stamps_5(unsigned long long*, int, int);
 extern "C" int llz_stamps_6(unsigned long long*, int, int);
 extern "C" int llz_stamps_7(unsigned long long*, int, int);
 extern "C" int llz_stamps_8(unsigned long long*, int, int);
+extern "C" int llz_stamps_9(unsigned long long*, int, int);
 
 // Measurement builds: the phase timestamps of rows 0 .. rows - 1 (kStampSlots
 // per row, 0 where a row did not reach the boundary) into dst.
@@ -74,7 +78,7 @@ extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int cle
   if (rows <= 0 || rows > llz::kStampRows || !dst) return -1;
   static int (*const get[])(unsigned long long*, int, int) = {llz_stamps_0, llz_stamps_1, llz_stamps_2, llz_stamps_3,
                                                               llz_stamps_4, llz_stamps_5, llz_stamps_6, llz_stamps_7,
-                                                              llz_stamps_8};
+                                                              llz_stamps_8, llz_stamps_9};
   static unsigned long long part[llz::kStampRows * llz::kStampSlots];
   const size_t n = (size_t)rows * llz::kStampSlots;
   if (!clear)

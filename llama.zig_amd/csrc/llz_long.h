@@ -1,0 +1,280 @@
+// llz_long.h -- rows beyond the single pass's residency (129024 logits, up to
+// kLongMax): k_long, one workgroup per row.
+//
+// k_stats keeps a row's estimates in registers and LDS; a longer row does
+// not fit, and its streaming normaliser (llz_norm.h) reads the row twice
+// after a scan for the maximum, with two barriers per 8192 logits: 256 us for a
+// 151936-logit row, also where the call asks for the token alone.  Here the
+// row is streamed once, a window of kLongU segment loads in flight per wave:
+// per 256-logit segment the running maximum and the sum of the estimates q =
+// exp2(v l2e - c_w) (phase L of k_stats), and, on token-only calls, the
+// elements that may be candidates.  Those are pushed as they pass: an element
+// whose term may reach tok_theta against the row's maximum reaches it
+// against any smaller one, so the test against the wave's running maximum
+// (lagging by at most a window) collects a superset; a full buffer is
+// filtered again against the maximum reached.  token_select then decides the
+// row as on k_stats's token path (s_est and w_est from the segment sums).
+// A row it does not decide, and every row of the other calls, goes on to the
+// selection stage with the maximum known.
+//
+// 64 rows of 151936 logits with top-k, top-p and min-p: 303 us before, 35 us
+// now.  Bound by one CU's share of HBM while
+// the rows are fewer than the CUs.
+#pragma once
+
+#include "llz_fast.h"
+#include "llz_select.h"
+#include "llz_token.h"
+
+namespace llz {
+
+constexpr int kLongU = 8;        // segment loads in flight per wave
+constexpr int kLongBuf = 512;    // candidate buffer entries per wave
+
+struct LongShared {
+  uint64_t tl[2 * kTokCap];                      // collected, then sorted
+  uint8_t part[(kNT / kWave) * kTokCap];         // token_sort's partial ranks
+  float bv[kNT / kWave][kLongBuf];               // per wave: candidates' logits
+  uint32_t bp[kNT / kWave][kLongBuf];            //   and positions
+  float mw[kNT / kWave], cw[kNT / kWave], qs[kNT / kWave], qw[kNT / kWave];
+  uint32_t tcand, tfail;
+};
+
+union LongLds {
+  LongShared lng;
+  SampleShared select;
+};
+
+template <bool FASTLD, int XM>
+__device__ __forceinline__ void long_row(const KArgs& A, int row, LongLds& U, PenShared& pen_sh, int wslot) {
+  constexpr int W = kNT / kWave, SEG = fastp::SEG;
+  constexpr bool XF = XM != kXmNone;
+  const RowParams& P = A.P;
+  const RowPtrs& Q = A.Q;
+  LongShared& F = U.lng;
+  LLZ_STAMP(row, 0);
+  const int t = (int)threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const int n = P.n;
+  const bool t1 = (P.flags & kFlagTIsOne) != 0u;
+  const float T = P.temperature, l2e = P.l2e_t;
+  using Src = typename std::conditional<XM == kXmCap, RowSrc,
+                                        typename std::conditional<XF, LightSrc, PlainSrc>::type>::type;
+  using OSrc = typename std::conditional<XF, RowSrc, PlainSrc>::type;
+  const float* xr = Q.src + (int64_t)row * P.src_stride;
+  const Src X = make_src<Src>(P, Q, row, &pen_sh);
+  OSrc O;
+  if constexpr (XF) {
+    O = row_orig(P, Q, row);
+  } else {
+    O = PlainSrc{Q.orig + (int64_t)row * P.orig_stride};
+  }
+  const float u_row = Q.uniforms[row];
+  if constexpr (XF) {
+    if (P.xf_src & kXfPen) {  // each id < n penalised once (sampler.zig:62-70)
+      const uint32_t id = pen_window_id(P, Q, row);
+      bool first = id < (uint32_t)n;
+      for (int j = 0; j < P.pen_w; ++j) {
+        const uint32_t o = readlane_u32(id, j);
+        first = first && !(j < lane && o == id);
+      }
+      pen_list(pen_sh, first ? id : (id | 0x80000000u));
+    }
+  }
+  if (t == 0) {
+    F.tcand = 0u;
+    F.tfail = 0u;
+  }
+  lds_barrier();
+
+  const int G = (n + SEG - 1) / SEG;
+  const int nseg = max(0, (G - w + W - 1) / W);  // wave w: segments w, w + W, ...
+  const bool tok = (P.flags & kFlagTokenOnly) != 0u && P.tok_theta > 0.0f && l2e > 0.0f && l2e <= 0x1p40f;
+  // an element passes while v >= mx - dv: its term may reach tok_theta
+  // against the maximum mx seen so far (2^-8 octaves to spare for the
+  // roundings here and of the reference's argument)
+  const float dv = tok ? (-__builtin_amdgcn_logf(P.tok_theta) + 0x1p-8f) / l2e * (1.0f + 0x1p-20f) : 0.0f;
+  // (nothing passes before a finite logit was seen)
+  auto thr_of = [&](float x) { return x > -kInf ? x - dv - fabsf(x) * 0x1p-22f : kInf; };
+  float mx = -kInf, cw = 0.0f, thr = kInf;
+  float qsum = 0.0f, qwsum = 0.0f;  // lane 63: the wave's sum of estimates, and weighted by n - the segment's start
+  int nb = 0;                       // the wave's buffered candidates
+  bool ovf = false;
+  const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+  auto load = [&](int k) -> float4 {
+    const int pos = (w + W * k) * SEG + lane * 4;
+    if constexpr (FASTLD) {
+      const float4 v = ld_nt4(xr + (k < nseg && pos < n ? pos : 0));
+      return k < nseg && pos < n ? v : make_float4(-kInf, -kInf, -kInf, -kInf);
+    } else {
+      return rd4_any(xr, k < nseg ? pos : n, n);
+    }
+  };
+  // drop the buffered elements below the threshold reached
+  auto compact = [&]() {
+    int o = 0;
+    for (int b = 0; b < nb; b += kWave) {
+      const int i = b + lane;
+      const float v = i < nb ? F.bv[w][i] : -kInf;
+      const uint32_t p = i < nb ? F.bp[w][i] : 0u;
+      const bool keep = i < nb && v >= thr;
+      const uint64_t km = bal64(keep);
+      __builtin_amdgcn_wave_barrier();
+      if (keep) {
+        const int s = o + (int)__popcll(km & lt);  // s <= i: never past what is still to be read
+        F.bv[w][s] = v;
+        F.bp[w][s] = p;
+      }
+      o += (int)__popcll(km);
+      __builtin_amdgcn_wave_barrier();
+    }
+    nb = o;
+  };
+  float4 cur[kLongU], nxt[kLongU];
+#pragma unroll
+  for (int u = 0; u < kLongU; ++u) cur[u] = load(u);
+  for (int k0 = 0; k0 < nseg; k0 += kLongU) {
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u) nxt[u] = load(k0 + kLongU + u);
+    if constexpr (XF) {
+#pragma unroll
+      for (int u = 0; u < kLongU; ++u) cur[u] = X.fix4((w + W * (k0 + u)) * SEG + lane * 4, cur[u], k0 + u < nseg ? n : 0);
+    }
+    float ml = -kInf;
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)  // fmaxf skips NaN (sampler.zig:80-81)
+      ml = fmaxf(ml, fmaxf(fmaxf(cur[u].x, cur[u].y), fmaxf(cur[u].z, cur[u].w)));
+    ml = wave_max_f32(ml);
+    mx = fmaxf(mx, ml);
+    if (k0 == 0) cw = (fabsf(mx) <= 3.0e38f ? mx : 0.0f) * l2e;
+    thr = thr_of(mx);
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u) {
+      const int seg0 = (w + W * (k0 + u)) * SEG;
+      const float4 v = cur[u];
+      const float q0 = __builtin_amdgcn_exp2f(fmaf(v.x, l2e, -cw)), q1 = __builtin_amdgcn_exp2f(fmaf(v.y, l2e, -cw));
+      const float q2 = __builtin_amdgcn_exp2f(fmaf(v.z, l2e, -cw)), q3 = __builtin_amdgcn_exp2f(fmaf(v.w, l2e, -cw));
+      const float a = wave_fold_f32((q0 + q1) + (q2 + q3));
+      qsum += a;
+      qwsum += a * (float)(n - min(seg0, n));
+      if (tok) {
+        const bool hit = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)) >= thr;
+        if (bal64(hit) != 0ull) {
+          if (nb > kLongBuf - SEG) {
+            compact();
+            ovf = ovf || nb > kLongBuf - SEG;
+            if (ovf) nb = 0;
+          }
+          const float vs[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const bool in = vs[c] >= thr;
+            const uint64_t im = bal64(in);
+            if (in) {
+              const int s = nb + (int)__popcll(im & lt);
+              F.bv[w][s] = vs[c];
+              F.bp[w][s] = (uint32_t)(seg0 + lane * 4 + c);
+            }
+            nb += (int)__popcll(im);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u) cur[u] = nxt[u];
+  }
+  if (lane == kWave - 1) {
+    F.qs[w] = qsum;
+    F.qw[w] = qwsum;
+  }
+  if (lane == 0) {
+    F.mw[w] = mx;
+    F.cw[w] = cw;
+    if (ovf) F.tfail = 1u;
+  }
+  lds_barrier();
+  LLZ_STAMP(row, 1);
+  float m = -kInf, s_est = 0.0f, w_est = 0.0f;
+  bool bad = false, nanrow = false;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    m = fmaxf(m, F.mw[i]);
+    nanrow = nanrow || F.qs[i] != F.qs[i];  // q >= 0 otherwise, so no inf - inf
+  }
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const float awi = fmaf(m, -l2e, F.cw[i]);
+    const float ri = __builtin_amdgcn_exp2f(awi);
+    bad = bad || (G > i && !(fabsf(awi) <= 64.0f));
+    s_est += G > i ? F.qs[i] * ri : 0.0f;
+    w_est += G > i ? F.qw[i] * ri : 0.0f;
+  }
+  // a NaN logit or an infinite maximum makes the reference's sum NaN: the
+  // selection stage handles that row
+  const bool nan_sum = nanrow || !(fabsf(m) <= 3.0e38f);
+  if (tok && !bad && !nan_sum && F.tfail == 0u) {
+    const float theta = P.tok_theta;
+    thr = thr_of(m);
+    for (int b = 0; b < nb; b += kWave) {
+      const int i = b + lane;
+      const float v = i < nb ? F.bv[w][i] : -kInf;
+      const bool live = i < nb && v >= thr;
+      if (bal64(live) == 0ull) continue;
+      const float e = live ? exact_term(v, m, T, t1) : 0.0f;  // sampler.zig:85
+      const bool cand = live && e >= theta;
+      const uint64_t cb = bal64(cand);
+      if (cb != 0ull) {
+        uint32_t b0 = 0u;
+        if (lane == 0) b0 = atomicAdd(&F.tcand, (uint32_t)__popcll(cb));
+        const uint32_t s = readlane_u32(b0, 0) + (uint32_t)__popcll(cb & lt);
+        if (cand && s < (uint32_t)kTokCap) F.tl[s] = ((uint64_t)(~__float_as_uint(e)) << 32) | F.bp[w][i];
+      }
+    }
+    lds_barrier();
+    LLZ_STAMP(row, 33);
+    const int tc = (int)F.tcand;
+    if (tc <= kTokCap) {
+      token_sort(F.tl, F.tl + kTokCap, F.part, tc);
+      LLZ_STAMP(row, 34);
+      if (w == 0) {
+        // typical-p: decided where it drops nothing or nothing is kept
+        // before it (no interval of the entropy here)
+        if (P.typical_p > 0.0f && P.typical_p < 1.0f)
+          token_select<true>(kernel_args_ptr(), row, F.tl + kTokCap, tc, s_est, w_est, 0.0, -1.0, u_row, theta, &F.tfail);
+        else
+          token_select<false>(kernel_args_ptr(), row, F.tl + kTokCap, tc, s_est, w_est, 0.0, -1.0, u_row, theta, &F.tfail);
+      }
+      lds_barrier();
+      if (F.tfail == 0u) {
+        LLZ_STAMP(row, 15);
+        return;
+      }
+    }
+  }
+  lds_barrier();  // every wave is done with F: the selection stage takes the memory
+  select_row(P, Q, U.select, m, nan_sum ? __builtin_nanf("") : 0.0f, 0u, !nan_sum, u_row, false, 0ull, 0u, X, O, XF ? &pen_sh : nullptr, kernel_args_ptr(), row,
+             wslot, P.cand_theta);
+  LLZ_STAMP(row, 15);
+}
+
+// One workgroup per row, or (claim) one per CU taking further rows as
+// k_stats_rows does.
+template <bool FASTLD, int XM>
+__global__ __launch_bounds__(kNT) void k_long(KArgs A) {
+  __shared__ LongLds U;
+  __shared__ PenShared pen_sh;
+  __shared__ int next_row;
+  for (int row = (int)blockIdx.x;;) {
+    const __attribute__((address_space(4))) KArgs* Ap =
+        (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(Ap));
+    long_row<FASTLD, XM>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
+    if (A.P.grid >= A.P.rows) return;
+    if (threadIdx.x == 0) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid);
+    __syncthreads();
+    row = next_row;
+    if (row >= A.P.rows) return;
+  }
+}
+
+}  // namespace llz

@@ -505,32 +505,6 @@ union StatsShared {
   SampleShared select;  // then the selection stage
 };
 
-// The next row beyond the grid for a workgroup that finished one: a counter
-// word tagged with the low 40 bits of the call's epoch (a word left by
-// another call, or not yet written, counts as 0 for this one).  Returns grid +
-// the count before the claim (>= rows: nothing left).  The first claim of a
-// call installs its tag (compare-and-swap); every later one is a single
-// fetch-and-add, which the device serves back to back, where a
-// compare-and-swap loop lets one claim through per round trip to memory
-// (with rows of some 40 us, the workgroups then queued for their claims).
-// The count stays below 2^24: at most rows + grid claims.
-__device__ __noinline__ int claim_row(unsigned long long* word, unsigned long long epoch, int grid) {
-  constexpr unsigned long long kCnt = (1ull << 24) - 1;
-  const unsigned long long tag = (epoch & ((1ull << 40) - 1)) << 24;
-  unsigned long long old = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (;;) {
-    if ((old & ~kCnt) == tag) {
-      const unsigned long long prev = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return grid + (int)(prev & kCnt);
-    }
-    unsigned long long expected = old;
-    if (__hip_atomic_compare_exchange_strong(word, &expected, tag | 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT))
-      return grid;
-    old = expected;
-  }
-}
-
 // FASTLD: 16-byte aligned rows with n % 4 == 0; otherwise rows of any length
 // and (4-byte) alignment, through the same 16-byte loads, which need 4-byte
 // alignment only, with the last n % 4 logits taken after the loop.  (Element

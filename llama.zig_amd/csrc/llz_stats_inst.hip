@@ -5,6 +5,8 @@
 //        with typical-p, soft-capped (a: 16-byte aligned rows; b: claimed rows)
 //   5, 6 k_split on plain rows: 16-byte aligned, any (a: float4 per thread)
 //   7, 8 k_split on transformed rows, the same (a: float4 per thread; b: soft-capped)
+//   9    k_long (a: 16-byte aligned rows; b: transform mode)
+#include "llz_long.h"
 #include "llz_stats.h"
 
 #ifndef LLZ_INST
@@ -26,6 +28,10 @@ StatsKernel LLZ_CAT(stats_kernel_, LLZ_INST)(int a, int b) {
   (void)b;
   return a == 1 ? k_split<1, kXmNone, F> : a == 2 ? k_split<2, kXmNone, F> : a == 4 ? k_split<4, kXmNone, F>
                                        : a == 8 ? k_split<8, kXmNone, F> : nullptr;
+#elif LLZ_INST == 9
+  if (b == kXmCap) return a != 0 ? k_long<true, kXmCap> : k_long<false, kXmCap>;
+  if (b == kXmLight) return a != 0 ? k_long<true, kXmLight> : k_long<false, kXmLight>;
+  return a != 0 ? k_long<true, kXmNone> : k_long<false, kXmNone>;
 #else
   constexpr bool F = LLZ_INST == 7;
   if (b != 0) return a == 1 ? k_split<1, kXmCap, F> : k_split<2, kXmCap, F>;

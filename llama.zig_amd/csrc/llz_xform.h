@@ -77,11 +77,12 @@ __device__ __forceinline__ float cap_est(float r, float a2, float c) {
 __device__ __forceinline__ float pen_est(float v, float rp, float rp_inv) { return v > 0.0f ? v * rp_inv : v * rp; }
 
 // The penalised positions of one row, ascending, and for each of the
-// single-pass kernel's eight waves the segments (256 logits; wave w owns
-// segments w, w + 8, ...) holding one: bit k of wmask[w] for segment w + 8k.
+// kernels' eight waves the segments (256 logits; wave w owns segments w,
+// w + 8, ...) holding one: bit k % 64 of wmask[w + 8 (k / 64)] for segment
+// w + 8k, k < 128.
 struct PenShared {
   uint32_t pos[kPenMax];
-  uint64_t wmask[8];
+  uint64_t wmask[16];
   int n;
 };
 
@@ -111,11 +112,11 @@ __device__ __forceinline__ void pen_list(PenShared& ps, uint32_t idf) {
     const uint32_t o = readlane_u32(id, __ffsll((long long)bm) - 1);
     rank += o < id ? 1u : 0u;
     const uint32_t g = o >> 8;  // its segment
-    if ((int)(g & 7u) == lane && (g >> 3) < 64u) wm |= 1ull << (g >> 3);
+    if ((int)((g & 7u) | ((g >> 9) << 3)) == lane) wm |= 1ull << ((g >> 3) & 63u);  // lane < 16: g < 1024
   }
   if (first) ps.pos[rank] = id;
   if (lane == 0) ps.n = __popcll(km);
-  if (lane < 8) ps.wmask[lane] = wm;
+  if (lane < 16) ps.wmask[lane] = wm;
 }
 
 // A row of logits as the chain reads it (see the file comment).  CAP =
@@ -140,7 +141,7 @@ struct RowSrcT {
   __device__ __forceinline__ bool penalised(int i) const {
     // the segment's bit first (one LDS read; most segments hold none)
     const uint32_t g = (uint32_t)i >> 8;
-    if ((g >> 3) < 64u && ((pen->wmask[g & 7u] >> (g >> 3)) & 1ull) == 0ull) return false;
+    if (g < 1024u && ((pen->wmask[(g & 7u) | ((g >> 9) << 3)] >> ((g >> 3) & 63u)) & 1ull) == 0ull) return false;
     const int np = pen->n;
     // lower bound of i in the sorted list
     int lo = 0, hi = np;

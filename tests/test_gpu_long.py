@@ -1,0 +1,107 @@
+"""Rows beyond the single pass's residency (129024 logits) on k_long, against
+the oracle: the shortest and longest such rows, remainders and unaligned rows,
+token-only and exact calls, every transform, penalised positions past segment
+512, special values, candidate buffers that fill and overflow; and typical-p
+decided from the candidate list, inside it and past it."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import llz
+import oracle_lib as O
+from llz.workloads import Params
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+FILTERS = Params(1.0, 40, 0.95, 0.05, 1.0, 0, 1.0)
+DEFAULT = Params(0.8, 0, 0.9, 0.0, 1.0, 0, 1.0)
+FULL = Params(0.8, 50, 0.9, 0.02, 0.98, 0, 1.0)
+TYPICAL = Params(0.7, 0, 1.0, 0.0, 0.95, 0, 1.0)
+
+
+def _rows(n, seed):
+    g = np.random.default_rng([n, seed])
+    x = g.normal(0.0, 2.5, size=(8, n)).astype(np.float32)
+    x -= (1.1 * np.log(g.permuted(np.tile(np.arange(1, n + 1), (8, 1)), axis=1))).astype(np.float32)
+    x[1, -1] = 30.0                              # the maximum is the row's last logit
+    x[2] = np.sort(x[2])                         # the running maximum rises to the end: buffers refiltered
+    x[3] = np.float32(0.5)                       # all equal: buffers overflow
+    x[4, :n // 2] = -np.inf
+    x[5, g.integers(0, n, 3)] = np.nan
+    x[6, 7] = np.inf
+    x[7] = g.normal(0.0, 2.0, n).astype(np.float32)
+    x[7, ::9973] += 14.0
+    return x
+
+
+def _check(x, params, *, post=None, prev=None, offset=0, pad=0, exact=False):
+    rows, n = x.shape
+    u = llz.rng_uniforms(5, rows)
+    flat = torch.zeros(rows * (n + pad) + offset, dtype=torch.float32, device="cuda")
+    xd = flat[offset:].view(rows, n + pad)[:, :n]
+    xd.copy_(torch.from_numpy(x))
+    pv = None if prev is None else torch.from_numpy(prev.astype(np.int32)).cuda()
+    llz.debug_set_split(1)
+    try:
+        r = llz.sample_rows(xd, llz.SamplerConfig.of(params), torch.from_numpy(u).cuda(), pv, post=post, kept_cap=64,
+                            probs=exact, stats=exact, path=True)
+        torch.cuda.synchronize()
+    finally:
+        llz.debug_set_split(0)
+    tok, con = r.tokens.cpu().numpy().view(np.uint32), r.consumed.cpu().numpy()
+    kc, ids = r.kept_count.cpu().numpy().view(np.uint32), r.kept_ids.cpu().numpy().view(np.uint32)
+    xs = x if post is None else O.logit_post(x, post.final_logit_softcapping, post.logit_scale)
+    for i in range(rows):
+        o = O.sample_row(xs[i], params, u[i], prev_tokens=None if prev is None else prev[i])
+        ctx = (i, hex(int(r.row_path[i].item()) & 0xFFFFFFFF))
+        assert (tok[i], con[i], kc[i]) == (o.token, o.consumed, o.kept_count), ctx
+        k = min(o.kept_count, 64)
+        assert np.array_equal(ids[i, :k], o.kept_ids()[:k]), ctx
+    return r.row_path.cpu().numpy().view(np.uint32)
+
+
+@pytest.mark.parametrize("n,offset,pad", [(129028, 0, 0), (129025, 1, 0), (131075, 3, 5), (151936, 0, 0),
+                                          (262143, 2, 1), (262144, 0, 0), (262145, 1, 0)])
+@pytest.mark.parametrize("params", [FILTERS, DEFAULT, FULL], ids=["filters", "default", "full"])
+def test_long_rows_token_call(n, offset, pad, params):
+    path = _check(_rows(n, 1), params, offset=offset, pad=pad)
+    if params is FILTERS and n <= 262144:
+        assert path[0] & llz.PATH_TOKEN_ONLY and path[1] & llz.PATH_TOKEN_ONLY
+
+
+def test_long_rows_exact_call():
+    _check(_rows(140001, 2), FILTERS, exact=True)
+
+
+@pytest.mark.parametrize("n", [129028, 200003])
+@pytest.mark.parametrize("post,window", [((0.0, 0.5), 0), ((30.0, 0.5), 0), ((0.0, 1.0), 40), ((30.0, 1.0), 64),
+                                         ((0.0, 1.0), 200)])
+def test_long_rows_transforms(n, post, window):
+    x = _rows(n, 3)
+    g = np.random.default_rng(n)
+    prev, params = None, FILTERS
+    if window:
+        params = dataclasses.replace(FILTERS, repetition_window=window, repetition_penalty=1.3)
+        prev = g.integers(0, n + 50, size=(x.shape[0], window)).astype(np.uint32)
+        prev[:, 0] = np.nanargmax(x, axis=1)
+        prev[:, 1] = n - 1
+        prev[:, 2] = prev[:, 0]
+    _check(x, params, post=llz.LogitPost(*post), prev=prev)
+
+
+@pytest.mark.parametrize("n", [4099, 60000, 129028, 151936])
+def test_typical_alone(n):
+    """A heavy tail with strong tokens cuts inside the list; flatter rows past it."""
+    g = np.random.default_rng(n)
+    x = g.gumbel(0.0, 1.5, size=(6, n)).astype(np.float32)
+    for r in range(3):
+        x[r, g.choice(n, 20, replace=False)] += np.float32(8.0)
+    x[4] = g.normal(0.0, 0.3, n).astype(np.float32)
+    x[5] = np.round(x[5])  # many equal devs
+    path = _check(x, TYPICAL)
+    assert not np.any(path[:3] & llz.PATH_FULL_SORT), path
+    assert path[4] & llz.PATH_FULL_SORT
+    for p in (0.3, 0.999):
+        _check(x, dataclasses.replace(TYPICAL, typical_p=p), exact=True)
