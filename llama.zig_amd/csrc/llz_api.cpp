@@ -576,24 +576,40 @@ struct llz_sampler {
   hipStream_t stream;
   int32_t cap_n;       // capacity (vocab) of the buffers below
   int32_t cap_prev;
-  float* d_logits;     // staging for host logits
-  uint32_t* d_prev;
-  float* d_u;
-  uint32_t* d_token;
-  uint8_t* d_consumed;
+  // one row's inputs, laid out alike in pinned host memory and on the device
+  // (Stage): the uniform, the history and the logits go over in one go
+  char* h_stage;
+  char* d_stage;
+  struct HostOut {
+    uint32_t token;
+    uint8_t consumed;
+  }* h_out;            // pinned: the kernels write the results here
+  uint32_t* d_token;   // greedy rows: their workgroups combine through the token word, on the device
   void* d_ws;
   size_t ws_bytes;
 };
 
+namespace {
+// Offsets in a row's staging area.
+struct Stage {
+  size_t prev, logits, total;
+  Stage(int32_t n, int32_t n_prev)
+      : prev(16), logits(align_up(16 + (size_t)n_prev * sizeof(uint32_t))),
+        total(align_up(logits + (size_t)n * sizeof(float))) {}
+};
+// Host logits are staged in pieces: while the CPU copies a piece into pinned
+// memory, the GPU reads the one before.
+constexpr size_t kStagePiece = 128u << 10;
+}  // namespace
+
 static void sampler_free_buffers(llz_sampler* s) {
-  (void)hipFree(s->d_logits);
-  (void)hipFree(s->d_prev);
-  (void)hipFree(s->d_u);
+  (void)hipHostFree(s->h_stage);
+  (void)hipHostFree(s->h_out);
+  (void)hipFree(s->d_stage);
   (void)hipFree(s->d_token);
-  (void)hipFree(s->d_consumed);
   (void)hipFree(s->d_ws);
-  s->d_logits = nullptr; s->d_prev = nullptr; s->d_u = nullptr; s->d_token = nullptr;
-  s->d_consumed = nullptr; s->d_ws = nullptr; s->ws_bytes = 0; s->cap_n = 0; s->cap_prev = 0;
+  s->h_stage = nullptr; s->h_out = nullptr; s->d_stage = nullptr; s->d_token = nullptr;
+  s->d_ws = nullptr; s->ws_bytes = 0; s->cap_n = 0; s->cap_prev = 0;
 }
 
 int llz_sampler_create(const llz_sampler_config* cfg, int32_t device, llz_sampler** out) {
@@ -653,45 +669,56 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
   if (hipSetDevice(s->device) != hipSuccess) return LLZ_E_HIP;
   const size_t need_ws = llz_sample_workspace_bytes(1, n, cfg, n_prev);
   if (n > s->cap_n || n_prev > s->cap_prev || need_ws > s->ws_bytes) {
+    const int32_t cn = std::max(n, s->cap_n), cp = std::max(n_prev, s->cap_prev);
+    const size_t cw = std::max(need_ws, s->ws_bytes), st = Stage(cn, cp).total;
     sampler_free_buffers(s);
-    const int32_t cn = n, cp = n_prev > 0 ? n_prev : 1;
-    if (hipMalloc(&s->d_logits, (size_t)cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->d_prev, (size_t)cp * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc(&s->d_u, sizeof(float)) != hipSuccess ||
-        hipMalloc(&s->d_token, sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc(&s->d_consumed, 1) != hipSuccess ||
-        hipMalloc(&s->d_ws, need_ws) != hipSuccess) {
+    if (hipHostMalloc((void**)&s->h_stage, st, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&s->h_out, sizeof(*s->h_out), hipHostMallocDefault) != hipSuccess ||
+        hipMalloc((void**)&s->d_stage, st) != hipSuccess || hipMalloc((void**)&s->d_token, sizeof(uint32_t)) != hipSuccess ||
+        hipMalloc(&s->d_ws, cw) != hipSuccess) {
+      (void)hipGetLastError();
       sampler_free_buffers(s);
       return LLZ_E_OOM;
     }
     s->cap_n = cn;
     s->cap_prev = cp;
-    s->ws_bytes = need_ws;
+    s->ws_bytes = cw;
   }
+  // The inputs through pinned memory, read by a copy kernel on the sampler's
+  // stream; the results written by the sampling kernel into pinned memory.
+  // (Pageable copies of the logits, the history and the uniform, and two
+  // more for the results, took 81 us of a call alone and 148 us back to back.)
+  const Stage at(n, n_prev);
+  std::memcpy(s->h_stage, &u, sizeof(float));
+  if (n_prev > 0) std::memcpy(s->h_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t));
   const float* d_in = logits;
-  if (!is_device_ptr(logits)) {
-    if (hipMemcpyAsync(s->d_logits, logits, (size_t)n * sizeof(float), hipMemcpyHostToDevice,
-                       s->stream) != hipSuccess)
+  const bool on_host = !is_device_ptr(logits);
+  if (on_host) d_in = (const float*)(s->d_stage + at.logits);
+  // the staged bytes [0, end): the head, then with host logits all of them
+  const size_t bytes = (size_t)n * sizeof(float), end = on_host ? at.logits + bytes : at.logits;
+  for (size_t from = 0, off = 0; from < end;) {
+    size_t upto = at.logits;
+    if (on_host) {
+      const size_t piece = std::min(kStagePiece, bytes - off);
+      std::memcpy(s->h_stage + at.logits + off, (const char*)logits + off, piece);
+      off += piece;
+      upto = at.logits + off;
+    }
+    // whole 16-byte units: the areas are padded to 256 bytes, and pieces but the last are whole
+    if (launch_stage(s->d_stage + from, s->h_stage + from, (upto - from + 15) / 16, s->stream) != hipSuccess)
       return LLZ_E_HIP;
-    d_in = s->d_logits;
+    from = upto;
   }
-  if (n_prev > 0 && hipMemcpyAsync(s->d_prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t),
-                                   hipMemcpyHostToDevice, s->stream) != hipSuccess)
-    return LLZ_E_HIP;
-  if (hipMemcpyAsync(s->d_u, &u, sizeof(float), hipMemcpyHostToDevice, s->stream) != hipSuccess)
-    return LLZ_E_HIP;
-  int rc = llz_sample_rows(d_in, n, 1, n, cfg, nullptr, n_prev > 0 ? s->d_prev : nullptr, n_prev, 0,
-                           s->d_u, s->d_token, s->d_consumed, nullptr, s->d_ws, s->ws_bytes,
-                           s->stream);
+  const bool greedy = cfg->temperature <= 0.0f;
+  int rc = llz_sample_rows(d_in, n, 1, n, cfg, nullptr, n_prev > 0 ? (const uint32_t*)(s->d_stage + at.prev) : nullptr,
+                           n_prev, 0, (const float*)s->d_stage, greedy ? s->d_token : &s->h_out->token,
+                           &s->h_out->consumed, nullptr, s->d_ws, s->ws_bytes, s->stream);
   if (rc != LLZ_OK) return rc;
-  uint32_t tok = 0;
-  uint8_t con = 0;
-  if (hipMemcpyAsync(&tok, s->d_token, sizeof(tok), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-      hipMemcpyAsync(&con, s->d_consumed, 1, hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-      hipStreamSynchronize(s->stream) != hipSuccess)
+  if (greedy && hipMemcpyAsync(&s->h_out->token, s->d_token, sizeof(uint32_t), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
     return LLZ_E_HIP;
-  *token = tok;
-  *consumed = (con != 0 && cfg->temperature > 0.0f) ? 1 : 0;
+  if (hipStreamSynchronize(s->stream) != hipSuccess) return LLZ_E_HIP;
+  *token = s->h_out->token;
+  *consumed = (s->h_out->consumed != 0 && !greedy) ? 1 : 0;
   return LLZ_OK;
 }
 

@@ -175,6 +175,7 @@ hipError_t launch_penalty(const float* logits, int64_t stride, int rows, int n, 
 hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, uint32_t xf, float cap,
                          float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
                          uint32_t* path, hipStream_t st);
+hipError_t launch_stage(void* dst, const void* pinned, size_t units16, hipStream_t st);
 hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_begin, hipEvent_t ev_end,
                          hipStream_t st);
 hipError_t launch_math_probe(const float* in, float* out_exp, float* out_log, float* out_expm1, float* out_tanh,

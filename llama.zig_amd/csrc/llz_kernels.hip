@@ -189,8 +189,25 @@ __global__ __launch_bounds__(256) void k_hw_error(int op, uint32_t first, uint32
 }
 
 // ---------------------------------------------------------------------------
+// k_stage: pinned host memory to device memory, 16 bytes per thread.  On the
+// compute queue, so that the sampling kernel behind it needs no signal from
+// a copy engine.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_stage(uint4* __restrict__ dst, const uint4* __restrict__ src, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
+// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
+hipError_t launch_stage(void* dst, const void* pinned, size_t units16, hipStream_t st) {
+  if (units16 == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_stage, dim3((unsigned)((units16 + 255) / 256)), dim3(256), 0, st, (uint4*)dst,
+                     (const uint4*)pinned, (uint32_t)units16);
+  return hipGetLastError();
+}
+
 __global__ void k_zero_u32(uint32_t* p) { *p = 0u; }
 
 hipError_t launch_hw_error(int op, uint32_t first, uint32_t count, uint32_t* max_err, hipStream_t st) {
