@@ -48,11 +48,13 @@ constexpr int kBucketMinN = 8192;  // shorter rows keep the sorting path
 // f32 rounding (each about 2^-24).
 constexpr double kBucketDelta = 0x1p-13;
 constexpr int kCountShift = 44;  // histogram word: count << 44 | sum of scaled significands
-// Bucket arrays are padded by one entry per 64 buckets: wave 0's scans give
-// each lane 64 consecutive buckets, which unpadded would sit in one LDS bank.
+// Bucket arrays are padded by one entry per 64 buckets: wave 0's scan of the
+// list's places gives each lane 64 consecutive buckets, which unpadded would
+// sit in one LDS bank.
 constexpr int kNBP = kNB + kNB / 64;
 __device__ __forceinline__ int bix(int b) { return b + (b >> 6); }
 
+constexpr int kJgBias = 128;  // binades -120 .. 126
 enum : uint8_t { kBNone = 0, kBEmpty = 1, kBPlain = 2, kBExact = 3, kBExactTie = 4 };
 
 struct BucketShared {  // arrays indexed through bix()
@@ -65,12 +67,18 @@ struct BucketShared {  // arrays indexed through bix()
     };
     uint64_t hist[kNBP];   // histogram passes: count << 44 | the significands of p scaled to the bucket's top binade
   };
-  int8_t jg[kNBP];      // PLAIN: the binade of the running value
-  uint8_t cls[kNBP];
-  uint8_t tie[kNBP];    // PLAIN: bit 0 a term is a tie on grid jg, bit 1 the sum reached kSat
+  uint16_t cj[kNBP];    // class (bits 0-2); PLAIN: the binade of the running value, + kJgBias (bits 3-10)
+  uint8_t tie[kNBP];    // PLAIN: a term is a tie on its grid
   uint64_t list[kBList];  // EXACT buckets' elements, (key << 32 | id), sorted
   uint32_t nlist;
   uint32_t ctl[8];
+  __device__ __forceinline__ uint32_t cls(int b) const { return cj[bix(b)] & 7u; }
+  __device__ __forceinline__ int jg(int b) const { return (int)(cj[bix(b)] >> 3) - kJgBias; }
+  __device__ __forceinline__ void set_cls(int b, uint32_t c) { cj[bix(b)] = (uint16_t)((cj[bix(b)] & ~7u) | c); }
+  uint32_t nties, ties[8];  // buckets a tie made EXACT
+  uint16_t run_b[64];       // bucket_order: the list's runs
+  uint32_t wc[8];  // bucket_scan: per wave, its buckets' count and mass
+  double wm[8];
 };
 
 struct BucketResult {
@@ -81,18 +89,68 @@ struct BucketResult {
   uint32_t why;     // the bucket path declined: 1 + step (diagnostic, status bits 8-15)
 };
 
-// Eight stored keys from pos (absent positions: 0xffffffff, which no bucket
-// range holds).
-__device__ __forceinline__ void bucket_keys8(const uint32_t* Kp, int pos, int n, uint32_t (&k)[8]) {
-  if (pos + 8 <= n && (reinterpret_cast<uintptr_t>(Kp + pos) & 15u) == 0u) {
-    const uint4 a = *reinterpret_cast<const uint4*>(Kp + pos);
-    const uint4 b = *reinterpret_cast<const uint4*>(Kp + pos + 4);
-    k[0] = a.x; k[1] = a.y; k[2] = a.z; k[3] = a.w;
-    k[4] = b.x; k[5] = b.y; k[6] = b.z; k[7] = b.w;
-  } else {
+typedef uint32_t llz_u4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// One pass of a workgroup over n elements, V per thread and tile, with the
+// loads of the next kDepth tiles in flight: a pass whose work per tile is
+// short is bound by the bytes it has in flight (8 words per thread took 97-118
+// us over a row's 256000 stored keys, 54-80 with four tiles).  load(pos,
+// out) must not read out of bounds for any pos; body(pos, values) must not
+// hold a barrier.
+template <int NT, int V, int D, typename T, typename Load, typename Body>
+__device__ __forceinline__ void pipelined_tiles(int n, Load load, Body body) {
+  constexpr int TILE = NT * V;
+  const int p0 = (int)threadIdx.x * V;
+  T buf[D][V];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) k[i] = pos + i < n ? Kp[pos + i] : 0xffffffffu;
+  for (int d = 0; d < D; ++d) load(d * TILE + p0, buf[d]);
+  for (int base = 0; base < n; base += D * TILE) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int pos = base + d * TILE + p0;
+      T cur[V];
+#pragma unroll
+      for (int k = 0; k < V; ++k) cur[k] = buf[d][k];
+      if (base + (D + d) * TILE < n) load(pos + D * TILE, buf[d]);
+      if (base + d * TILE < n) body(pos, cur);
+    }
   }
+}
+
+// A pass over a row's stored keys (n >= 8), absent positions as 0xffffffff,
+// which no bucket range holds.
+template <int NT, typename Body>
+__device__ __forceinline__ void key_pass(const uint32_t* Kp, int n, Body body) {
+  const __attribute__((address_space(1))) uint32_t* g = (const __attribute__((address_space(1))) uint32_t*)Kp;
+  pipelined_tiles<NT, 8, 4, uint32_t>(
+      n,
+      [&](int pos, uint32_t (&k)[8]) {
+        const int pc = min(pos, n - 8);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const llz_u4u q = *(const __attribute__((address_space(1))) llz_u4u*)(g + pc + 4 * h);
+          k[4 * h + 0] = q.x; k[4 * h + 1] = q.y; k[4 * h + 2] = q.z; k[4 * h + 3] = q.w;
+        }
+      },
+      [&](int pos, uint32_t (&k)[8]) {
+        if (pos > n - 8) {  // the row's end: read again, element by element
+#pragma unroll
+          for (int i = 0; i < 8; ++i) k[i] = pos + i < n ? g[pos + i] : 0xffffffffu;
+        }
+        body(pos, k);
+      });
+}
+
+// RN(e / S) for 2^-90 <= e <= 1 and 2^-20 <= S <= 2^40 from y = RN(1 / S), by
+// Markstein's method (llz_math.h): the first correction makes the quotient
+// faithful, and the second, from a faithful quotient and the correctly
+// rounded reciprocal, rounds correctly; remainders are exact in an fma, and
+// no operation underflows in this range.  Six operations, where the IEEE
+// division takes about twelve.
+__device__ __forceinline__ float div_by(float e, float S, float y) {
+  const float q0 = e * y;
+  const float q1 = fmaf(fmaf(-S, q0, e), y, q0);
+  return fmaf(fmaf(-S, q1, e), y, q1);
 }
 
 __device__ __forceinline__ float key_p(uint32_t key) { return __uint_as_float(~key); }
@@ -157,18 +215,19 @@ __device__ float wave_seq_stop(float s, int len, float thr, int& stop, float& be
   return s;
 }
 
-// Wave 0: exclusive prefixes of the buckets' counts and masses, 64 buckets a
-// lane; calls cls_of(b, excl_count, excl_mass) for every bucket in order
-// within the lane.
-template <typename ClsFn>
+// Every thread: exclusive prefixes of the buckets' counts and masses, kNB / NT
+// consecutive buckets a thread; calls cls_of(b, excl_count, excl_mass) for
+// each of them in order.  (One wave with 64 buckets a lane took 14-24 us.)
+template <int NT, typename ClsFn>
 __device__ __forceinline__ void bucket_scan(BucketShared& bs, ClsFn cls_of) {
-  constexpr int PL = kNB / kWave;
-  const int lane = lane_id();
+  constexpr int PL = kNB / NT;
+  const int t = (int)threadIdx.x, lane = lane_id(), w = wave_id();
   uint32_t c = 0;
   double ms = 0.0;
+#pragma unroll
   for (int i = 0; i < PL; ++i) {
-    c += bs.cnt[bix(lane * PL + i)];
-    ms += (double)bs.mass[bix(lane * PL + i)];
+    c += bs.cnt[bix(t * PL + i)];
+    ms += (double)bs.mass[bix(t * PL + i)];
   }
   uint32_t ci = c;
   double mi = ms;
@@ -181,14 +240,25 @@ __device__ __forceinline__ void bucket_scan(BucketShared& bs, ClsFn cls_of) {
       mi += om;
     }
   }
+  if (lane == kWave - 1) {
+    bs.wc[w] = ci;
+    bs.wm[w] = mi;
+  }
+  __syncthreads();
   uint32_t ec = ci - c;
   double em = mi - ms;
+  for (int i = 0; i < w; ++i) {
+    ec += bs.wc[i];
+    em += bs.wm[i];
+  }
+#pragma unroll
   for (int i = 0; i < PL; ++i) {
-    const int b = lane * PL + i;
+    const int b = t * PL + i;
     cls_of(b, ec, em);
     ec += bs.cnt[bix(b)];
     em += (double)bs.mass[bix(b)];
   }
+  __syncthreads();
 }
 
 // Bucket of a key in the fine range [kmin, kcut): (key - kmin) >> shift.
@@ -199,60 +269,78 @@ struct BucketRange {
   __device__ __forceinline__ int of(uint32_t key) const { return (int)min((key - kmin) >> shift, (uint32_t)kNB - 1u); }
 };
 
-// Pass B: the PLAIN buckets' integer sums of RN(p / u) on their grids, with
-// tie and saturation flags; then a bucket holding a tie becomes EXACT and one
-// whose sum saturated (a wrong prediction) NONE, where a walk stops.
+// Pass B over [blo, bhi) = the whole range when every EXACT bucket's elements
+// fit the list (`gather`): the PLAIN buckets' integer sums of RN(p / u) on
+// their grids, with tie flags, and the EXACT buckets' elements put in their
+// places of the list (bs.off, each bucket's run in any order).  Then a bucket
+// holding a tie becomes EXACT: with `gather`, ExactTie, still to be gathered.
 template <int NT>
-__device__ void bucket_sums(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs) {
+__device__ void bucket_sums(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs, bool gather) {
   const int t = (int)threadIdx.x;
   for (int b = t; b < kNB; b += NT) {
     bs.sum[bix(b)] = 0u;
     bs.tie[bix(b)] = 0u;
   }
   __syncthreads();
-  for (int base = 0; base < n; base += NT * 8) {
-    const int pos = base + t * 8;
-    uint32_t k[8];
-    bucket_keys8(Kp, pos, n, k);
+  // per element one LDS read (its bucket's class and grid, all eight in
+  // flight) and one atomic without a result; the few EXACT elements, whose
+  // atomics return their place, follow one per lane and step
+  key_pass<NT>(Kp, n, [&](int pos, uint32_t (&k)[8]) {
+    uint32_t bb[8], cj[8], ex = 0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (!br.in(k[i])) continue;
-      const int b = br.of(k[i]);
-      if (bs.cls[bix(b)] == kBPlain) {
-        bool tie;
-        const uint32_t r = grid_round(key_p(k[i]), bs.jg[bix(b)], tie);  // <= kSat
-        // terms <= kSat and a flag once the sum reaches kSat: no wrap goes unseen
-        const uint32_t old = atomicAdd(&bs.sum[bix(b)], r);
-        if (tie) bs.tie[bix(b)] |= 1u;
-        if (old >= kSat) bs.tie[bix(b)] |= 2u;
-      }
+      const bool in = br.in(k[i]);
+      bb[i] = (uint32_t)bix(in ? br.of(k[i]) : 0);
+      cj[i] = in ? bs.cj[bb[i]] : 0u;
     }
-  }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t cl = cj[i] & 7u;
+      bool tie;
+      const uint32_t r = grid_round(key_p(k[i]), (int)(cj[i] >> 3) - kJgBias, tie);
+      // a PLAIN bucket's mass lies within one binade, 2^23 units of its grid:
+      // its sum cannot wrap
+      if (cl == kBPlain) {
+        atomicAdd(&bs.sum[bb[i]], r);
+        if (tie) bs.tie[bb[i]] = 1u;
+      }
+      ex |= (cl == kBExact ? 1u : 0u) << i;
+    }
+    if (!gather) ex = 0u;
+    while (ex != 0u) {
+      const int i = __ffs((int)ex) - 1;
+      ex &= ex - 1u;
+      uint32_t key = 0u, b = 0u;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        key = q == i ? k[q] : key;
+        b = q == i ? bb[q] : b;
+      }
+      bs.list[atomicAdd(&bs.off[b], 1u)] = ((uint64_t)key << 32) | (uint32_t)(pos + i);
+    }
+  });
   __syncthreads();
   for (int b = t; b < kNB; b += NT) {
-    if (bs.cls[bix(b)] == kBPlain && (bs.tie[bix(b)] & 2u))
-      bs.cls[bix(b)] = kBNone;
-    else if (bs.cls[bix(b)] == kBPlain && bs.tie[bix(b)])
-      bs.cls[bix(b)] = kBExact;
+    const uint32_t cl = bs.cls(b);
+    if (gather && cl == kBExact) bs.off[bix(b)] -= bs.cnt[bix(b)];  // back to the run's start
+    if (cl == kBPlain && bs.tie[bix(b)]) bs.set_cls(b, gather ? kBExactTie : kBExact);
   }
   __syncthreads();
 }
 
-// The EXACT buckets from `blo` on whose elements fit the list together:
-// gathered, sorted, and each bucket's place in the list.  Returns the end of
-// that bucket range (kNB when every remaining one fits), or blo when a single
-// bucket holds more than the list.
+// Wave 0: the EXACT buckets from `blo` on whose elements fit the list
+// together: each bucket's place in the list, and the end of that range (kNB
+// when every remaining one fits), for every thread.
 template <int NT>
-__device__ int bucket_batch(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs, int blo) {
-  const int t = (int)threadIdx.x;
+__device__ int bucket_places(BucketShared& bs, int blo) {
   if (wave_id() == 0) {
-    // the range: EXACT counts from blo in bucket order, 64 buckets a lane
+    // EXACT counts from blo in bucket order, 64 buckets a lane
     constexpr int PL = kNB / kWave;
     const int lane = lane_id();
     uint32_t c = 0;
     for (int i = 0; i < PL; ++i) {
       const int b = lane * PL + i;
-      c += (b >= blo && bs.cls[bix(b)] == kBExact) ? bs.cnt[bix(b)] : 0u;
+      c += (b >= blo && bs.cls(b) == kBExact) ? bs.cnt[bix(b)] : 0u;
     }
     uint32_t ci = c;
 #pragma unroll
@@ -264,45 +352,177 @@ __device__ int bucket_batch(const uint32_t* Kp, int n, const BucketRange& br, Bu
     int bhi = kNB;
     for (int i = 0; i < PL; ++i) {
       const int b = lane * PL + i;
-      const bool ex = b >= blo && bs.cls[bix(b)] == kBExact;
+      const bool ex = b >= blo && bs.cls(b) == kBExact;
       if (ex && run + bs.cnt[bix(b)] > (uint32_t)kBList && b < bhi) bhi = b;
       bs.off[bix(b)] = run;
       run += ex ? bs.cnt[bix(b)] : 0u;
     }
     bhi = (int)wave_min_u32((uint32_t)bhi);
+    const uint32_t total = readlane_u32(ci, kWave - 1);
     if (lane == 0) {
       bs.ctl[6] = (uint32_t)bhi;
+      bs.ctl[7] = total;  // the list's length when bhi == kNB
       bs.nlist = 0u;
     }
   }
   __syncthreads();
-  const int bhi = (int)bs.ctl[6];
-  if (bhi == blo) return blo;
-  for (int base = 0; base < n; base += NT * 8) {
-    const int pos = base + t * 8;
-    uint32_t k[8];
-    bucket_keys8(Kp, pos, n, k);
+  return (int)bs.ctl[6];
+}
+
+// The elements of the buckets of class CLS in [blo, bhi), put in their places.
+template <int NT>
+__device__ void bucket_gather(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs, int blo, int bhi,
+                              uint32_t cls) {
+  const int t = (int)threadIdx.x;
+  key_pass<NT>(Kp, n, [&](int pos, uint32_t (&k)[8]) {
+    uint32_t ex = 0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if (!br.in(k[i])) continue;
-      const int b = br.of(k[i]);
-      if (b >= blo && b < bhi && bs.cls[bix(b)] == kBExact) {
-        const uint32_t slot = atomicAdd(&bs.nlist, 1u);  // < kBList: the range's counts fit
-        bs.list[slot] = ((uint64_t)k[i] << 32) | (uint32_t)(pos + i);
-      }
+      const bool in = br.in(k[i]);
+      const int b = in ? br.of(k[i]) : 0;
+      ex |= (in && b >= blo && b < bhi && bs.cls(b) == cls ? 1u : 0u) << i;
+    }
+    while (ex != 0u) {
+      const int i = __ffs((int)ex) - 1;
+      ex &= ex - 1u;
+      uint32_t key = 0u;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) key = q == i ? k[q] : key;
+      bs.list[atomicAdd(&bs.off[bix(br.of(key))], 1u)] = ((uint64_t)key << 32) | (uint32_t)(pos + i);
+    }
+  });
+  __syncthreads();
+  for (int b = blo + t; b < bhi; b += NT)
+    if (bs.cls(b) == cls) bs.off[bix(b)] -= bs.cnt[bix(b)];
+  __syncthreads();
+}
+
+// The same for at most kTieMax buckets b[0, nb) whose keys are told by their
+// ranges alone, without a look at a class per element.
+constexpr int kTieMax = 8;
+template <int NT>
+__device__ void bucket_gather_few(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs, const uint32_t* b,
+                                  int nb) {
+  uint32_t lo[kTieMax], wd[kTieMax];
+#pragma unroll
+  for (int q = 0; q < kTieMax; ++q) {
+    const uint32_t bq = q < nb ? b[q] : 0u;
+    lo[q] = br.kmin + (bq << br.shift);
+    // (the last bucket holds every key up to the range's end)
+    wd[q] = q < nb ? (bq == (uint32_t)kNB - 1u ? br.kcut - lo[q] : min(1u << br.shift, br.kcut - lo[q])) : 0u;
+  }
+  key_pass<NT>(Kp, n, [&](int pos, uint32_t (&k)[8]) {
+    uint32_t ex = 0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      bool hit = false;
+#pragma unroll
+      for (int q = 0; q < kTieMax; ++q) hit = hit || k[i] - lo[q] < wd[q];
+      ex |= (hit ? 1u : 0u) << i;
+    }
+    while (ex != 0u) {
+      const int i = __ffs((int)ex) - 1;
+      ex &= ex - 1u;
+      uint32_t key = 0u;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) key = q == i ? k[q] : key;
+      bs.list[atomicAdd(&bs.off[bix(br.of(key))], 1u)] = ((uint64_t)key << 32) | (uint32_t)(pos + i);
+    }
+  });
+  __syncthreads();
+  if (threadIdx.x < (unsigned)nb) bs.off[bix((int)b[threadIdx.x])] -= bs.cnt[bix((int)b[threadIdx.x])];
+  __syncthreads();
+}
+
+// Orders each bucket's run of the list[0, nl) (runs of some 100 to 300
+// elements on near-flat rows).  Each of the up to kOrdRuns runs is cut into 64
+// equal steps of its keys; an element's place is first that of its step (a
+// count per step, a scan per run), then, among the step's few elements, that
+// of its key.  scr: 64 kOrdRuns words.  (The bitonic network over the list
+// took some 70 us, counting each run's smaller keys 97 us; this 8.)  More runs
+// than that are counted.
+constexpr int kOrdRuns = 64;
+template <int NT>
+__device__ void bucket_order(const BucketRange& br, BucketShared& bs, int nl, uint32_t* scr) {
+  constexpr int PT = kBList / NT;
+  const int t = (int)threadIdx.x, lane = lane_id(), w = wave_id();
+  uint64_t k[PT];
+  uint32_t at[PT];
+  // number the runs in the list (bs.tie: a bucket's ties are known by now)
+  if (t == 0) bs.nties = 0u;
+  for (int i = t; i < 64 * kOrdRuns; i += NT) scr[i] = 0u;
+  lds_barrier();
+  for (int b = t; b < kNB; b += NT) {
+    const uint32_t c = bs.cnt[bix(b)], o = bs.off[bix(b)];
+    if (bs.cls(b) == kBExact && c > 0u && o + c <= (uint32_t)nl) {
+      const uint32_t q = atomicAdd(&bs.nties, 1u);
+      bs.tie[bix(b)] = (uint8_t)min(q, 255u);
+      if (q < (uint32_t)kOrdRuns) bs.run_b[q] = (uint16_t)b;
     }
   }
-  __syncthreads();
-  const int nl = (int)bs.nlist;
-  int ns = 1;
-  while (ns < nl) ns <<= 1;
-  for (int i = nl + t; i < ns; i += NT) bs.list[i] = ~0ull;
   lds_barrier();
-  // keys order the buckets, so the sorted list holds each bucket's elements
-  // at its place (the exclusive count of EXACT buckets from blo before it)
-  lds_bitonic_sort_u64<NT>(bs.list, ns);
-  __syncthreads();
-  return bhi;
+  const int nr = (int)bs.nties;
+  if (nr > kOrdRuns) {
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+      const int i = q * NT + t;
+      k[q] = i < nl ? bs.list[i] : ~0ull;
+      at[q] = 0u;
+      if (i < nl) {
+        const int b = br.of((uint32_t)(k[q] >> 32));
+        const uint32_t s = bs.off[bix(b)], e = s + bs.cnt[bix(b)];
+        uint32_t r = 0u;
+        for (uint32_t j = s; j < e; ++j) r += bs.list[j] < k[q] ? 1u : 0u;
+        at[q] = s + r;
+      }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < PT; ++q)
+      if (q * NT + t < nl) bs.list[at[q]] = k[q];
+    lds_barrier();
+    return;
+  }
+  const int sh = max(0, br.shift - 6);
+  auto step_of = [&](uint64_t key) {
+    const uint32_t kk = (uint32_t)(key >> 32), b = (uint32_t)br.of(kk);
+    return ((uint32_t)bs.tie[bix((int)b)] << 6) | min((kk - br.kmin - (b << br.shift)) >> sh, 63u);
+  };
+  uint32_t st[PT];
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    const int i = q * NT + t;
+    k[q] = i < nl ? bs.list[i] : ~0ull;
+    st[q] = i < nl ? step_of(k[q]) : 0u;
+    at[q] = i < nl ? atomicAdd(&scr[st[q]], 1u) : 0u;
+  }
+  lds_barrier();
+  // per run: its steps' starts, with their counts above (places fit 13 bits)
+  static_assert(kBList < (1 << 13), "a place and a count share a word");
+  for (int r = w; r < nr; r += NT / kWave) {
+    const uint32_t c = scr[64 * r + lane];
+    const uint32_t in = wave_incl_scan_op(c, 0u, [](uint32_t x, uint32_t y) { return x + y; });
+    scr[64 * r + lane] = (bs.off[bix((int)bs.run_b[r])] + in - c) | (c << 16);
+  }
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < PT; ++q)
+    if (q * NT + t < nl) bs.list[(scr[st[q]] & 0xffffu) + at[q]] = k[q];
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < PT; ++q) {
+    if (q * NT + t < nl) {
+      const uint32_t x = scr[st[q]], s = x & 0xffffu, c = x >> 16;
+      uint32_t r = 0u;
+      for (uint32_t j = s; j < s + c; ++j) r += bs.list[j] < k[q] ? 1u : 0u;
+      at[q] = s + r;
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int q = 0; q < PT; ++q)
+    if (q * NT + t < nl) bs.list[at[q]] = k[q];
+  lds_barrier();
 }
 
 // Why a walk stops (kWalkOk: the chain ended; kWalkMore: it reached the end
@@ -323,8 +543,8 @@ __device__ uint32_t bucket_walk(const BucketShared& bs, float& v, float& before,
   before = v;
   for (int b0 = b_from & ~(kWave - 1); b0 < b_to; b0 += kWave) {
     const int b = b0 + lane;  // < kNB
-    const uint32_t cl = bs.cls[bix(b)];
-    const int jb = bs.jg[bix(b)];
+    const uint32_t cl = bs.cls(b);
+    const int jb = bs.jg(b);
     const uint32_t sm = bs.sum[bix(b)], ct = bs.cnt[bix(b)], of = bs.off[bix(b)];
     int i = b0 < b_from ? b_from - b0 : 0;
     const int iend = min(kWave, b_to - b0);
@@ -384,15 +604,61 @@ __device__ uint32_t bucket_walk(const BucketShared& bs, float& v, float& before,
 template <bool SUB, int NT>
 __device__ uint32_t bucket_chain(const uint32_t* Kp, int n, const BucketRange& br, BucketShared& bs, float v0,
                                  uint32_t lim, float thr, float& v_out, float& before_out, uint32_t& pos_out,
-                                 bool& stop_out, uint32_t& id_out, int row) {
-  bucket_sums<NT>(Kp, n, br, bs);
+                                 bool& stop_out, uint32_t& id_out, int row, uint32_t* scr) {
+  // one pass when every EXACT bucket fits the list; the buckets a tie made
+  // EXACT, if any, take another, behind the others in the list
+  bool all = bucket_places<NT>(bs, 0) == kNB;
+  uint32_t nl = bs.ctl[7];
+  bucket_sums<NT>(Kp, n, br, bs, all);
   LLZ_STAMP(row, 29);
+  if (all) {
+    if (threadIdx.x == 0) {
+      bs.nlist = nl;
+      bs.nties = 0u;
+    }
+    __syncthreads();
+    for (int b = (int)threadIdx.x; b < kNB; b += NT) {
+      if (bs.cls(b) == kBExactTie) {
+        bs.off[bix(b)] = atomicAdd(&bs.nlist, bs.cnt[bix(b)]);
+        const uint32_t q = atomicAdd(&bs.nties, 1u);
+        if (q < (uint32_t)kTieMax) bs.ties[q] = (uint32_t)b;
+      }
+    }
+    __syncthreads();
+    const uint32_t nt = bs.nlist;
+    const int ntie = (int)bs.nties;
+    all = nt <= (uint32_t)kBList;
+    if (all && ntie > 0) {
+      if (ntie <= kTieMax)
+        bucket_gather_few<NT>(Kp, n, br, bs, bs.ties, ntie);
+      else
+        bucket_gather<NT>(Kp, n, br, bs, 0, kNB, kBExactTie);
+    }
+    nl = nt;
+    for (int b = (int)threadIdx.x; b < kNB; b += NT)
+      if (bs.cls(b) == kBExactTie) bs.set_cls(b, kBExact);
+    __syncthreads();
+    LLZ_STAMP(row, 59);
+    if (all) bucket_order<NT>(br, bs, (int)nl, scr);
+  }
   float v = v0, before = v0;
   uint32_t pos = 0, id = 0xffffffffu, why = kWalkMore;
   bool stop = false;
   for (int blo = 0; why == kWalkMore;) {
-    const int bhi = bucket_batch<NT>(Kp, n, br, bs, blo);
-    if (bhi == blo) return 16u;  // one bucket holds more than the list
+    // (in batches: the EXACT buckets from blo on that fit the list together)
+    int bhi = kNB;
+    if (!all) {
+      bhi = bucket_places<NT>(bs, blo);
+      if (bhi == blo) return 16u;  // one bucket holds more than the list
+      bucket_gather<NT>(Kp, n, br, bs, blo, bhi, kBExact);
+      // the list's length: the places' end
+      uint32_t end = 0u;
+      for (int b = blo + (int)threadIdx.x; b < bhi; b += NT)
+        if (bs.cls(b) == kBExact) end = max(end, bs.off[bix(b)] + bs.cnt[bix(b)]);
+      atomicMax(&bs.nlist, end);
+      __syncthreads();
+      bucket_order<NT>(br, bs, (int)bs.nlist, scr);
+    }
     if (blo == 0) LLZ_STAMP(row, 30);
     if (wave_id() == 0) {
       why = bucket_walk<SUB>(bs, v, before, pos, lim, thr, stop, id, blo, bhi);

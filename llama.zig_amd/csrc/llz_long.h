@@ -157,7 +157,7 @@ __device__ __forceinline__ void long_row(const KArgs& A, int row, LongLds& U, Pe
       const float a = wave_fold_f32((q0 + q1) + (q2 + q3));
       qsum += a;
       qwsum += a * (float)(n - min(seg0, n));
-      if (tok) {
+      if (tok && !ovf) {  // (a row whose candidates flood the buffer is not decided here)
         const bool hit = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)) >= thr;
         if (bal64(hit) != 0ull) {
           if (nb > kLongBuf - SEG) {

@@ -1497,6 +1497,8 @@ template <class Src>
 __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, const RowParams& P, uint32_t* Ak,
                                SampleShared& sh, int& bank, BucketResult& res, int row) {
   BucketShared& bs = sh.u.bkt;
+  uint32_t* const scr = reinterpret_cast<uint32_t*>(sh.cand);  // the candidate list is not used on this path
+  static_assert(sizeof(sh.cand) >= 64 * kOrdRuns * sizeof(uint32_t), "the ordering's counts fit");
   const int t = (int)threadIdx.x;
   const bool t1 = (P.flags & kFlagTIsOne) != 0;
   const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
@@ -1519,42 +1521,45 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   {
     constexpr int TV = RowTiles8::V;
     const RowTiles8 rt(X.x, n);
-    float raw[TV];
-    rt.load(t * TV, raw);
-    for (int base = 0; base < n; base += kNT * TV) {
-      const int pos = base + t * TV;
-      rt.fix_tail(pos, raw);
-      float v[TV];
+    const float T = P.temperature, yS = 1.0f / S;
+    const bool s_in = S >= 0x1p-20f && S <= 0x1p40f;
+    pipelined_tiles<kNT, TV, 3, float>(
+        n, [&](int pos, float (&r)[TV]) { rt.load(pos, r); },
+        [&](int pos, float (&raw)[TV]) {
+          rt.fix_tail(pos, raw);
+          uint32_t key[TV];
 #pragma unroll
-      for (int k = 0; k < TV; ++k) v[k] = pos + k < n ? X.fix(pos + k, raw[k]) : 0.0f;
-      if (base + kNT * TV < n) rt.load(pos + kNT * TV, raw);
-      uint32_t key[TV];
-#pragma unroll
-      for (int k = 0; k < TV; ++k) {
-        const float p = row_exp(v[k], m, P.temperature, t1) / S;
-        const bool in = pos + k < n;
-        key[k] = in ? ~__float_as_uint(p) : 0xffffffffu;
-        if (in) {
-          km += p >= thr_m ? 1u : 0u;
-          if (key[k] < fk) {  // positions ascend within a thread: the first of equal keys stays
-            fk = key[k];
-            fid = (uint32_t)(pos + k);
+          for (int k = 0; k < TV; ++k) {
+            const bool in = pos + k < n;
+            const float e = row_exp(in ? X.fix(pos + k, raw[k]) : 0.0f, m, T, t1);
+            float p = div_by(e, S, yS);
+            if (!(s_in && e >= 0x1p-90f)) p = e / S;
+            key[k] = in ? ~__float_as_uint(p) : 0xffffffffu;
+            if (in) {
+              km += p >= thr_m ? 1u : 0u;
+              if (key[k] < fk) {  // positions ascend within a thread: the first of equal keys stays
+                fk = key[k];
+                fid = (uint32_t)(pos + k);
+              }
+              if (k == 0) {  // every eighth element, weight 8 (count and mass)
+                const uint32_t cb = min((key[k] - kmin) >> kCoarseShift, (uint32_t)kNB - 1u);
+                atomicAdd(&bs.hist[bix(cb)], 8ull * hist_word(key[k], coarse_Etop((int)cb)));
+              }
+            }
           }
-          if (k == 0) {  // every eighth element, weight 8 (count and mass)
-            const uint32_t cb = min((key[k] - kmin) >> kCoarseShift, (uint32_t)kNB - 1u);
-            atomicAdd(&bs.hist[bix(cb)], 8ull * hist_word(key[k], coarse_Etop((int)cb)));
-          }
-        }
-      }
-      if (pos + TV <= n && (reinterpret_cast<uintptr_t>(Ak + pos) & 15u) == 0u) {
-        *reinterpret_cast<uint4*>(Ak + pos) = make_uint4(key[0], key[1], key[2], key[3]);
-        *reinterpret_cast<uint4*>(Ak + pos + 4) = make_uint4(key[4], key[5], key[6], key[7]);
-      } else {
+          if (pos + TV <= n) {
 #pragma unroll
-        for (int k = 0; k < TV; ++k)
-          if (pos + k < n) Ak[pos + k] = key[k];
-      }
-    }
+            for (int h = 0; h < 2; ++h) {
+              llz_u4u q;
+              q.x = key[4 * h + 0]; q.y = key[4 * h + 1]; q.z = key[4 * h + 2]; q.w = key[4 * h + 3];
+              *reinterpret_cast<llz_u4u*>(Ak + pos + 4 * h) = q;
+            }
+          } else {
+#pragma unroll
+            for (int k = 0; k < TV; ++k)
+              if (pos + k < n) Ak[pos + k] = key[k];
+          }
+        });
   }
   km = P.min_p > 0.0f ? wg_sum_sat<kNT>(km, 0x7fffffffu, sh.wg, bank) : (uint32_t)n;
   const uint32_t gk = wg_min_u32<kNT>(fk, sh.wg, bank);
@@ -1569,15 +1574,15 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   // count reaches Lw or whose mass passes top-p, both with a margin for the
   // histogram's sampling (about sqrt(8 count): 0.6% at 217k elements); a cut
   // beyond the region only sends the row to the sorting path
-  if (wave_id() == 0) {
+  {
     int cs = kNB - 1;
-    bucket_scan(bs, [&](int b, uint32_t ec, double em) {
+    bucket_scan<kNT>(bs, [&](int b, uint32_t ec, double em) {
       const uint32_t ic = ec + bs.cnt[bix(b)];
       const double im = em + (double)bs.mass[bix(b)];
       if (b < cs && ((double)ic >= 1.05 * Lw + 2048.0 || (topp && im > (double)P.top_p * 1.05))) cs = b;
     });
-    cs = (int)wave_min_u32((uint32_t)cs);
-    if (lane_id() == 0) bs.ctl[0] = (uint32_t)cs;
+    const uint32_t cmin = wg_min_u32<kNT>((uint32_t)cs, sh.wg, bank);
+    if (t == 0) bs.ctl[0] = cmin;
   }
   __syncthreads();
   BucketRange br;
@@ -1593,10 +1598,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   auto fine_Etop = [&](int b) { return key_E(br.kmin + ((uint32_t)b << br.shift)); };
   for (int b = t; b < kNB; b += kNT) bs.hist[bix(b)] = 0ull;
   lds_barrier();
-  for (int base = 0; base < n; base += kNT * 8) {
-    const int pos = base + t * 8;
-    uint32_t k[8];
-    bucket_keys8(Ak, pos, n, k);
+  key_pass<kNT>(Ak, n, [&](int, uint32_t (&k)[8]) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if (br.in(k[i])) {
@@ -1604,15 +1606,15 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
         atomicAdd(&bs.hist[bix(b)], hist_word(k[i], fine_Etop(b)));
       }
     }
-  }
+  });
   __syncthreads();
   for (int b = t; b < kNB; b += kNT) hist_unpack(bs.hist[bix(b)], fine_Etop(b), bs.cnt[bix(b)], bs.mass[bix(b)]);
   __syncthreads();
 
   LLZ_STAMP(row, 24);
   // ---- the running sum of top-p and the total (sampler.zig:112-117, :156-159)
-  if (wave_id() == 0) {
-    bucket_scan(bs, [&](int b, uint32_t ec, double em) {
+  {
+    bucket_scan<kNT>(bs, [&](int b, uint32_t ec, double em) {
       const uint32_t c = bs.cnt[bix(b)];
       const uint32_t ic = ec + c;
       const double im = em + (double)bs.mass[bix(b)];
@@ -1630,8 +1632,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
         cl = exact ? kBExact : kBPlain;
         j = exact ? 0 : elo;
       }
-      bs.cls[bix(b)] = cl;
-      bs.jg[bix(b)] = (int8_t)j;
+      bs.cj[bix(b)] = (uint16_t)((uint32_t)cl | ((uint32_t)(j + kJgBias) << 3));
     });
   }
   __syncthreads();
@@ -1639,7 +1640,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
   float v, before;
   uint32_t pos, id;
   bool stop;
-  uint32_t why = bucket_chain<false, kNT>(Ak, n, br, bs, 0.0f, Lw, topp ? P.top_p : -1.0f, v, before, pos, stop, id, row);
+  uint32_t why = bucket_chain<false, kNT>(Ak, n, br, bs, 0.0f, Lw, topp ? P.top_p : -1.0f, v, before, pos, stop, id, row, scr);
   if (why != 0u) {
     res.why = why;
     return false;
@@ -1656,8 +1657,8 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
 
   // ---- the draw (sampler.zig:162-168)
   const float r0 = u * total;
-  if (wave_id() == 0) {
-    bucket_scan(bs, [&](int b, uint32_t ec, double em) {
+  {
+    bucket_scan<kNT>(bs, [&](int b, uint32_t ec, double em) {
       const uint32_t c = bs.cnt[bix(b)];
       const uint32_t ic = ec + c;
       const double im = em + (double)bs.mass[bix(b)];
@@ -1675,13 +1676,12 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
         cl = exact ? kBExact : kBPlain;
         j = exact ? 0 : elo;
       }
-      bs.cls[bix(b)] = cl;
-      bs.jg[bix(b)] = (int8_t)j;
+      bs.cj[bix(b)] = (uint16_t)((uint32_t)cl | ((uint32_t)(j + kJgBias) << 3));
     });
   }
   __syncthreads();
   LLZ_STAMP(row, 27);
-  why = bucket_chain<true, kNT>(Ak, n, br, bs, r0, K, -1.0f, v, before, pos, stop, id, row);
+  why = bucket_chain<true, kNT>(Ak, n, br, bs, r0, K, -1.0f, v, before, pos, stop, id, row, scr);
   LLZ_STAMP(row, 28);
   if (why != 0u) {
     res.why = 32u + why;

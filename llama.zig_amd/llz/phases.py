@@ -55,7 +55,7 @@ PHASES = [
     ("C: walk (w0)", 20, 21), ("C: after walk", 21, 6),
     ("buckets: keys + coarse histogram", 8, 23), ("buckets: fine histogram", 23, 24),
     ("buckets: top-p classes", 24, 25), ("buckets: top-p chain", 25, 26), ("buckets: draw classes", 26, 27),
-    ("buckets: draw chain", 27, 28), ("buckets draw: sums", 27, 29), ("buckets draw: 1st gather+sort", 29, 30),
+    ("buckets: draw chain", 27, 28), ("buckets draw: sums", 27, 29), ("buckets draw: ties gathered", 29, 59), ("buckets draw: ordered", 59, 30), ("buckets draw: 1st gather+sort", 29, 30),
     ("buckets draw: 1st walk", 30, 31), ("buckets draw: rest", 31, 28),
     ("token-only: scan", 2, 32), ("M start (max, barrier)", 1, 38), ("token: estimate + scan", 38, 39),
     ("token: queue + loads issued + barrier", 39, 32), ("token-only: re-read and exact terms", 32, 33), ("token-only: sort", 33, 34),
