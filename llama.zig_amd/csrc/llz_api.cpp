@@ -65,7 +65,7 @@ uint32_t post_bits(const llz_logit_post* post) {
 // fallback buffer sets (25 B per logit each, fb_slots_for) with their owner
 // words; the penalised copy only for windows too long to fuse.
 struct Layout {
-  size_t status, claim, cand, qovf, owner, fb, fb_mask, penal, split, total;
+  size_t status, claim, cand, qovf, owner, fb, fb_mask, penal, split, und, total;
   int fb_slots;
   bool has_penal;
 };
@@ -104,6 +104,8 @@ Layout layout_of(int32_t rows, int32_t vocab, const llz_sampler_config* cfg, int
   // last, so that a workspace without it holds every other part at the same
   // offsets: calls of at most kSplitRows rows, the split rows' chunk records
   L.split = off;   if (rows <= kSplitRows) off = align_up(off + r * sizeof(SplitRow));
+  // (or, for calls of more rows than a grid, k_tok's marks)
+  L.und = off;     if (rows > kMaxGrid) off = align_up(off + r * sizeof(uint32_t));
   L.total = off;
   return L;
 }
@@ -403,6 +405,15 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
   Q.claim = (unsigned long long*)(ws + L.claim);
   Q.prev_win = (xf_src & kXfPen) ? d_prev_tokens + (n_prev - window) : nullptr;
   Q.split = P.split_s > 0 ? (SplitRow*)(ws + L.split) : nullptr;
+  // more rows than CUs, the token alone, rows the single pass could keep
+  // resident and that are not soft-capped (their exact tanh is left to
+  // k_stats's estimates): k_tok decides what it can with two rows per CU
+  // (top-p alone over many rows stays with k_stats_rows: most of its rows
+  // need the exact normaliser, and the pass would be lost on them)
+  const bool ends = tok_minp || (cfg->top_k > 0 && cfg->top_k <= 128);
+  if (tok_only && ends && P.tok_theta > 0.0f && P.grid < rows && rows > kMaxGrid && workspace_bytes >= L.total &&
+      vocab <= kResidentMax && !(xf_src & kXfCap))
+    Q.und = (uint32_t*)(ws + L.und);
   e = launch_sample(P, Q, g_ev_begin, g_ev_end, st);
   if (e != hipSuccess) report_hip("llz_sample_rows: launch", e);
   return e == hipSuccess ? LLZ_OK : LLZ_E_HIP;

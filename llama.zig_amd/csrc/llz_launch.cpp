@@ -16,6 +16,7 @@ StatsKernel stats_kernel_6(int, int);
 StatsKernel stats_kernel_7(int, int);
 StatsKernel stats_kernel_8(int, int);
 StatsKernel stats_kernel_9(int, int);
+StatsKernel stats_kernel_10(int, int);
 
 // Every row's statistics, then its selection.
 hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_begin, hipEvent_t ev_end,
@@ -51,6 +52,11 @@ hipError_t launch_sample(const RowParams& P, const RowPtrs& Q, hipEvent_t ev_beg
   if (!kern) return hipErrorInvalidValue;
   const dim3 grid(split ? P.rows * P.split_s : (claim ? P.grid : P.rows)), block(kStatsNT);
   void* args[] = {const_cast<KArgs*>(&A)};
+  if (Q.und) {  // the token-only pass over every row first; kern then takes the rows it marked
+    const dim3 tg(P.rows < 3 * P.grid ? P.rows : 3 * P.grid);
+    if (hipLaunchKernel((const void*)stats_kernel_10(fastld, xm), tg, block, args, 0, st) != hipSuccess)
+      return hipErrorLaunchFailure;
+  }
   if (hipLaunchKernel((const void*)kern, grid, block, args, 0, st) != hipSuccess) return hipErrorLaunchFailure;
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -71,6 +77,7 @@ extern "C" int llz_stamps_6(unsigned long long*, int, int);
 extern "C" int llz_stamps_7(unsigned long long*, int, int);
 extern "C" int llz_stamps_8(unsigned long long*, int, int);
 extern "C" int llz_stamps_9(unsigned long long*, int, int);
+extern "C" int llz_stamps_10(unsigned long long*, int, int);
 
 // Measurement builds: the phase timestamps of rows 0 .. rows - 1 (kStampSlots
 // per row, 0 where a row did not reach the boundary) into dst.
@@ -78,7 +85,7 @@ extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int cle
   if (rows <= 0 || rows > llz::kStampRows || !dst) return -1;
   static int (*const get[])(unsigned long long*, int, int) = {llz_stamps_0, llz_stamps_1, llz_stamps_2, llz_stamps_3,
                                                               llz_stamps_4, llz_stamps_5, llz_stamps_6, llz_stamps_7,
-                                                              llz_stamps_8, llz_stamps_9};
+                                                              llz_stamps_8, llz_stamps_9, llz_stamps_10};
   static unsigned long long part[llz::kStampRows * llz::kStampSlots];
   const size_t n = (size_t)rows * llz::kStampSlots;
   if (!clear)

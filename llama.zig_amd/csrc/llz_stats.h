@@ -1904,7 +1904,31 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
   __shared__ StatsShared U;
   __shared__ PenShared pen_sh;
   __shared__ int next_row;
-  for (int row = (int)blockIdx.x;;) {
+  // behind k_tok: the rows it marked, this workgroup's share of them (grid
+  // rows apart, shifted from one stretch to the next so that rows of one
+  // parity do not all meet the same XCDs); usually none
+  const bool listed = A.Q.und != nullptr;
+  int i0 = 0;          // listed: stretches looked at so far
+  uint64_t marks = 0;  //   and those of the last 64 whose row is marked
+  auto next_listed = [&]() -> int {
+    const int g = A.P.grid, b = (int)blockIdx.x;
+    while (marks == 0ull && (int64_t)i0 * g < A.P.rows) {
+      const int i = i0 + lane_id();
+      const int64_t r = (int64_t)i * g + (b + i * 37) % g;
+      marks = bal64(r < A.P.rows && A.Q.und[r < A.P.rows ? r : 0] == (uint32_t)A.P.epoch);
+      i0 += kWave;
+    }
+    if (marks == 0ull) return A.P.rows;
+    const int i = i0 - kWave + __ffsll((long long)marks) - 1;
+    marks &= marks - 1ull;
+    return i * g + (b + i * 37) % g;
+  };
+  int row0 = (int)blockIdx.x;
+  if (listed) {
+    row0 = __builtin_amdgcn_readfirstlane(next_listed());
+    if (row0 >= A.P.rows) return;
+  }
+  for (int row = row0;;) {
     // the arguments through a pointer the compiler cannot see through, so
     // that each row loads them where it uses them instead of holding them in
     // registers across rows
@@ -1912,9 +1936,9 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
         (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
     stats_row<FASTLD, XM, EXT>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
-    if (threadIdx.x == 0) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid);
+    if (threadIdx.x == 0 && !listed) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid);
     __syncthreads();  // also: every wave is done with this row's shared memory
-    row = next_row;
+    row = listed ? __builtin_amdgcn_readfirstlane(next_listed()) : next_row;
     if (row >= A.P.rows) return;
   }
 }

@@ -6,6 +6,7 @@
 //   5, 6 k_split on plain rows: 16-byte aligned, any (a: float4 per thread)
 //   7, 8 k_split on transformed rows, the same (a: float4 per thread; b: soft-capped)
 //   9    k_long (a: 16-byte aligned rows; b: transform mode)
+//   10   k_tok (a: 16-byte aligned rows; b: transform mode, not soft-capped)
 #include "llz_long.h"
 #include "llz_stats.h"
 
@@ -28,6 +29,9 @@ StatsKernel LLZ_CAT(stats_kernel_, LLZ_INST)(int a, int b) {
   (void)b;
   return a == 1 ? k_split<1, kXmNone, F> : a == 2 ? k_split<2, kXmNone, F> : a == 4 ? k_split<4, kXmNone, F>
                                        : a == 8 ? k_split<8, kXmNone, F> : nullptr;
+#elif LLZ_INST == 10
+  if (b == kXmLight) return a != 0 ? k_tok<true, kXmLight> : k_tok<false, kXmLight>;
+  return a != 0 ? k_tok<true, kXmNone> : k_tok<false, kXmNone>;
 #elif LLZ_INST == 9
   if (b == kXmCap) return a != 0 ? k_long<true, kXmCap> : k_long<false, kXmCap>;
   if (b == kXmLight) return a != 0 ? k_long<true, kXmLight> : k_long<false, kXmLight>;

@@ -105,3 +105,39 @@ def test_typical_alone(n):
     assert path[4] & llz.PATH_FULL_SORT
     for p in (0.3, 0.999):
         _check(x, dataclasses.replace(TYPICAL, typical_p=p), exact=True)
+
+
+@pytest.mark.parametrize("n,pad", [(4096, 0), (30001, 0), (50000, 3), (129024, 0)])
+@pytest.mark.parametrize("params", [FILTERS, DEFAULT, FULL, dataclasses.replace(DEFAULT, top_k=50)],
+                         ids=["filters", "default", "full", "topk"])
+def test_more_rows_than_cus(n, pad, params):
+    """k_tok over 300 rows: decided, flooded (all equal, flat), NaN, infinite
+    and penalised rows, more candidates than the list holds under top-k."""
+    rows = 300
+    g = np.random.default_rng(n)
+    base = _rows(n, 4)
+    base = np.concatenate([base, g.normal(0.0, 2.0, size=(4, n)).astype(np.float32),
+                           g.normal(0.0, 0.3, size=(1, n)).astype(np.float32)])
+    pick = g.integers(0, base.shape[0], rows)
+    pick[:base.shape[0]] = np.arange(base.shape[0])
+    x = base[pick]
+    u = llz.rng_uniforms(9, rows)
+    for window in (0, 32):
+        p = dataclasses.replace(params, repetition_window=window, repetition_penalty=1.2 if window else 1.0)
+        prev = g.integers(0, n, size=(rows, 32)).astype(np.uint32)
+        flat = torch.empty(rows, n + pad, dtype=torch.float32, device="cuda")
+        flat[:, :n].copy_(torch.from_numpy(x))
+        r = llz.sample_rows(flat[:, :n], llz.SamplerConfig.of(p), torch.from_numpy(u).cuda(),
+                            torch.from_numpy(prev.astype(np.int32)).cuda(), kept_cap=64, probs=False, path=True)
+        torch.cuda.synchronize()
+        tok, con, kc, _ = _oracle_rows(x, p, u, prev)
+        assert np.array_equal(r.tokens.cpu().numpy().view(np.uint32), tok)
+        assert np.array_equal(r.consumed.cpu().numpy(), con)
+        assert np.array_equal(r.kept_count.cpu().numpy().view(np.uint32), kc)
+        path = r.row_path.cpu().numpy().view(np.uint32)
+        assert not np.any(path & 0x80000000)
+
+
+def _oracle_rows(x, p, u, prev):
+    tok, con, kept = O.sample_rows(x, p, u, prev_tokens=prev, threads=16)
+    return tok, con, kept, None
