@@ -354,7 +354,7 @@ __global__ __launch_bounds__(kNT) void k_long(KArgs A) {
     asm volatile("" : "+s"(Ap));
     long_row<FASTLD, XM>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
     if (A.P.grid >= A.P.rows) return;
-    if (threadIdx.x == 0) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid);
+    if (threadIdx.x == 0) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid, A.P.rows);
     __syncthreads();
     row = next_row;
     if (row >= A.P.rows) return;
@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kNT, 4) void k_tok(KArgs A) {
     const bool done = tok_stream<FASTLD, XM, 4, true>(P, Q, row, F, pen_sh, X, m, nanrow);
     if (threadIdx.x == 0) {
       if (!done) Q.und[row] = (uint32_t)P.epoch;
-      next_row = claim_row(A.Q.claim, A.P.epoch, (int)gridDim.x);
+      next_row = claim_row(A.Q.claim, A.P.epoch, (int)gridDim.x, A.P.rows);
     }
     __syncthreads();
     row = next_row;

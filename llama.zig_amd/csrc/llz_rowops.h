@@ -113,14 +113,18 @@ __device__ __forceinline__ float4 rd4_any(const float* xr, int pos, int n) {
 // fetch-and-add, which the device serves back to back, where a
 // compare-and-swap loop lets one claim through per round trip to memory
 // (with rows of some 40 us, the workgroups then queued for their claims).
-// The count stays below 2^24: at most rows + grid claims.
-[[maybe_unused]] static __device__ __noinline__ int claim_row(unsigned long long* word, unsigned long long epoch, int grid) {
+// The count stays below 2^24.  A launch makes exactly `rows` claims (rows -
+// grid rows are taken, and each of the grid's workgroups is told once that
+// none is left): the last one clears the word, so that a captured launch, whose
+// replays carry one epoch, finds it free each time.
+[[maybe_unused]] static __device__ __noinline__ int claim_row(unsigned long long* word, unsigned long long epoch, int grid, int rows) {
   constexpr unsigned long long kCnt = (1ull << 24) - 1;
   const unsigned long long tag = (epoch & ((1ull << 40) - 1)) << 24;
   unsigned long long old = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (;;) {
     if ((old & ~kCnt) == tag) {
       const unsigned long long prev = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((int)(prev & kCnt) == rows - 1) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return grid + (int)(prev & kCnt);
     }
     unsigned long long expected = old;

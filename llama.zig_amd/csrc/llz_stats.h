@@ -1936,7 +1936,7 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
         (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
     stats_row<FASTLD, XM, EXT>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
-    if (threadIdx.x == 0 && !listed) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid);
+    if (threadIdx.x == 0 && !listed) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid, A.P.rows);
     __syncthreads();  // also: every wave is done with this row's shared memory
     row = listed ? __builtin_amdgcn_readfirstlane(next_listed()) : next_row;
     if (row >= A.P.rows) return;

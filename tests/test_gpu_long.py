@@ -141,3 +141,33 @@ def test_more_rows_than_cus(n, pad, params):
 def _oracle_rows(x, p, u, prev):
     tok, con, kept = O.sample_rows(x, p, u, prev_tokens=prev, threads=16)
     return tok, con, kept, None
+
+
+@pytest.mark.parametrize("params,n", [(FILTERS, 20000), (DEFAULT, 20000), (FILTERS, 131076)],
+                         ids=["k_tok", "claimed rows", "claimed long rows"])
+def test_replayed_calls_of_more_rows_than_cus(params, n):
+    """A captured call's replays carry one epoch: every replay samples every
+    row of the logits it finds, also beyond the grid."""
+    rows = 800 if n < 100000 else 300
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.empty(rows, n, device="cuda")
+    u = torch.rand(rows, generator=g, device="cuda")
+    call = llz.PreparedCall(rows, n, llz.SamplerConfig.of(params), "cuda:0")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        captured = llz.PreparedCall(rows, n, llz.SamplerConfig.of(params), "cuda:0", stream=side)
+        x.normal_(0.0, 2.5, generator=g)
+        captured(x, u)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured(x, u)
+    for _ in range(4):
+        x.normal_(0.0, 2.5, generator=g)
+        torch.cuda.synchronize()
+        want = call(x, u)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured.result.tokens, want.tokens)
+        assert torch.equal(captured.result.consumed, want.consumed)
