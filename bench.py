@@ -14,8 +14,9 @@ with the post-processing and the penalty (the reference's decode step), and
 A step is one llz_sample_rows call over one resident batch.  Inputs rotate
 over enough distinct device buffers that each step reads its logits from HBM,
 not from the 256 MB Infinity Cache.  Each line carries the roofline of the
-step's one kernel (k_stats; k_split for token-only calls of at most 32 rows,
-which read each row with several workgroups), the fraction of rows on each
+step's kernel (k_stats; k_split for token-only calls of at most 32 rows,
+which read each row with several workgroups; k_long for rows beyond 129024
+logits; k_tok and k_stats_rows for token-only calls of more rows than CUs), the fraction of rows on each
 path, and the CPU baseline (the reference sampler restated in C) timed on
 this host with one thread and with the host's share of threads.
 """
@@ -252,8 +253,8 @@ def run_workload(line: str, steps: int, warmup: int, args) -> dict:
     # W untimed warmup steps right before the timed region (after the spot
     # check, whose host work leaves the GPU idle), a synchronisation, then the
     # timed region: K steps back to back on one stream, bracketed by HIP
-    # events on that stream.  The sampling kernel is the only kernel of a step, so the
-    # events' interval over K is its average launch duration (the host
+    # events on that stream.  The sampling kernels are the only kernels of a step, so the
+    # events' interval over K is their average duration (the host
     # enqueues faster than the GPU runs, so launches follow each other with
     # no idle gap).  The first dispatch after the synchronisation's idle gap
     # runs about 12 us longer than the others (kernel trace of this command),
@@ -286,6 +287,10 @@ def run_workload(line: str, steps: int, warmup: int, args) -> dict:
     traffic = None
     kernel = "k_split" if path_fracs["split"] >= 0.5 else "k_stats"
     traffic_src = os.path.join("profiles", f"{kernel}_{line}_traffic.json")
+    if vocab > 129024 and kernel == "k_stats":
+        kernel = "k_long"  # rows beyond the single pass
+    elif line == "c5":
+        kernel = "k_tok + k_stats_rows"  # the streaming pass, then the rows it leaves
     if os.path.exists(os.path.join(ROOT, traffic_src)):
         with open(os.path.join(ROOT, traffic_src)) as f:
             traffic = json.load(f).get("hbm_bytes_per_launch")
