@@ -661,13 +661,17 @@ void llz_sampler_set_state(llz_sampler* s, const uint64_t state[4]) {
   if (s && state) std::memcpy(s->prng, state, sizeof(s->prng));
 }
 
-static bool is_device_ptr(const void* p) {
+// Where the caller's data lies: on the device, in host memory that HIP knows
+// (pinned or managed) or in the process's own.
+enum class Mem { kDevice, kHip, kHost };
+static Mem mem_of(const void* p) {
   hipPointerAttribute_t a;
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return Mem::kHost;
   }
-  return a.type == hipMemoryTypeDevice;
+  if (a.type == hipMemoryTypeUnregistered) return Mem::kHost;
+  return a.type == hipMemoryTypeDevice ? Mem::kDevice : Mem::kHip;
 }
 
 // One row through llz_sample_rows with the caller's uniform: token and the
@@ -699,12 +703,17 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
   // stream; the results written by the sampling kernel into pinned memory.
   // (Pageable copies of the logits, the history and the uniform, and two
   // more for the results, took 81 us of a call alone and 148 us back to back.)
+  // Pinned and managed memory may still be written by work queued on the
+  // default stream, which the sampler's stream waits for and the CPU does
+  // not: copies on the sampler's stream read it, behind that work.
   const Stage at(n, n_prev);
   std::memcpy(s->h_stage, &u, sizeof(float));
-  if (n_prev > 0) std::memcpy(s->h_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t));
+  const bool prev_cpu = n_prev > 0 && mem_of(prev_tokens) == Mem::kHost;
+  if (prev_cpu) std::memcpy(s->h_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t));
   const float* d_in = logits;
-  const bool on_host = !is_device_ptr(logits);
-  if (on_host) d_in = (const float*)(s->d_stage + at.logits);
+  const Mem where = mem_of(logits);
+  const bool on_host = where == Mem::kHost;
+  if (where != Mem::kDevice) d_in = (const float*)(s->d_stage + at.logits);
   // the staged bytes [0, end): the head, then with host logits all of them
   const size_t bytes = (size_t)n * sizeof(float), end = on_host ? at.logits + bytes : at.logits;
   for (size_t from = 0, off = 0; from < end;) {
@@ -720,6 +729,14 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
       return LLZ_E_HIP;
     from = upto;
   }
+  // behind the staged head, which covers the history's place
+  if (n_prev > 0 && !prev_cpu &&
+      hipMemcpyAsync(s->d_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t), hipMemcpyDefault,
+                     s->stream) != hipSuccess)
+    return LLZ_E_HIP;
+  if (where == Mem::kHip &&
+      hipMemcpyAsync(s->d_stage + at.logits, logits, bytes, hipMemcpyDefault, s->stream) != hipSuccess)
+    return LLZ_E_HIP;
   const bool greedy = cfg->temperature <= 0.0f;
   int rc = llz_sample_rows(d_in, n, 1, n, cfg, nullptr, n_prev > 0 ? (const uint32_t*)(s->d_stage + at.prev) : nullptr,
                            n_prev, 0, (const float*)s->d_stage, greedy ? s->d_token : &s->h_out->token,
