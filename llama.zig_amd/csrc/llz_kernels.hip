@@ -82,24 +82,26 @@ __device__ __forceinline__ uint64_t amax_key(float v, uint32_t i) {
 }
 
 __global__ __launch_bounds__(kArgNT) void k_argmax(const float* __restrict__ logits, int64_t stride,
-                                                   int n, int chunks, int per_chunk, uint32_t xf, float cap,
+                                                   int n, int chunks, uint32_t per_chunk, uint32_t xf, float cap,
                                                    float inv_scale, uint32_t* __restrict__ tokens,
                                                    uint8_t* __restrict__ consumed, uint32_t* __restrict__ kept_count,
                                                    uint32_t* __restrict__ path) {
   __shared__ uint64_t best[kArgNT / kWave];
   const int row = (int)(blockIdx.x / (unsigned)chunks), c = (int)(blockIdx.x % (unsigned)chunks);
   const float* x = logits + (int64_t)row * stride;
-  const int p0 = c * per_chunk, p1 = min(n, p0 + per_chunk);  // chunks divide the row: p0 < n
+  // chunks divide the row: p0 < n (positions unsigned: a step past a row of
+  // nearly 2^31 logits stays above its end)
+  const uint32_t p0 = (uint32_t)c * per_chunk, p1 = min((uint32_t)n, p0 + per_chunk);
   uint64_t bk = 0ull;  // below every element's key
   if (p1 - p0 >= 4) {
     // starts past the chunk's last four logits are moved back to them: an
     // element read twice changes no maximum, and no load needs a branch
-    for (int base = p0; base < p1; base += kArgStep) {
+    for (uint32_t base = p0; base < p1; base += kArgStep) {
       llz_f4u v[kArgUnroll];
       uint32_t pos[kArgUnroll];
 #pragma unroll
       for (int u = 0; u < kArgUnroll; ++u) {
-        pos[u] = (uint32_t)min(base + (u * kArgNT + (int)threadIdx.x) * 4, p1 - 4);
+        pos[u] = min(base + ((uint32_t)u * kArgNT + threadIdx.x) * 4u, p1 - 4u);
         v[u] = *reinterpret_cast<const llz_f4u*>(x + pos[u]);
       }
 #pragma unroll
@@ -108,8 +110,8 @@ __global__ __launch_bounds__(kArgNT) void k_argmax(const float* __restrict__ log
         for (int k = 0; k < 4; ++k) bk = max(bk, amax_key(logit_post(v[u][k], xf, cap, inv_scale), pos[u] + (uint32_t)k));
     }
   } else {
-    for (int i = p0 + (int)threadIdx.x; i < p1; i += kArgNT)
-      bk = max(bk, amax_key(logit_post(x[i], xf, cap, inv_scale), (uint32_t)i));
+    for (uint32_t i = p0 + threadIdx.x; i < p1; i += kArgNT)
+      bk = max(bk, amax_key(logit_post(x[i], xf, cap, inv_scale), i));
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) bk = max(bk, (uint64_t)__shfl_xor((unsigned long long)bk, m, kWave));
@@ -238,10 +240,11 @@ hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, u
                          float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
                          uint32_t* path, hipStream_t st) {
   // chunks per row: as many as fill kArgGroups workgroups, none below kArgChunk logits
-  const int most = std::max(1, (n + kArgChunk - 1) / kArgChunk);
-  const int want = std::min(most, std::max(1, kArgGroups / rows));
-  const int per = ((n + want - 1) / want + 3) & ~3;
-  const int chunks = (n + per - 1) / per;
+  const uint32_t un = (uint32_t)n;
+  const uint32_t most = (un + kArgChunk - 1) / kArgChunk;
+  const uint32_t want = std::min(most, (uint32_t)std::max(1, kArgGroups / rows));
+  const uint32_t per = ((un + want - 1) / want + 3u) & ~3u;
+  const int chunks = (int)((un + per - 1) / per);
   hipLaunchKernelGGL(k_argmax, dim3((unsigned)rows * (unsigned)chunks), dim3(kArgNT), 0, st, logits, stride, n, chunks,
                      per, xf, cap, inv_scale, tokens, consumed, kept_count, path);
   return hipGetLastError();

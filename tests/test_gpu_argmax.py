@@ -51,3 +51,12 @@ def test_argmax_chunks(n, rows, offset):
     xd.copy_(torch.from_numpy(x))
     for fill in (0, n - 1, -1, n, 0x7FFFFFFF):
         assert np.array_equal(_argmax(xd, fill), want), fill
+
+
+@pytest.mark.parametrize("n", [2**31 - 1, 2**31 - 4096])
+def test_argmax_longest_rows(n):
+    """Chunk positions past the end of the longest rows stay above it."""
+    x = torch.full((1, n), -1.0, dtype=torch.float32, device="cuda")
+    for at in (n - 1, n // 2):
+        x[0, at] = x[0, at] + 2.0 + (n - at) * 1e-9
+        assert _argmax(x, 0)[0] == at
