@@ -311,7 +311,7 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
                         !(typical_on && (xf_src & kXfCap));
   P.flags = (cfg->temperature == 1.0f ? kFlagTIsOne : 0u) | (vec ? kFlagVecSrc : 0u) | kFlagFallback |
             (tok_only ? kFlagTokenOnly : 0u);
-  if (vocab > kResidentMax && vocab <= kLongMax && std::fabs(P.l2e_t) <= 0x1p40f) P.flags |= kFlagLong;
+  if (vocab > kResidentMax && vocab <= kLongMax && P.l2e_t > 0.0f && P.l2e_t <= 0x1p40f) P.flags |= kFlagLong;
   P.xf_src = xf_src;
   P.xf_orig = xb;
   P.cap = cap;

@@ -151,7 +151,10 @@ __device__ __forceinline__ bool tok_stream(const RowParams& P, const RowPtrs& Q,
       ml = fmaxf(ml, fmaxf(fmaxf(cur[u].x, cur[u].y), fmaxf(cur[u].z, cur[u].w)));
     ml = wave_max_f32(ml);
     mx = fmaxf(mx, ml);
-    if (k0 == 0) cw = (fabsf(mx) <= 3.0e38f ? mx : 0.0f) * l2e;
+    // a finite offset whatever the maximum: an infinite one would make the
+    // estimates of -inf logits and absent positions NaN (a maximum whose
+    // product overflows fails the |awi| test below)
+    if (k0 == 0) cw = fabsf(mx * l2e) <= 3.0e38f ? mx * l2e : 0.0f;
     // the threshold against the largest maximum any wave has published (no
     // barrier: an older one only lets more pass)
     if (lane == 0) F.mw[w] = mx;
@@ -221,7 +224,9 @@ __device__ __forceinline__ bool tok_stream(const RowParams& P, const RowPtrs& Q,
 #pragma unroll
   for (int i = 0; i < W; ++i) {
     m = fmaxf(m, F.mw[i]);
-    nanrow = nanrow || F.qs[i] != F.qs[i];  // q >= 0 otherwise, so no inf - inf
+    // only a NaN logit makes an estimate NaN (l2e > 0, the offset finite), and
+    // q >= 0 otherwise, so no inf - inf
+    nanrow = nanrow || F.qs[i] != F.qs[i];
   }
 #pragma unroll
   for (int i = 0; i < W; ++i) {
@@ -233,8 +238,8 @@ __device__ __forceinline__ bool tok_stream(const RowParams& P, const RowPtrs& Q,
   }
   m_out = m;
   nan_out = nanrow;
-  // a NaN logit or an infinite maximum makes the reference's sum NaN: the
-  // selection stage handles that row
+  // (a NaN logit or an infinite maximum makes the reference's sum NaN: the
+  // selection stage handles that row)
   if (tok && !bad && !nanrow && fabsf(m) <= 3.0e38f && F.tfail == 0u) {
     float theta = P.tok_theta;
     thr = thr_of(m);
