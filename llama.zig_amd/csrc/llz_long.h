@@ -340,7 +340,7 @@ __device__ __forceinline__ void long_row(const KArgs& A, int row, LongLds& U, Pe
   float m;
   bool nanrow;
   if (tok_stream<FASTLD, XM, 8, false>(P, Q, row, U.lng, pen_sh, X, m, nanrow)) return;
-  const bool nan_sum = nanrow || !(fabsf(m) <= 3.0e38f);
+  const bool nan_sum = nanrow || !(fabsf(m) < kInf);
   select_row(P, Q, U.select, m, nan_sum ? __builtin_nanf("") : 0.0f, 0u, !nan_sum, Q.uniforms[row], false, 0ull, 0u, X, O,
              XF ? &pen_sh : nullptr, kernel_args_ptr(), row, wslot, P.cand_theta);
   LLZ_STAMP(row, 15);

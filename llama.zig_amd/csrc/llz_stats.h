@@ -1346,7 +1346,8 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   }
   // a NaN logit or an infinite maximum makes the reference's sum NaN: the
   // selection handles that row without the phases below
-  const bool nan_sum = nanrow || !(fabsf(m) <= 3.0e38f);
+  // (a finite maximum above 3e38 fails the |awi| test below)
+  const bool nan_sum = nanrow || !(fabsf(m) < kInfS);
   bool certified = true;
   float S = __builtin_nanf("");
   uint32_t cc = 0;

@@ -57,7 +57,7 @@ def _masked(n, low, seed=0):
     head = min(n // 2, 16384)
     x[0, :head] = low                      # every wave's first segments
     x[1, :n - 300] = low
-    x[2, :] = max(low, np.float32(-3e38))  # nothing left but the mask
+    x[2, :] = low                          # nothing left but the mask
     x[3, :head] = low
     x[3, head::2] = -np.inf                # both masks in a row
     x[4, ::2] = low
@@ -82,3 +82,15 @@ def test_long_rows_infinite_temperature(n):
     x = np.random.default_rng(n).normal(0.0, 2.0, size=(2, n)).astype(np.float32)
     for p in (FILTERS, DEFAULT):
         _check(x, dataclasses.replace(p, temperature=float("inf")))
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["token", "exact"])
+@pytest.mark.parametrize("n", [3, 2000, 4099, 50000, 129024, 129028])
+def test_largest_finite_maxima(n, exact):
+    """A maximum beyond 3e38 is a number, not an infinity."""
+    x = np.full((3, n), LOW, np.float32)
+    x[1] = np.random.default_rng(n).normal(0.0, 2.0, n)
+    x[1, n // 2] = -LOW
+    x[2] = np.float32(3.2e38)
+    for p in (FILTERS, DEFAULT, dataclasses.replace(FILTERS, temperature=60.0)):
+        _check(x, p, exact=exact)
