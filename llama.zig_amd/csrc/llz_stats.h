@@ -627,9 +627,10 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     my_a = __int_as_float(llz_writelane_i32(__builtin_amdgcn_readlane(__float_as_int(a), kWave - 1), k, __float_as_int(my_a)));
   };
   auto set_cw = [&](float mr) {
-    // any finite reference of this wave: |m - mr| is checked in phase M
-    if (!(fabsf(mr) <= 3.0e38f)) mr = 0.0f;
+    // any finite reference of this wave: |m - mr| is checked in phase M (an
+    // infinite offset would make a -inf logit's estimate NaN)
     cw = mr * l2e_t;
+    if (!(fabsf(cw) <= 3.0e38f)) cw = 0.0f;
   };
   {
     // A window of kLoadWindow loads in flight per wave, one issued as each
@@ -703,7 +704,11 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       v.w = -kInfS;
       if (nv <= w * SEG) set_cw(wave_max_f32(max4(v)));  // the wave holds no other logit
       if constexpr (XM != kXmCap) mx = max3_raw(max3_raw(mx, v.x, v.y), v.z, v.w);
-      const float4 q = q_of(v, l2e_t, cw);
+      // absent positions: an infinite offset, as in seg_q (l2e_t may be 0)
+      float4 q = q_of(v, l2e_t, cw);
+      q.y = a1 ? q.y : 0.0f;
+      q.z = a2 ? q.z : 0.0f;
+      q.w = 0.0f;
       if (kt >= KV && own) *reinterpret_cast<float4*>(&F.u.data[w][kt - KV][lane4]) = q;
 #pragma unroll
       for (int k = 0; k < KV; ++k) {

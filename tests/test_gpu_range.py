@@ -94,3 +94,19 @@ def test_largest_finite_maxima(n, exact):
     x[2] = np.float32(3.2e38)
     for p in (FILTERS, DEFAULT, dataclasses.replace(FILTERS, temperature=60.0)):
         _check(x, p, exact=exact)
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["token", "exact"])
+@pytest.mark.parametrize("n,offset", [(2049, 0), (4100, 0), (4099, 1), (32003, 0), (128256, 0), (129021, 1)])
+@pytest.mark.parametrize("low,t,scale", [(-1e38, 0.25, 1.0), (-3e38, 1.0, 1.0), (LOW, 0.7, 2.0), (LOW, 40.0, 1.0)])
+def test_resident_rows_low_masks(n, offset, low, t, scale, exact):
+    _check(_masked(n, np.float32(low)), dataclasses.replace(FILTERS, temperature=t),
+           post=llz.LogitPost(0.0, scale) if scale != 1.0 else None, offset=offset, exact=exact)
+
+
+@pytest.mark.parametrize("n", [5, 2049, 4100, 129021, 129024])
+def test_resident_rows_infinite_temperature(n):
+    x = np.random.default_rng(n).normal(0.0, 2.0, size=(3, n)).astype(np.float32)
+    x[2, n // 2] = -np.inf  # (-inf - max) / inf: NaN, in the reference too
+    for p in (FILTERS, DEFAULT):
+        _check(x, dataclasses.replace(p, temperature=float("inf")))
