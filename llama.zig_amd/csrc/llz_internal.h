@@ -126,7 +126,7 @@ struct RowParams {
 // Split rows: one chunk's summary and the row's record in the workspace
 // (words written and read only through device-coherent atomic accesses).
 struct SplitRec {
-  unsigned long long tag;  // the call's epoch once the words below are final
+  unsigned long long tag;  // the call's epoch once the words below are final (until the merge clears it)
   unsigned long long mc;   // bits of the chunk's maximum m (NaNs skipped) | bits of c = RN(m l2e_t) << 32
   unsigned long long sv;   // bits of s = sum of exp2(fma(v, l2e_t, -c)) | bits of vt << 32, the largest
                            // logit of the chunk's possible candidates left out of its list (-inf: none)

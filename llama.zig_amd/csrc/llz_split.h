@@ -34,6 +34,12 @@
 // release fence at agent scope would write back the whole L2 of each
 // workgroup's XCD, microseconds per workgroup.)
 //
+// A captured launch's replays carry one epoch, so a launch leaves no word
+// that would count in the next: a merging workgroup clears the tags (every
+// one has been stored by then; a workgroup that reads them later sees some
+// cleared and leaves the row to it), and chunk 0's workgroup clears the
+// row's word before it publishes.
+//
 //   m = max m_c; the normaliser's estimate sum_c s_c exp2(fma(m, -l2e_t,
 //   c_c)) (the chunk sums scaled to the row's maximum, as phase M scales
 //   the waves' sums); the list: the chunks' entries whose exact term
@@ -137,6 +143,9 @@ __device__ __forceinline__ bool split_chunk(const KArgs& A, int row, int c, Spli
       v[j] = rd4_any(xr, pos, n);
     }
   }
+  // (complete before this chunk's tag is stored, so before any workgroup
+  // takes the row)
+  if (c == 0 && t == 0) dev_st(&R.elect, 0ull);
   if constexpr (XF) {
     const uint32_t xf = P.xf_src;
     // main.zig:653-666 on each logit of the row (positions past it stay -inf)
@@ -400,6 +409,8 @@ __device__ __forceinline__ bool split_merge(const KArgs& A, int row, SplitShared
     const int i = h * kSplitNT + t;
     en[h] = dev_ld(&R.cand[i < nslots ? i : 0]);
   }
+  // every tag has been stored: none is left for a replay
+  if (w == kSplitW - 1 && lane < ns) dev_st(&R.rec[lane].tag, 0ull);
   if (w == 0) {
     const bool on = lane < ns;
     float mc = ninf, cc = 0.0f, sc = 0.0f, vt = ninf, wc = 0.0f;

@@ -10,6 +10,7 @@ split rows off, whichever path a row takes.
 """
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -319,3 +320,72 @@ def test_top_p_cut_certified_by_position_weighted_interval(cuda, split):
         g = _run(cuda, x[r:r + 1], params, u[r:r + 1], cap=256, split=split)
         assert g["path"][0] & PATH_TOKEN_ONLY, f"row {r}: path {g['path'][0]:#x}"
         _check_oracle(x[r:r + 1], params, u[r:r + 1], g)
+
+
+def test_split_rows_replayed(cuda):
+    """A captured call's replays carry one epoch: every replay decides its rows
+    from the chunks of its own logits, rows that need the single-row path
+    (too many candidates, a NaN) in consecutive replays too,
+    with and without the caller's workspace."""
+    import torch
+
+    dev = torch.device(cuda)
+    n, rows = 128256, 2
+    chain = WORKLOADS["c2"].params
+    cfg = llz.SamplerConfig.of(chain)
+    g = np.random.default_rng(3)
+
+    def inputs(k):
+        x = g.normal(0.0, 2.0, size=(rows, n)).astype(np.float32)
+        for r in range(rows):
+            x[r, g.choice(n, 8, replace=False)] += np.float32(12.0)
+        if k % 3 == 1:
+            x[0] = g.normal(0.0, 0.1, n).astype(np.float32)  # flat: a list that overflows
+        if k % 3 == 2:
+            x[:, 5] = np.nan
+        return x, g.random(rows, dtype=np.float32)
+
+    xd = torch.empty(rows, n, device=dev)
+    ud = torch.empty(rows, device=dev)
+    side = torch.cuda.Stream()
+    noalloc = dict(tokens=torch.empty(rows, dtype=torch.int32, device=dev),
+                   consumed=torch.empty(rows, dtype=torch.uint8, device=dev))
+    c = cfg.to_c()
+
+    def call_noalloc():
+        rc = llz.library().llz_sample_rows_noalloc(
+            xd.data_ptr(), n, rows, n, ctypes.byref(c), None, None, 0, 0, ud.data_ptr(), noalloc["tokens"].data_ptr(),
+            noalloc["consumed"].data_ptr(), None, side.cuda_stream)
+        assert rc == 0
+
+    with torch.cuda.stream(side):
+        prepared = llz.PreparedCall(rows, n, cfg, dev, stream=side, path=True)
+        graphs = []
+        for call in (lambda: prepared(xd, ud), call_noalloc):
+            xd.zero_()
+            ud.fill_(0.5)
+            call()
+            side.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                call()
+            graphs.append(graph)
+    split, single = 0, 0
+    for k in (0, 1, 1, 2, 2, 0, 1, 0, 0, 2):
+        x, u = inputs(k)
+        xd.copy_(torch.from_numpy(x))
+        ud.copy_(torch.from_numpy(u))
+        torch.cuda.synchronize()
+        want = [O.sample_row(x[r], chain, u[r], detail=False) for r in range(rows)]
+        for graph, out in zip(graphs, (prepared.result.__dict__, noalloc)):
+            out["tokens"].fill_(-7)
+            out["consumed"].fill_(9)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert out["tokens"].tolist() == [o.token for o in want], k
+            assert out["consumed"].tolist() == [o.consumed for o in want], k
+        path = prepared.result.row_path.cpu().numpy().view(np.uint32)
+        split += int(np.sum((path & PATH_SPLIT) != 0))
+        single += int(np.sum((path & PATH_SPLIT) == 0))
+    assert split >= 4 and single >= 6, (split, single)  # both ends were reached
