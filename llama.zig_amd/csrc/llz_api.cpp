@@ -372,6 +372,10 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
         break;
       }
     }
+    // (the null stream cannot be captured)
+    hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
+    if (P.split_s > 0 && st && hipStreamIsCapturing(st, &cap_st) != hipSuccess) return LLZ_E_HIP;
+    if (cap_st != hipStreamCaptureStatusNone) P.flags |= kFlagReplay;
     // a chunk's possible candidates: d2 = (m_c - v) l2e_t < log2(1 / theta)
     // + 2^-8 (rounded up to a float)
     const double b = std::log2(1.0 / (double)P.tok_theta) + 0x1p-8;

@@ -40,6 +40,7 @@ constexpr uint32_t kFlagTokenOnly = 8u;  // no probabilities or row statistics r
 constexpr uint32_t kFlagXfExact = 16u;   // transformed rows the single pass cannot estimate: the exact streaming path
 
 constexpr uint32_t kFlagLong = 32u;      // rows of k_long: beyond the single pass's residency, up to kLongMax logits
+constexpr uint32_t kFlagReplay = 64u;    // a captured launch: its replays carry the same arguments, the epoch among them
 
 // RowParams.xf_src / xf_orig: transforms applied as a row is read
 constexpr uint32_t kXfCap = 1u;    // v = tanh(v / cap) * cap   (main.zig:653-658)
@@ -126,7 +127,7 @@ struct RowParams {
 // Split rows: one chunk's summary and the row's record in the workspace
 // (words written and read only through device-coherent atomic accesses).
 struct SplitRec {
-  unsigned long long tag;  // the call's epoch once the words below are final (until the merge clears it)
+  unsigned long long tag;  // the call's epoch once the words below are final (kFlagReplay: until the merge clears it)
   unsigned long long mc;   // bits of the chunk's maximum m (NaNs skipped) | bits of c = RN(m l2e_t) << 32
   unsigned long long sv;   // bits of s = sum of exp2(fma(v, l2e_t, -c)) | bits of vt << 32, the largest
                            // logit of the chunk's possible candidates left out of its list (-inf: none)

@@ -34,11 +34,12 @@
 // release fence at agent scope would write back the whole L2 of each
 // workgroup's XCD, microseconds per workgroup.)
 //
-// A captured launch's replays carry one epoch, so a launch leaves no word
-// that would count in the next: a merging workgroup clears the tags (every
-// one has been stored by then; a workgroup that reads them later sees some
-// cleared and leaves the row to it), and chunk 0's workgroup clears the
-// row's word before it publishes.
+// A captured launch's replays carry one epoch, so such a launch (kFlagReplay)
+// leaves no word that would count in the next: a merging workgroup clears the
+// tags (every one has been stored by then; a workgroup that reads them later
+// sees some cleared and leaves the row to it), and chunk 0's workgroup clears
+// the row's word before it publishes.  Other launches have an epoch of their
+// own and leave these stores out (0.2 us of a row's chain of round trips).
 //
 //   m = max m_c; the normaliser's estimate sum_c s_c exp2(fma(m, -l2e_t,
 //   c_c)) (the chunk sums scaled to the row's maximum, as phase M scales
@@ -145,7 +146,7 @@ __device__ __forceinline__ bool split_chunk(const KArgs& A, int row, int c, Spli
   }
   // (complete before this chunk's tag is stored, so before any workgroup
   // takes the row)
-  if (c == 0 && t == 0) dev_st(&R.elect, 0ull);
+  if ((P.flags & kFlagReplay) != 0u && c == 0 && t == 0) dev_st(&R.elect, 0ull);
   if constexpr (XF) {
     const uint32_t xf = P.xf_src;
     // main.zig:653-666 on each logit of the row (positions past it stay -inf)
@@ -410,7 +411,7 @@ __device__ __forceinline__ bool split_merge(const KArgs& A, int row, SplitShared
     en[h] = dev_ld(&R.cand[i < nslots ? i : 0]);
   }
   // every tag has been stored: none is left for a replay
-  if (w == kSplitW - 1 && lane < ns) dev_st(&R.rec[lane].tag, 0ull);
+  if ((P.flags & kFlagReplay) != 0u && w == kSplitW - 1 && lane < ns) dev_st(&R.rec[lane].tag, 0ull);
   if (w == 0) {
     const bool on = lane < ns;
     float mc = ninf, cc = 0.0f, sc = 0.0f, vt = ninf, wc = 0.0f;
