@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kNT) void k_long(KArgs A) {
 
 // The token-only pass over many rows (see the head of the file): up to three
 // workgroups per CU, each claiming row after row; an undecided row's word in
-// Q.und becomes the call's tag.
+// Q.und becomes the call's tag, a decided row's its complement.
 template <bool FASTLD, int XM>
 __global__ __launch_bounds__(kNT, 4) void k_tok(KArgs A) {
   __shared__ LongShared F;
@@ -385,7 +385,9 @@ __global__ __launch_bounds__(kNT, 4) void k_tok(KArgs A) {
     bool nanrow;
     const bool done = tok_stream<FASTLD, XM, 4, true>(P, Q, row, F, pen_sh, X, m, nanrow);
     if (threadIdx.x == 0) {
-      if (!done) Q.und[row] = (uint32_t)P.epoch;
+      // (written for decided rows too: a replay of a captured launch carries
+      // the same tag, and would find the marks of every replay before it)
+      Q.und[row] = done ? ~(uint32_t)P.epoch : (uint32_t)P.epoch;
       next_row = claim_row(A.Q.claim, A.P.epoch, (int)gridDim.x, A.P.rows);
     }
     __syncthreads();

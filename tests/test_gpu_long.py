@@ -171,3 +171,37 @@ def test_replayed_calls_of_more_rows_than_cus(params, n):
         torch.cuda.synchronize()
         assert torch.equal(captured.result.tokens, want.tokens)
         assert torch.equal(captured.result.consumed, want.consumed)
+
+
+def test_replays_mark_undecided_rows_anew():
+    """k_tok's marks are one replay's own: rows left undecided by one replay
+    and decided by the next are not sampled a second time there."""
+    rows, n = 600, 20000
+    side = torch.cuda.Stream()
+    x = torch.empty(rows, n, device="cuda")
+    u = torch.rand(rows, device="cuda")
+    cfg = llz.SamplerConfig.of(FILTERS)
+    eager = llz.PreparedCall(rows, n, cfg, "cuda:0")
+    with torch.cuda.stream(side):
+        captured = llz.PreparedCall(rows, n, cfg, "cuda:0", stream=side)
+        x.normal_(0.0, 2.5)
+        captured(x, u)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured(x, u)
+    # the marks: the workspace's last section, padded to 256 bytes
+    marks = captured.workspace[-(-(-rows * 4 // 256) * 256):][:rows * 4].view(torch.int32)
+    hot = torch.empty(rows, n, device="cuda").normal_(0.0, 2.5)
+    flat = torch.full((rows, n), 0.5, device="cuda")  # every row's candidates overflow its buffers
+    half = torch.where(torch.arange(rows, device="cuda")[:, None] % 2 == 0, hot, flat)
+    tag = None
+    for logits, left in ((flat, rows), (hot, 0), (half, rows // 2), (hot, 0)):
+        x.copy_(logits)
+        torch.cuda.synchronize()
+        want = eager(x, u).tokens.clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured.result.tokens, want)
+        tag = marks[0].item() if tag is None else tag
+        assert left <= int((marks == tag).sum()) <= left + rows // 50  # (a few hot rows' cuts are too close to call)
