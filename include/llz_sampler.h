@@ -169,6 +169,10 @@ int llz_sample_rows_noalloc(const float *d_logits, int64_t row_stride, int32_t r
  * executeTopK / topk_bda.glsl (compute_graph.zig:948-984, which scales by
  * 1 / logit_scale at topk_bda.glsl:38-40), keeping the reference sampler's
  * tie-break: values that become equal after the scale keep the first index.
+ * Long rows are read by several workgroups, which combine through the row's
+ * token word when it lies in the stream's device's memory (until the call is
+ * done it may hold another chunk's index); tokens elsewhere (pinned or managed
+ * host memory) are stored once, by one workgroup per row.
  * Asynchronous on `stream`. */
 int llz_argmax_rows(const float *d_logits, int64_t row_stride, int32_t rows, int32_t vocab,
                     const llz_logit_post *post, uint32_t *d_tokens, void *stream);

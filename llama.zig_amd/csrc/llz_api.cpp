@@ -131,11 +131,9 @@ float candidate_theta(const llz_sampler_config* cfg, int32_t vocab) {
   return theta;
 }
 
-// The number of CUs of the device a stream runs on (cached per device; the
-// last stream's device is remembered per thread, since asking the runtime for
-// a stream's device costs more than a launch).
-int device_cus(hipStream_t st) {
-  static std::atomic<int> cache[64];
+// The device a stream runs on, or -1 (the last stream's is remembered per
+// thread, since asking the runtime for it costs more than a launch).
+int device_of(hipStream_t st) {
   thread_local hipStream_t last_st = nullptr;
   thread_local int last_dev = -1;
   int dev = 0;
@@ -148,6 +146,13 @@ int device_cus(hipStream_t st) {
   } else if (hipGetDevice(&dev) != hipSuccess) {
     return -1;
   }
+  return dev;
+}
+
+// The number of CUs of that device (cached per device), or -1.
+int device_cus(hipStream_t st) {
+  static std::atomic<int> cache[64];
+  const int dev = device_of(st);
   if (dev < 0 || dev >= 64) return -1;
   int c = cache[dev].load(std::memory_order_relaxed);
   if (c <= 0) {
@@ -155,6 +160,36 @@ int device_cus(hipStream_t st) {
     cache[dev].store(c, std::memory_order_relaxed);
   }
   return c;
+}
+
+// Where the caller's data lies: on a device (*dev: which), in host memory that
+// HIP knows (pinned or managed) or in the process's own.
+enum class Mem { kDevice, kHip, kHost };
+Mem mem_of(const void* p, int* dev = nullptr) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return Mem::kHost;
+  }
+  if (dev) *dev = a.device;
+  if (a.type == hipMemoryTypeUnregistered) return Mem::kHost;
+  return a.type == hipMemoryTypeDevice ? Mem::kDevice : Mem::kHip;
+}
+
+// Greedy rows.  Their chunks combine by compare-and-swap of the row's token
+// word, which only memory of the stream's own device is sure to serve (host
+// memory needs the bus's atomics): tokens that lie elsewhere are stored by
+// one workgroup per row.
+hipError_t greedy_rows(const float* d_logits, int64_t row_stride, int32_t rows, int32_t vocab, uint32_t xf, float cap,
+                       float inv, uint32_t* d_tokens, uint8_t* d_consumed, const llz_sample_extras* extras,
+                       hipStream_t st) {
+  int chunks = argmax_chunks(rows, vocab);
+  if (chunks > 1) {
+    int dev = -1;
+    if (mem_of(d_tokens, &dev) != Mem::kDevice || dev != device_of(st)) chunks = 1;
+  }
+  return launch_argmax(d_logits, row_stride, rows, vocab, chunks, xf, cap, inv, d_tokens, d_consumed,
+                       extras ? extras->d_kept_count : nullptr, extras ? extras->d_row_path : nullptr, st);
 }
 
 int check_common(const float* d_logits, int64_t row_stride, int32_t rows, int32_t vocab) {
@@ -206,8 +241,8 @@ int llz_argmax_rows(const float* d_logits, int64_t row_stride, int32_t rows, int
   const uint32_t xb = post_bits(post);
   // main.zig:664: the inverse is one f32 division
   const float inv = (xb & kXfScale) ? 1.0f / post->logit_scale : 1.0f;
-  hipError_t e = launch_argmax(d_logits, row_stride, rows, vocab, xb, post ? post->final_logit_softcapping : 0.0f,
-                               inv, d_tokens, nullptr, nullptr, nullptr, (hipStream_t)stream);
+  hipError_t e = greedy_rows(d_logits, row_stride, rows, vocab, xb, post ? post->final_logit_softcapping : 0.0f, inv,
+                             d_tokens, nullptr, nullptr, (hipStream_t)stream);
   return e == hipSuccess ? LLZ_OK : LLZ_E_HIP;
 }
 
@@ -237,9 +272,7 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
 
   // sampler.zig:50 -- greedy rows never draw
   if (cfg->temperature <= 0.0f) {
-    hipError_t e = launch_argmax(d_logits, row_stride, rows, vocab, xb, cap, inv, d_tokens, d_consumed,
-                                 extras ? extras->d_kept_count : nullptr, extras ? extras->d_row_path : nullptr,
-                                 st);
+    hipError_t e = greedy_rows(d_logits, row_stride, rows, vocab, xb, cap, inv, d_tokens, d_consumed, extras, st);
     return e == hipSuccess ? LLZ_OK : LLZ_E_HIP;
   }
   if (!d_uniforms) return LLZ_E_INVALID_ARG;
@@ -663,19 +696,6 @@ void llz_sampler_get_state(const llz_sampler* s, uint64_t state[4]) {
 
 void llz_sampler_set_state(llz_sampler* s, const uint64_t state[4]) {
   if (s && state) std::memcpy(s->prng, state, sizeof(s->prng));
-}
-
-// Where the caller's data lies: on the device, in host memory that HIP knows
-// (pinned or managed) or in the process's own.
-enum class Mem { kDevice, kHip, kHost };
-static Mem mem_of(const void* p) {
-  hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return Mem::kHost;
-  }
-  if (a.type == hipMemoryTypeUnregistered) return Mem::kHost;
-  return a.type == hipMemoryTypeDevice ? Mem::kDevice : Mem::kHip;
 }
 
 // One row through llz_sample_rows with the caller's uniform: token and the

@@ -174,7 +174,8 @@ constexpr int kStatsNT = 512;  // threads of its workgroups
 hipError_t launch_penalty(const float* logits, int64_t stride, int rows, int n, const uint32_t* prev,
                           int n_prev, int64_t prev_stride, int window, float penalty, uint32_t xf, float cap,
                           float inv_scale, float* out, hipStream_t st);
-hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, uint32_t xf, float cap,
+int argmax_chunks(int rows, int n);  // k_argmax: chunks per row
+hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, int chunks, uint32_t xf, float cap,
                          float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
                          uint32_t* path, hipStream_t st);
 hipError_t launch_stage(void* dst, const void* pinned, size_t units16, hipStream_t st);

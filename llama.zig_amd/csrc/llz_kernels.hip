@@ -60,7 +60,8 @@ __global__ __launch_bounds__(kMaxNT) void k_penalty(const float* __restrict__ lo
 // word, and while its own best beats the element the word names it swaps its
 // index in.  The word needs no initialisation: what an earlier call left
 // there is either not an index of the row (any element beats it) or names a
-// real element of it, which the row's best beats or equals.
+// real element of it, which the row's best beats or equals.  (Token words in
+// host memory take one chunk per row: stored, not exchanged over the bus.)
 //
 // Bound by HBM latency and launch: a workgroup per row with one 4-byte load
 // in flight per thread took 19.9 us for 32 x 50021 (0.32 TB/s); chunks of at
@@ -236,17 +237,25 @@ hipError_t launch_penalty(const float* logits, int64_t stride, int rows, int n, 
   return hipGetLastError();
 }
 
-hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, uint32_t xf, float cap,
-                         float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
-                         uint32_t* path, hipStream_t st) {
-  // chunks per row: as many as fill kArgGroups workgroups, none below kArgChunk logits
+// chunks per row: as many as fill kArgGroups workgroups, none below kArgChunk
+// logits but the last, and none empty
+static uint32_t argmax_per_chunk(int n, int chunks) {
+  return (((uint32_t)n + (uint32_t)chunks - 1) / (uint32_t)chunks + 3u) & ~3u;
+}
+
+int argmax_chunks(int rows, int n) {
   const uint32_t un = (uint32_t)n;
   const uint32_t most = (un + kArgChunk - 1) / kArgChunk;
   const uint32_t want = std::min(most, (uint32_t)std::max(1, kArgGroups / rows));
-  const uint32_t per = ((un + want - 1) / want + 3u) & ~3u;
-  const int chunks = (int)((un + per - 1) / per);
+  const uint32_t per = argmax_per_chunk(n, (int)want);
+  return (int)((un + per - 1) / per);
+}
+
+hipError_t launch_argmax(const float* logits, int64_t stride, int rows, int n, int chunks, uint32_t xf, float cap,
+                         float inv_scale, uint32_t* tokens, uint8_t* consumed, uint32_t* kept_count,
+                         uint32_t* path, hipStream_t st) {
   hipLaunchKernelGGL(k_argmax, dim3((unsigned)rows * (unsigned)chunks), dim3(kArgNT), 0, st, logits, stride, n, chunks,
-                     per, xf, cap, inv_scale, tokens, consumed, kept_count, path);
+                     argmax_per_chunk(n, chunks), xf, cap, inv_scale, tokens, consumed, kept_count, path);
   return hipGetLastError();
 }
 

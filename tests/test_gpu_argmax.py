@@ -60,3 +60,46 @@ def test_argmax_longest_rows(n):
     for at in (n - 1, n // 2):
         x[0, at] = x[0, at] + 2.0 + (n - at) * 1e-9
         assert _argmax(x, 0)[0] == at
+
+
+@pytest.mark.parametrize("rows,n", [(1, 50021), (3, 131075), (300, 8193)])
+def test_argmax_tokens_in_host_memory(rows, n):
+    """Tokens in pinned host memory are stored, not combined through the word
+    (argmax_rows and greedy rows of llz_sample_rows)."""
+    import llz
+
+    g = np.random.default_rng(n)
+    x = torch.from_numpy(g.integers(-40, 41, size=(rows, n)).astype(np.float32)).cuda()
+    want = np.array([O.lib().llz_oracle_argmax(O._fptr(r), n) for r in x.cpu().numpy()], np.uint32)
+    tok = torch.full((rows,), -1, dtype=torch.int32, pin_memory=True)
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    args = (C.c_void_p(x.data_ptr()), n, rows, n)
+    assert llz.library().llz_argmax_rows(*args, None, C.c_void_p(tok.data_ptr()), st) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(tok.numpy().view(np.uint32), want)
+    tok.fill_(n - 1)
+    cfg = llz.SamplerConfig(temperature=0.0).to_c()
+    assert llz.library().llz_sample_rows(*args, C.byref(cfg), None, None, 0, 0, None, C.c_void_p(tok.data_ptr()), None,
+                                         None, None, 0, st) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(tok.numpy().view(np.uint32), want)
+
+
+def test_argmax_replayed():
+    import llz
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.empty(8, 50021, device="cuda").normal_(0.0, 2.0, generator=g)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        llz.argmax_rows(x)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            tok = llz.argmax_rows(x)
+    for _ in range(4):
+        x.normal_(0.0, 2.0, generator=g)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(tok.long(), x.argmax(1))
