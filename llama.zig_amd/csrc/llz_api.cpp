@@ -706,9 +706,14 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
     return LLZ_E_INVALID_ARG;
   if (cfg->temperature != cfg->temperature) return LLZ_E_INVALID_ARG;
   if (hipSetDevice(s->device) != hipSuccess) return LLZ_E_HIP;
-  const size_t need_ws = llz_sample_workspace_bytes(1, n, cfg, n_prev);
-  if (n > s->cap_n || n_prev > s->cap_prev || need_ws > s->ws_bytes) {
-    const int32_t cn = std::max(n, s->cap_n), cp = std::max(n_prev, s->cap_prev);
+  // of the history, the ids that the penalty reads: its window
+  const int32_t win = cfg->temperature > 0.0f && penalty_active(cfg, n_prev) ? penalty_window(cfg, n_prev) : 0;
+  prev_tokens += n_prev - win;
+  const size_t need_ws = llz_sample_workspace_bytes(1, n, cfg, win);
+  if (n > s->cap_n || win > s->cap_prev || need_ws > s->ws_bytes) {
+    // (a window over the whole of a growing history: room for as many again)
+    const int32_t cn = std::max(n, s->cap_n);
+    const int32_t cp = win > s->cap_prev ? std::max(256, (int32_t)std::min<int64_t>((int64_t)win * 2, INT32_MAX)) : s->cap_prev;
     const size_t cw = std::max(need_ws, s->ws_bytes), st = Stage(cn, cp).total;
     sampler_free_buffers(s);
     if (hipHostMalloc((void**)&s->h_stage, st, hipHostMallocDefault) != hipSuccess ||
@@ -730,10 +735,10 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
   // Pinned and managed memory may still be written by work queued on the
   // default stream, which the sampler's stream waits for and the CPU does
   // not: copies on the sampler's stream read it, behind that work.
-  const Stage at(n, n_prev);
+  const Stage at(n, win);
   std::memcpy(s->h_stage, &u, sizeof(float));
-  const bool prev_cpu = n_prev > 0 && mem_of(prev_tokens) == Mem::kHost;
-  if (prev_cpu) std::memcpy(s->h_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t));
+  const bool prev_cpu = win > 0 && mem_of(prev_tokens) == Mem::kHost;
+  if (prev_cpu) std::memcpy(s->h_stage + at.prev, prev_tokens, (size_t)win * sizeof(uint32_t));
   const float* d_in = logits;
   const Mem where = mem_of(logits);
   const bool on_host = where == Mem::kHost;
@@ -754,16 +759,16 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
     from = upto;
   }
   // behind the staged head, which covers the history's place
-  if (n_prev > 0 && !prev_cpu &&
-      hipMemcpyAsync(s->d_stage + at.prev, prev_tokens, (size_t)n_prev * sizeof(uint32_t), hipMemcpyDefault,
+  if (win > 0 && !prev_cpu &&
+      hipMemcpyAsync(s->d_stage + at.prev, prev_tokens, (size_t)win * sizeof(uint32_t), hipMemcpyDefault,
                      s->stream) != hipSuccess)
     return LLZ_E_HIP;
   if (where == Mem::kHip &&
       hipMemcpyAsync(s->d_stage + at.logits, logits, bytes, hipMemcpyDefault, s->stream) != hipSuccess)
     return LLZ_E_HIP;
   const bool greedy = cfg->temperature <= 0.0f;
-  int rc = llz_sample_rows(d_in, n, 1, n, cfg, nullptr, n_prev > 0 ? (const uint32_t*)(s->d_stage + at.prev) : nullptr,
-                           n_prev, 0, (const float*)s->d_stage, greedy ? s->d_token : &s->h_out->token,
+  int rc = llz_sample_rows(d_in, n, 1, n, cfg, nullptr, win > 0 ? (const uint32_t*)(s->d_stage + at.prev) : nullptr,
+                           win, 0, (const float*)s->d_stage, greedy ? s->d_token : &s->h_out->token,
                            &s->h_out->consumed, nullptr, s->d_ws, s->ws_bytes, s->stream);
   if (rc != LLZ_OK) return rc;
   if (greedy && hipMemcpyAsync(&s->h_out->token, s->d_token, sizeof(uint32_t), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
