@@ -104,8 +104,9 @@ Layout layout_of(int32_t rows, int32_t vocab, const llz_sampler_config* cfg, int
   // last, so that a workspace without it holds every other part at the same
   // offsets: calls of at most kSplitRows rows, the split rows' chunk records
   L.split = off;   if (rows <= kSplitRows) off = align_up(off + r * sizeof(SplitRow));
-  // (or, for calls of more rows than a grid, k_tok's marks)
-  L.und = off;     if (rows > kMaxGrid) off = align_up(off + r * sizeof(uint32_t));
+  // (or, for calls of more rows than a grid, k_tok's undecided rows: their
+  // number, then the list)
+  L.und = off;     if (rows > kMaxGrid) off = align_up(off + kAlign + r * sizeof(uint32_t));
   L.total = off;
   return L;
 }
@@ -405,10 +406,6 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
         break;
       }
     }
-    // (the null stream cannot be captured)
-    hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
-    if (P.split_s > 0 && st && hipStreamIsCapturing(st, &cap_st) != hipSuccess) return LLZ_E_HIP;
-    if (cap_st != hipStreamCaptureStatusNone) P.flags |= kFlagReplay;
     // a chunk's possible candidates: d2 = (m_c - v) l2e_t < log2(1 / theta)
     // + 2^-8 (rounded up to a float)
     const double b = std::log2(1.0 / (double)P.tok_theta) + 0x1p-8;
@@ -442,15 +439,36 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
   Q.claim = (unsigned long long*)(ws + L.claim);
   Q.prev_win = (xf_src & kXfPen) ? d_prev_tokens + (n_prev - window) : nullptr;
   Q.split = P.split_s > 0 ? (SplitRow*)(ws + L.split) : nullptr;
-  // more rows than CUs, the token alone, rows the single pass could keep
+  // More rows than CUs, the token alone, rows the single pass could keep
   // resident and that are not soft-capped (their exact tanh is left to
-  // k_stats's estimates): k_tok decides what it can with two rows per CU
-  // (top-p alone over many rows stays with k_stats_rows: most of its rows
-  // need the exact normaliser, and the pass would be lost on them)
-  const bool ends = tok_minp || (cfg->top_k > 0 && cfg->top_k <= 128);
-  if (tok_only && ends && P.tok_theta > 0.0f && P.grid < rows && rows > kMaxGrid && workspace_bytes >= L.total &&
-      vocab <= kResidentMax && !(xf_src & kXfCap))
-    Q.und = (uint32_t*)(ws + L.und);
+  // k_stats's estimates): k_tok, two or three rows per CU at a time, decides
+  // what it can.  It is run where it pays for the rows it leaves, which
+  // k_stats_rows reads again behind it (us against k_stats_rows alone):
+  // - with a min-p of at least 2^-6: lower ones list more terms than it holds
+  //   (2048 x 128256, 0.002: 424 against 335), and without one most rows are
+  //   left (top-k and top-p: 587 against 427);
+  // - with typical-p only where that drops nothing, which is certain when it is
+  //   at least top-p (full chain, 300 to 4096 rows: 119 against 131 to 494
+  //   against 704; a typical-p of 0.5: 1519 against 1293);
+  // - without typical-p from 4 rounds of k_stats_rows on at 64k logits, and
+  //   more for longer rows: its tail of some 5 us per round is saved, one row's
+  //   exact phases (45 us at 32k logits, 100 at 128k) are added when any row is
+  //   left (1024 rows of 32000 and the filters chain 64 to 103 against 101 to
+  //   122, 4096 of 128256 457 to 470 against 543 to 558, but 512 of 128256 108
+  //   against 94 and 1024 of 128256 180 to 280 against 175 to 195).
+  const bool typ_none = typical_on && cfg->top_p > 0.0f && cfg->top_p < 1.0f && cfg->typical_p >= cfg->top_p;
+  const int64_t rounds = rows / std::max(1, P.grid);
+  const bool long_run = !typical_on && rounds * 16384 >= vocab;
+  if (tok_only && cfg->min_p >= 0x1p-6f && (typ_none || long_run) && P.grid < rows && rows > kMaxGrid &&
+      workspace_bytes >= L.total && vocab <= kResidentMax && !(xf_src & kXfCap)) {
+    Q.nund = (unsigned long long*)(ws + L.und);
+    Q.und = (uint32_t*)(ws + L.und + kAlign);
+  }
+  if ((Q.split || Q.und) && st) {  // (the null stream cannot be captured)
+    hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap_st) != hipSuccess) return LLZ_E_HIP;
+    if (cap_st != hipStreamCaptureStatusNone) P.flags |= kFlagReplay;
+  }
   e = launch_sample(P, Q, g_ev_begin, g_ev_end, st);
   if (e != hipSuccess) report_hip("llz_sample_rows: launch", e);
   return e == hipSuccess ? LLZ_OK : LLZ_E_HIP;

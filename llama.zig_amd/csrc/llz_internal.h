@@ -159,7 +159,8 @@ struct RowPtrs {
   uint32_t* qovf;         // [min(rows, kMaxGrid)][kQovfRow] k_stats special-queue overflow, per workgroup
   unsigned long long* claim;  // rows claimed beyond the grid: (epoch tag << 24) | count
   const uint32_t* prev_win;  // kXfPen: row 0's window (its last pen_w history tokens)
-  uint32_t* und;             // k_tok: [rows] the call's tag for the rows it leaves undecided, its complement for the others
+  uint32_t* und;             // k_tok: the rows it leaves undecided, in any order
+  unsigned long long* nund;  //   and how many: (epoch tag << 24) | count
   SplitRow* split;           // [rows] split rows' chunk summaries and lists
 };
 

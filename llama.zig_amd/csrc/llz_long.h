@@ -21,15 +21,16 @@
 // now.  Bound by one CU's share of HBM while
 // the rows are fewer than the CUs.
 //
-// Batches of more rows than CUs (token-only calls, rows the single pass could
-// keep resident) run the same stream in k_tok first: without the residency
-// and the selection stage a workgroup needs 45 KB of LDS and 80 VGPRs (98
-// transformed), so three share a CU (two) and one row's tail (re-reads, sort,
-// decisions: 20 us behind 18 us of loads in k_stats_rows) runs under the
-// others' loads.  Rows it does not
-// decide are marked and sampled by a k_stats_rows launch behind it.
-// 4096 rows of 128256 with every filter: 1043 us before, 516 now, 418 of them
-// k_tok (5.0 TB/s) and the rest some 7 marked rows.
+// Batches of more rows than CUs (token-only calls that the rule in
+// llz_api.cpp picks) run the same stream in k_tok first: without the residency
+// and the selection stage a workgroup needs 45 KB of LDS and 97 to 105 VGPRs,
+// so two share a CU (three where the registers allow) and one row's tail
+// (re-reads, sort, decisions: 20 us behind 18 us of loads in k_stats_rows)
+// runs under the others' loads.  Rows it does not decide are listed, and
+// sampled by a k_stats_rows launch behind it.
+// 4096 rows of 128256 with every filter: 705 us in k_stats_rows alone, 494 with
+// k_tok (4.2 TB/s; it takes 418 of them in the kernel trace, 5.0 TB/s, and the
+// rest is one listed row's exact phases).
 #pragma once
 
 #include "llz_fast.h"
@@ -367,8 +368,8 @@ __global__ __launch_bounds__(kNT) void k_long(KArgs A) {
 }
 
 // The token-only pass over many rows (see the head of the file): up to three
-// workgroups per CU, each claiming row after row; an undecided row's word in
-// Q.und becomes the call's tag, a decided row's its complement.
+// workgroups per CU, each claiming row after row; undecided rows go to the
+// list Q.und.
 template <bool FASTLD, int XM>
 __global__ __launch_bounds__(kNT, 4) void k_tok(KArgs A) {
   __shared__ LongShared F;
@@ -385,9 +386,10 @@ __global__ __launch_bounds__(kNT, 4) void k_tok(KArgs A) {
     bool nanrow;
     const bool done = tok_stream<FASTLD, XM, 4, true>(P, Q, row, F, pen_sh, X, m, nanrow);
     if (threadIdx.x == 0) {
-      // (written for decided rows too: a replay of a captured launch carries
-      // the same tag, and would find the marks of every replay before it)
-      Q.und[row] = done ? ~(uint32_t)P.epoch : (uint32_t)P.epoch;
+      if (!done) {
+        const int i = claim_row(Q.nund, P.epoch, 0, 0x7fffffff);  // (a count: k_stats_rows clears it)
+        if (i < P.rows) Q.und[i] = (uint32_t)row;
+      }
       next_row = claim_row(A.Q.claim, A.P.epoch, (int)gridDim.x, A.P.rows);
     }
     __syncthreads();

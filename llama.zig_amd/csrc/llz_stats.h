@@ -1910,28 +1910,33 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
   __shared__ StatsShared U;
   __shared__ PenShared pen_sh;
   __shared__ int next_row;
-  // behind k_tok: the rows it marked, this workgroup's share of them (grid
-  // rows apart, shifted from one stretch to the next so that rows of one
-  // parity do not all meet the same XCDs); usually none
-  const bool listed = A.Q.und != nullptr;
-  int i0 = 0;          // listed: stretches looked at so far
-  uint64_t marks = 0;  //   and those of the last 64 whose row is marked
-  auto next_listed = [&]() -> int {
-    const int g = A.P.grid, b = (int)blockIdx.x;
-    while (marks == 0ull && (int64_t)i0 * g < A.P.rows) {
-      const int i = i0 + lane_id();
-      const int64_t r = (int64_t)i * g + (b + i * 37) % g;
-      marks = bal64(r < A.P.rows && A.Q.und[r < A.P.rows ? r : 0] == (uint32_t)A.P.epoch);
-      i0 += kWave;
+  // behind k_tok: the rows it listed (often few or none), claimed one by one
+  const bool listed = A.Q.und != nullptr, replay = (A.P.flags & kFlagReplay) != 0u;
+  int nl = 0;  // listed: how many
+  auto next = [&]() -> int {  // thread 0
+    const int g = A.P.grid;
+    if (!listed) return claim_row(A.Q.claim, A.P.epoch, g, A.P.rows);
+    int i = nl;
+    if (replay) {
+      // from the first row on, nl + g claims in all (each workgroup is told
+      // once that none is left): the last one, when every workgroup has read
+      // the list's length, clears it, so that the next replay starts from an
+      // empty list.  (These claims cost a launch 7 us.)
+      i = claim_row(A.Q.claim, A.P.epoch, 0, nl + g);
+      if (i == nl + g - 1) __hip_atomic_store(A.Q.nund, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (nl > g) {
+      i = claim_row(A.Q.claim, A.P.epoch, g, nl);
     }
-    if (marks == 0ull) return A.P.rows;
-    const int i = i0 - kWave + __ffsll((long long)marks) - 1;
-    marks &= marks - 1ull;
-    return i * g + (b + i * 37) % g;
+    return i < nl ? (int)A.Q.und[i] : A.P.rows;
   };
   int row0 = (int)blockIdx.x;
   if (listed) {
-    row0 = __builtin_amdgcn_readfirstlane(next_listed());
+    const unsigned long long w = __hip_atomic_load(A.Q.nund, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr unsigned long long kCnt = (1ull << 24) - 1;
+    nl = (w & ~kCnt) == (A.P.epoch & ((1ull << 40) - 1)) << 24 ? min((int)(w & kCnt), A.P.rows) : 0;
+    if (threadIdx.x == 0) next_row = nl == 0 ? A.P.rows : replay ? next() : (row0 < nl ? (int)A.Q.und[row0] : A.P.rows);
+    __syncthreads();
+    row0 = next_row;
     if (row0 >= A.P.rows) return;
   }
   for (int row = row0;;) {
@@ -1942,9 +1947,9 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
         (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
     stats_row<FASTLD, XM, EXT>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
-    if (threadIdx.x == 0 && !listed) next_row = claim_row(A.Q.claim, A.P.epoch, A.P.grid, A.P.rows);
+    if (threadIdx.x == 0) next_row = next();
     __syncthreads();  // also: every wave is done with this row's shared memory
-    row = listed ? __builtin_amdgcn_readfirstlane(next_listed()) : next_row;
+    row = next_row;
     if (row >= A.P.rows) return;
   }
 }

@@ -143,8 +143,8 @@ def _oracle_rows(x, p, u, prev):
     return tok, con, kept, None
 
 
-@pytest.mark.parametrize("params,n", [(FILTERS, 20000), (DEFAULT, 20000), (FILTERS, 131076)],
-                         ids=["k_tok", "claimed rows", "claimed long rows"])
+@pytest.mark.parametrize("params,n", [(FILTERS, 20000), (FULL, 20000), (DEFAULT, 20000), (FILTERS, 131076)],
+                         ids=["token rows", "k_tok", "claimed rows", "claimed long rows"])
 def test_replayed_calls_of_more_rows_than_cus(params, n):
     """A captured call's replays carry one epoch: every replay samples every
     row of the logits it finds, also beyond the grid."""
@@ -173,14 +173,14 @@ def test_replayed_calls_of_more_rows_than_cus(params, n):
         assert torch.equal(captured.result.consumed, want.consumed)
 
 
-def test_replays_mark_undecided_rows_anew():
-    """k_tok's marks are one replay's own: rows left undecided by one replay
-    and decided by the next are not sampled a second time there."""
-    rows, n = 600, 20000
+def test_replays_list_undecided_rows_anew():
+    """k_tok's list of undecided rows is one replay's own: rows left undecided
+    by one replay and decided by the next are not sampled a second time."""
+    rows, n = 600, 20000  # (every filter: k_tok's call at any number of rows)
     side = torch.cuda.Stream()
     x = torch.empty(rows, n, device="cuda")
     u = torch.rand(rows, device="cuda")
-    cfg = llz.SamplerConfig.of(FILTERS)
+    cfg = llz.SamplerConfig.of(FULL)
     eager = llz.PreparedCall(rows, n, cfg, "cuda:0")
     with torch.cuda.stream(side):
         captured = llz.PreparedCall(rows, n, cfg, "cuda:0", stream=side)
@@ -190,18 +190,45 @@ def test_replays_mark_undecided_rows_anew():
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=side):
             captured(x, u)
-    # the marks: the workspace's last section, padded to 256 bytes
-    marks = captured.workspace[-(-(-rows * 4 // 256) * 256):][:rows * 4].view(torch.int32)
+    # the workspace's last section: the list's length, then (256 bytes on) the list
+    section = captured.workspace[-(-(-(256 + rows * 4) // 256) * 256):]
+    length, rows_listed = section[:8].view(torch.int64), section[256:256 + rows * 4].view(torch.int32)
     hot = torch.empty(rows, n, device="cuda").normal_(0.0, 2.5)
     flat = torch.full((rows, n), 0.5, device="cuda")  # every row's candidates overflow its buffers
     half = torch.where(torch.arange(rows, device="cuda")[:, None] % 2 == 0, hot, flat)
-    tag = None
-    for logits, left in ((flat, rows), (hot, 0), (half, rows // 2), (hot, 0)):
+    for logits, left in ((flat, rows), (hot, 0), (half, rows // 2), (hot, 0), (flat, rows)):
         x.copy_(logits)
+        rows_listed.fill_(-1)
         torch.cuda.synchronize()
         want = eager(x, u).tokens.clone()
+        captured.result.tokens.fill_(-5)
+        torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(captured.result.tokens, want)
-        tag = marks[0].item() if tag is None else tag
-        assert left <= int((marks == tag).sum()) <= left + rows // 50  # (a few hot rows' cuts are too close to call)
+        assert length.item() == 0
+        listed = rows_listed[rows_listed >= 0].sort().values
+        assert torch.equal(listed, listed.unique())
+        assert left <= listed.numel() <= left + rows // 50  # (a few hot rows' cuts are too close to call)
+
+
+@pytest.mark.parametrize("n,pad", [(4096, 0), (9001, 2)])
+def test_many_rows_without_typical(n, pad):
+    """k_tok's calls without typical-p: eight rounds of rows and more."""
+    rows = 8 * 256 + 37
+    g = np.random.default_rng(n)
+    base = np.concatenate([_rows(n, 6), g.normal(0.0, 2.0, size=(40, n)).astype(np.float32)])
+    x = base[g.integers(0, base.shape[0], rows)]
+    u = llz.rng_uniforms(3, rows)
+    prev = g.integers(0, n, size=(rows, 32)).astype(np.uint32)
+    for window in (0, 32):
+        p = dataclasses.replace(FILTERS, repetition_window=window, repetition_penalty=1.2 if window else 1.0)
+        flat = torch.empty(rows, n + pad, dtype=torch.float32, device="cuda")
+        flat[:, :n].copy_(torch.from_numpy(x))
+        r = llz.sample_rows(flat[:, :n], llz.SamplerConfig.of(p), torch.from_numpy(u).cuda(),
+                            torch.from_numpy(prev.astype(np.int32)).cuda(), kept_cap=8, probs=False)
+        torch.cuda.synchronize()
+        tok, con, kc, _ = _oracle_rows(x, p, u, prev)
+        assert np.array_equal(r.tokens.cpu().numpy().view(np.uint32), tok)
+        assert np.array_equal(r.consumed.cpu().numpy(), con)
+        assert np.array_equal(r.kept_count.cpu().numpy().view(np.uint32), kc)
