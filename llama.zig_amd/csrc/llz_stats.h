@@ -1261,7 +1261,10 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   {
     const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
     const bool topk = P.top_k > 0u && P.top_k <= (uint32_t)kCandCap / 2u;
-    if (fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f) {
+    // (the hint is for the register allocator: without it the search's live
+    // values spilled in the phases around it, 3 us of a 512-row call of
+    // k_stats_rows that never comes here)
+    if (__builtin_expect(fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f, 0)) {
       const float Rw = __builtin_amdgcn_exp2f(fmaf(m, -l2e_t, cw));
       const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
       // e: log2 of the threshold tried; below e_lo the terms do not fit the
