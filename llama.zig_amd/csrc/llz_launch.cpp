@@ -80,7 +80,8 @@ extern "C" int llz_stamps_9(unsigned long long*, int, int);
 extern "C" int llz_stamps_10(unsigned long long*, int, int);
 
 // Measurement builds: the phase timestamps of rows 0 .. rows - 1 (kStampSlots
-// per row, 0 where a row did not reach the boundary) into dst.
+// per row, 0 where a row did not reach the boundary) into dst.  A row that
+// k_tok (the last object) left to k_stats_rows has the latter's.
 extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int clear) {
   if (rows <= 0 || rows > llz::kStampRows || !dst) return -1;
   static int (*const get[])(unsigned long long*, int, int) = {llz_stamps_0, llz_stamps_1, llz_stamps_2, llz_stamps_3,
@@ -93,8 +94,12 @@ extern "C" int llz_debug_phase_stamps(unsigned long long* dst, int rows, int cle
   for (auto f : get) {
     const int rc = f(part, rows, clear);
     if (rc != 0) return rc;
-    if (!clear)
-      for (size_t i = 0; i < n; ++i) dst[i] |= part[i];  // one object ran each row
+    if (clear) continue;
+    for (int r = 0; r < rows; ++r) {
+      unsigned long long* to = dst + (size_t)r * llz::kStampSlots;
+      if (f == llz_stamps_10 && to[0] != 0) continue;
+      for (int k = 0; k < llz::kStampSlots; ++k) to[k] |= part[(size_t)r * llz::kStampSlots + k];  // (one other object ran it)
+    }
   }
   return 0;
 }

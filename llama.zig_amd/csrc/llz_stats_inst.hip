@@ -47,7 +47,8 @@ StatsKernel LLZ_CAT(stats_kernel_, LLZ_INST)(int a, int b) {
 
 #ifdef LLZ_PHASE_STAMPS
 // Measurement builds: this object's phase timestamps (each object has its
-// own copy of the array; one call's rows are all in one).
+// own copy of the array; a call's rows are all in one, but for k_tok's pass
+// over rows that another object then samples).
 extern "C" int LLZ_CAT(llz_stamps_, LLZ_INST)(unsigned long long* dst, int rows, int clear) {
   const size_t bytes = (size_t)rows * llz::kStampSlots * sizeof(unsigned long long);
   if (clear) {
