@@ -118,3 +118,51 @@ def test_bucket_path_duplicate_keys(cuda):
     u = llz.rng_uniforms(5, rows)
     g = _run(cuda, x, params, u)
     _check_oracle(x, params, u, g)
+
+
+def _tie_row(n, lo, hi, share, seed):
+    """A near-flat row in which a share of the terms of ranks lo .. hi - 1 (in
+    (p desc, id asc) order) are ties where the running sum meets them: half a
+    unit of its last place."""
+    g = np.random.default_rng(seed)
+    x = g.normal(0.0, 0.3, n).astype(np.float32)
+    x -= x.max()  # the maximum is 0, so the terms are exp(x)
+    S = np.cumsum(O.expf_array(x), dtype=np.float32)[-1]
+    p = O.expf_array(x) / S
+    order = np.lexsort((np.arange(n), -p))
+    ranks = np.arange(lo, hi)[g.random(hi - lo) < share]
+    ids = order[ranks]
+    # the sum's unit is 2^s units of p: a tie's last s bits are 10..0
+    run = np.cumsum(p[order], dtype=np.float32)[ranks]
+    s = (np.frexp(run)[1] - np.frexp(p[ids])[1]).astype(np.int64)
+    want = ((p[ids].view(np.uint32).astype(np.int64) & ~((1 << s) - 1)) | (1 << (s - 1))).astype(np.uint32)
+    near = np.log(want.view(np.float32).astype(np.float64) * float(S)).astype(np.float32)
+    open_ = np.ones(ids.size, bool)
+    for d in range(-12, 13):  # the logit whose p it is, if there is one
+        v = (near.view(np.int32) + d).view(np.float32)
+        hit = open_ & (v < 0) & ((O.expf_array(v) / S).view(np.uint32) == want)
+        x[ids[hit]] = v[hit]
+        open_ &= ~hit
+    # the last logit takes up what the normaliser lost
+    rest = np.cumsum(O.expf_array(x)[:-1], dtype=np.float32)[-1]
+    x[-1] = np.float32(np.log(float(S) - float(rest)))
+    assert np.cumsum(O.expf_array(x), dtype=np.float32)[-1] == S
+    return x, int(np.sum(~open_))
+
+
+@pytest.mark.parametrize("lo,hi,share,least", [
+    (1000, 2000, 0.2, 100),    # some hundred tied buckets: gathered by class, more than 64 runs to order
+    (1000, 1100, 0.02, 0),     # about as many as a row has anyway, gathered by their key ranges
+    (8200, 16300, 0.6, 3500),  # more elements in tied buckets than the list holds: batches
+], ids=["many", "few", "batches"])
+def test_bucket_path_ties(cuda, lo, hi, share, least):
+    made = [_tie_row(70001, lo, hi, share, seed) for seed in range(4)]
+    assert all(k >= least for _, k in made)
+    x = np.stack([r for r, _ in made])
+    params = Params(temperature=1.0, top_k=0, top_p=0.9, min_p=0.0, typical_p=1.0, repetition_window=0,
+                    repetition_penalty=1.0)
+    for u in (0.02, 0.3, 0.97):
+        uu = np.full(4, u, np.float32)
+        g = _run(cuda, x, params, uu)
+        assert np.all(g["path"] & llz.PATH_BUCKETS), g["path"]
+        _check_oracle(x, params, uu, g)

@@ -36,6 +36,13 @@ def _rows(n, seed):
     return x
 
 
+def _same(a, b):
+    """Bit for bit, any NaN like any other."""
+    a, b = np.atleast_1d(np.asarray(a, np.float32)), np.atleast_1d(np.asarray(b, np.float32))
+    nan = np.isnan(a)
+    return np.array_equal(nan, np.isnan(b)) and np.array_equal(a[~nan].view(np.uint32), b[~nan].view(np.uint32))
+
+
 def _check(x, params, *, post=None, prev=None, offset=0, pad=0, exact=False):
     rows, n = x.shape
     u = llz.rng_uniforms(5, rows)
@@ -59,6 +66,11 @@ def _check(x, params, *, post=None, prev=None, offset=0, pad=0, exact=False):
         assert (tok[i], con[i], kc[i]) == (o.token, o.consumed, o.kept_count), ctx
         k = min(o.kept_count, 64)
         assert np.array_equal(ids[i, :k], o.kept_ids()[:k]), ctx
+        if exact:
+            st, pr = r.row_stats[i].cpu().numpy(), r.kept_probs[i, :k].cpu().numpy()
+            assert _same(st[[0, 1, 3]], [o.max_logit, o.sum, o.total]), ctx
+            assert st[2] == 0.0 or _same(st[2], o.entropy), ctx
+            assert _same(pr, o.probs[ids[i, :k]]), ctx
     return r.row_path.cpu().numpy().view(np.uint32)
 
 

@@ -21,9 +21,10 @@ DEFAULT = Params(0.8, 0, 0.9, 0.0, 1.0, 0, 1.0)
 
 
 def _same(a, b):
-    a, b = np.asarray(a, np.float32), np.asarray(b, np.float32)
-    return np.array_equal(a.view(np.uint32)[~np.isnan(a)], b.view(np.uint32)[~np.isnan(b)]) and \
-        np.array_equal(np.isnan(a), np.isnan(b))
+    """Bit for bit, any NaN like any other."""
+    a, b = np.atleast_1d(np.asarray(a, np.float32)), np.atleast_1d(np.asarray(b, np.float32))
+    nan = np.isnan(a)
+    return np.array_equal(nan, np.isnan(b)) and np.array_equal(a[~nan].view(np.uint32), b[~nan].view(np.uint32))
 
 
 def _check(x, params, *, post=None, offset=0, exact=False):
@@ -46,7 +47,8 @@ def _check(x, params, *, post=None, offset=0, exact=False):
         assert np.array_equal(ids[i, :k], o.kept_ids()[:k]), ctx
         if exact:
             st = r.row_stats[i].cpu().numpy()
-            assert _same(st[:2], [o.max_logit, o.sum]) and _same(st[3], o.total), ctx
+            assert _same(st[[0, 1, 3]], [o.max_logit, o.sum, o.total]), ctx
+            assert st[2] == 0.0 or _same(st[2], o.entropy), ctx
             assert _same(r.kept_probs[i, :k].cpu().numpy(), o.probs[ids[i, :k]]), ctx
 
 
