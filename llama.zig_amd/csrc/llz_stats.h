@@ -513,7 +513,8 @@ union StatsShared {
 // read through post-processing and/or the fused repetition penalty
 // (llz_xform.h); otherwise as they are.
 // wslot: the workgroup's block of the special-queue overflow area.
-template <bool FASTLD, int XM, bool EXT = false>
+// ROWS: one of several rows of a workgroup (k_stats_rows).
+template <bool FASTLD, int XM, bool EXT = false, bool ROWS = false>
 __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& U, PenShared& pen_sh, int wslot) {
   constexpr bool XF = XM != kXmNone;
   const RowParams P = A.P;
@@ -1261,10 +1262,13 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   {
     const bool topp = P.top_p > 0.0f && P.top_p < 1.0f;
     const bool topk = P.top_k > 0u && P.top_k <= (uint32_t)kCandCap / 2u;
+    const bool search = fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f;
     // (the hint is for the register allocator: without it the search's live
     // values spilled in the phases around it, 3 us of a 512-row call of
-    // k_stats_rows that never comes here)
-    if (__builtin_expect(fits && P.cand_theta < 0x1p-10f && (topp || topk) && fabsf(m) <= 3.0e38f, 0)) {
+    // k_stats_rows that never comes here; in the other instantiations it has
+    // them spill more)
+    constexpr bool kRare = ROWS && XM != kXmCap && !EXT;
+    if (kRare ? __builtin_expect(search, 0) : search) {
       const float Rw = __builtin_amdgcn_exp2f(fmaf(m, -l2e_t, cw));
       const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
       // e: log2 of the threshold tried; below e_lo the terms do not fit the
@@ -1949,7 +1953,7 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
     const __attribute__((address_space(4))) KArgs* Ap =
         (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
-    stats_row<FASTLD, XM, EXT>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
+    stats_row<FASTLD, XM, EXT, true>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
     if (threadIdx.x == 0) next_row = next();
     __syncthreads();  // also: every wave is done with this row's shared memory
     row = next_row;
