@@ -450,16 +450,16 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
   // - with typical-p only where that drops nothing, which is certain when it is
   //   at least top-p (full chain, 300 to 4096 rows: 119 against 131 to 494
   //   against 704; a typical-p of 0.5: 1519 against 1293);
-  // - without typical-p from 4 rounds of k_stats_rows on at 64k logits, and
-  //   more for longer rows: its tail of some 5 us per round is saved, one row's
-  //   exact phases (45 us at 32k logits, 100 at 128k) are added when any row is
-  //   left (1024 rows of 32000 and the filters chain 64 to 103 against 101 to
-  //   122, 4096 of 128256 457 to 470 against 543 to 558, but 512 of 128256 108
-  //   against 94 and 1024 of 128256 180 to 280 against 175 to 195).
+  // - without typical-p up to 64k logits, or from 8 rounds of k_stats_rows on:
+  //   its tail of some 5 us per round is saved, one row's exact phases (45 us
+  //   at 32k logits, 100 at 128k) are added when any row is left (means over
+  //   eight batches of the filters chain: 300 rows of 32000 30 to 64 against 48
+  //   to 69, 512 of 64000 48 to 82 against 66 to 90, 4096 of 128256 457 to 470
+  //   against 543 to 558; but 300 of 128256 60 to 101 against 72 to 89, 1024 of
+  //   128256 165 to 183 against 161 to 181).
   const bool typ_none = typical_on && cfg->top_p > 0.0f && cfg->top_p < 1.0f && cfg->typical_p >= cfg->top_p;
-  const int64_t rounds = rows / std::max(1, P.grid);
-  const bool long_run = !typical_on && rounds * 16384 >= vocab;
-  if (tok_only && cfg->min_p >= 0x1p-6f && (typ_none || long_run) && P.grid < rows && rows > kMaxGrid &&
+  const bool pays = !typical_on && (vocab <= 65536 || rows / std::max(1, P.grid) >= 8);
+  if (tok_only && cfg->min_p >= 0x1p-6f && (typ_none || pays) && P.grid < rows && rows > kMaxGrid &&
       workspace_bytes >= L.total && vocab <= kResidentMax && !(xf_src & kXfCap)) {
     Q.nund = (unsigned long long*)(ws + L.und);
     Q.und = (uint32_t*)(ws + L.und + kAlign);
