@@ -1007,6 +1007,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // estimate does (estimates are within 2^-16 of the terms, and no term
   // exceeds its segment's sum), re-read and evaluated exactly; the list lies
   // in F.v, free once every wave has read the segment sums below.
+  int first_pass = 0;  // the threshold 2^-10 in the search below: 1 holds, -1 does not, 0 not known
   if (tok && !nanrow && fabsf(m) <= 3.0e38f && P.tok_theta > 0.0f) {
     LLZ_STAMP(row, 38);
     float s_est = 0.0f, w_est = 0.0f;
@@ -1071,7 +1072,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       if (tq < 0) tq = tqueue(Rw_t, thr_e);
       LLZ_STAMP(row, 39);
       LLZ_STAMP(row, 32);
-      if (tq > QCAP && lane == 0) atomicOr(&F.tfail, 1u);
+      if (tq > QCAP && lane == 0) atomicOr(&F.tfail, 2u);  // the list is not complete
       // The queued lanes' elements that may be candidates: the lane test
       // (tqueue against the row's maximum) element by element, on the same
       // estimates exp2(fma(v, l2e_t, -cw)) phase L computed.  When a wave
@@ -1223,7 +1224,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
           }
         }
       } else if (t == 0) {
-        F.tfail = 1u;
+        F.tfail |= 1u;
       }
       // LDS only: the outputs' global stores need not land before the
       // workgroup ends
@@ -1232,8 +1233,19 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
         LLZ_STAMP(row, 15);
         return;
       }
-      // not certified: the exact phases, with the segment sums the list
-      // overwrote written again (F.qpos is rewritten in phase S)
+      // not certified: the exact phases.  A complete list above 2^-10 answers
+      // the threshold search's first pass (below)
+      if (theta_t == P.tok_theta && P.tok_theta > P.cand_theta && tc <= kTokCap && F.tfail == 1u) {
+        float ls = 0.0f;
+        for (int i = lane; i < tc; i += kWave) ls += __uint_as_float(~(uint32_t)(tl[i] >> 32));
+        ls = wave_sum_f32(ls);
+        const bool holds = (P.top_p > 0.0f && P.top_p < 1.0f && ls >= P.top_p * s_est * (1.0f + 0x1p-7f)) ||
+                           (P.top_k > 0u && P.top_k <= (uint32_t)kCandCap / 2u && (uint32_t)tc > P.top_k);
+        first_pass = holds ? 1 : -1;
+        __syncthreads();
+      }
+      // the segment sums the list overwrote are written again (F.qpos is
+      // rewritten in phase S)
       if (lane < nseg_w) F.v.aseg[w + W * lane] = my_a;
       __syncthreads();
     }
@@ -1255,8 +1267,9 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
   // terms than top-k keeps: the kept prefix then ends inside the list, and
   // the selection's certified prefix checks that it does.  2^-10 serves most
   // rows; otherwise it is searched from there, one pass over the resident
-  // estimates per threshold (3.4 us).  When some threshold's terms neither
-  // fit nor hold it, none does: the row floods at once.
+  // estimates per threshold (3.4 us; 2^-10's is left out where the token
+  // path's list has told of it).  When some threshold's terms neither fit nor
+  // hold it, none does: the row floods at once.
   float theta_c = P.cand_theta;
   bool flood_c = false;
   {
@@ -1273,9 +1286,11 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
       const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
       // e: log2 of the threshold tried; below e_lo the terms do not fit the
       // list, above e_hi they do not hold the prefix
-      float e = -10.0f, e_hi = 0.0f, e_lo = -kInfS;
+      // (the token path's list, where it is complete, has told of 2^-10)
+      float e = first_pass < 0 ? -13.0f : -10.0f, e_hi = first_pass < 0 ? -10.0f : 0.0f, e_lo = -kInfS;
+      if (first_pass > 0) theta_c = 0x1p-10f;
       const float e_min = __builtin_amdgcn_logf(P.cand_theta) + 0.5f;
-      for (int pass = 0; pass < 6; ++pass) {
+      for (int pass = first_pass > 0 ? 6 : 0; pass < 6; ++pass) {
         const float th = __builtin_amdgcn_exp2f(e);
         const float tq_lo = th * (1.0f + 0x1p-9f) / Rw;
         float ms = 0.0f;
