@@ -285,12 +285,15 @@ def run_workload(line: str, steps: int, warmup: int, args) -> dict:
     # (rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE, scaled by a device copy),
     # not measured by this run
     traffic = None
-    kernel = "k_split" if path_fracs["split"] >= 0.5 else "k_stats"
-    traffic_src = os.path.join("profiles", f"{kernel}_{line}_traffic.json")
-    if vocab > 129024 and kernel == "k_stats":
+    if path_fracs["split"] >= 0.5:
+        kernel = "k_split"
+    elif vocab > 129024:
         kernel = "k_long"  # rows beyond the single pass
-    elif line == "c5":
+    elif rows > 256 and path_fracs["token_only"] >= 0.5:
         kernel = "k_tok + k_stats_rows"  # the streaming pass, then the rows it leaves
+    else:
+        kernel = "k_stats" if rows <= 256 else "k_stats_rows"
+    traffic_src = os.path.join("profiles", f"{kernel.split(' ')[0]}_{line}_traffic.json")
     if os.path.exists(os.path.join(ROOT, traffic_src)):
         with open(os.path.join(ROOT, traffic_src)) as f:
             traffic = json.load(f).get("hbm_bytes_per_launch")

@@ -748,8 +748,9 @@ static int sampler_run(llz_sampler* s, const llz_sampler_config* cfg, const floa
   }
   // The inputs through pinned memory, read by a copy kernel on the sampler's
   // stream; the results written by the sampling kernel into pinned memory.
-  // (Pageable copies of the logits, the history and the uniform, and two
-  // more for the results, took 81 us of a call alone and 148 us back to back.)
+  // Pageable copies of the logits, the history and the uniform, and two more
+  // for the results, took 77 us per call of 128256 logits from one buffer, 85
+  // from 512 buffers in turn and 119 over a growing history; 53, 58 and 53 now.
   // Pinned and managed memory may still be written by work queued on the
   // default stream, which the sampler's stream waits for and the CPU does
   // not: copies on the sampler's stream read it, behind that work.

@@ -141,7 +141,7 @@ __device__ __forceinline__ void key_pass(const uint32_t* Kp, int n, Body body) {
       });
 }
 
-// RN(e / S) for 2^-90 <= e <= 1 and 2^-20 <= S <= 2^40 from y = RN(1 / S), by
+// RN(e / S) for 2^-90 <= e <= 1 and 2^-20 <= S <= 2^20 from y = RN(1 / S), by
 // Markstein's method (llz_math.h): the first correction makes the quotient
 // faithful, and the second, from a faithful quotient and the correctly
 // rounded reciprocal, rounds correctly; remainders are exact in an fma, and

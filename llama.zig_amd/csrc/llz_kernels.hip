@@ -64,9 +64,10 @@ __global__ __launch_bounds__(kMaxNT) void k_penalty(const float* __restrict__ lo
 // host memory take one chunk per row: stored, not exchanged over the bus.)
 //
 // Bound by HBM latency and launch: a workgroup per row with one 4-byte load
-// in flight per thread took 19.9 us for 32 x 50021 (0.32 TB/s); chunks of at
-// least kArgChunk logits over up to kArgGroups workgroups, four 16-byte loads
-// in flight per thread, take 10.5 us of kernel where that took 21.3 (traced).
+// in flight per thread took 19.8 us per call of 32 x 50021, back to back;
+// chunks of at least kArgChunk logits over up to kArgGroups workgroups, four
+// 16-byte loads in flight per thread, take 9.9 (the kernel alone under the
+// profiler, which lengthens both: 21.3 and 10.6).
 // ---------------------------------------------------------------------------
 constexpr int kArgNT = 256;
 constexpr int kArgUnroll = 4;                            // float4 loads in flight per thread

@@ -1534,7 +1534,7 @@ __device__ bool select_buckets(const Src& X, int n, float m, float S, float u, c
     constexpr int TV = RowTiles8::V;
     const RowTiles8 rt(X.x, n);
     const float T = P.temperature, yS = 1.0f / S;
-    const bool s_in = S >= 0x1p-20f && S <= 0x1p40f;
+    const bool s_in = S >= 0x1p-20f && S <= 0x1p20f;  // (div_by's range; S <= n < 2^20)
     pipelined_tiles<kNT, TV, 3, float>(
         n, [&](int pos, float (&r)[TV]) { rt.load(pos, r); },
         [&](int pos, float (&raw)[TV]) {

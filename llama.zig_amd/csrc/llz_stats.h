@@ -46,7 +46,7 @@ __device__ __forceinline__ llz_f4v to_v4(float4 f) {
 
 __device__ __forceinline__ float4 neg_inf4() { return make_float4(-kInfS, -kInfS, -kInfS, -kInfS); }
 
-// Branch-free 16-byte reads of a row (llz_rowops.h's rd4): FASTLD: 16-byte
+// Branch-free 16-byte reads of a row (llz_rowops.h's rd4_any). FASTLD: 16-byte
 // aligned rows with n % 4 == 0, else any row.
 template <bool FASTLD>
 __device__ __forceinline__ float4 rd4(const float* xr, int pos, int n) {
