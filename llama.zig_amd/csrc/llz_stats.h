@@ -513,8 +513,9 @@ union StatsShared {
 // read through post-processing and/or the fused repetition penalty
 // (llz_xform.h); otherwise as they are.
 // wslot: the workgroup's block of the special-queue overflow area.
-// ROWS: one of several rows of a workgroup (k_stats_rows).
-template <bool FASTLD, int XM, bool EXT = false, bool ROWS = false>
+// KIND: the kernel.
+enum : int { kOneRow, kManyRows, kSplitRow };  // k_stats, k_stats_rows, k_split
+template <bool FASTLD, int XM, bool EXT = false, int KIND = kOneRow>
 __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& U, PenShared& pen_sh, int wslot) {
   constexpr bool XF = XM != kXmNone;
   const RowParams P = A.P;
@@ -1234,8 +1235,11 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
         return;
       }
       // not certified: the exact phases.  A complete list above 2^-10 answers
-      // the threshold search's first pass (below)
-      if (theta_t == P.tok_theta && P.tok_theta > P.cand_theta && tc <= kTokCap && F.tfail == 1u) {
+      // the threshold search's first pass (below; not in the plain and the
+      // soft-capped k_stats, which it cost more in spills than it saved: 0.1 us
+      // of 256 headline rows, 11 of 53 capped rows with every filter)
+      constexpr bool kFirst = !(KIND == kOneRow && ((XM == kXmNone && FASTLD) || XM == kXmCap));
+      if (kFirst && theta_t == P.tok_theta && P.tok_theta > P.cand_theta && tc <= kTokCap && F.tfail == 1u) {
         float ls = 0.0f;
         for (int i = lane; i < tc; i += kWave) ls += __uint_as_float(~(uint32_t)(tl[i] >> 32));
         ls = wave_sum_f32(ls);
@@ -1280,7 +1284,7 @@ __device__ __forceinline__ void stats_row(const KArgs& A, int row, StatsShared& 
     // values spilled in the phases around it, 3 us of a 512-row call of
     // k_stats_rows that never comes here; in the other instantiations it has
     // them spill more)
-    constexpr bool kRare = ROWS && XM != kXmCap && !EXT;
+    constexpr bool kRare = KIND == kManyRows && XM != kXmCap && !EXT;
     if (kRare ? __builtin_expect(search, 0) : search) {
       const float Rw = __builtin_amdgcn_exp2f(fmaf(m, -l2e_t, cw));
       const float tot = wave_fold_f32(lane < nseg_w ? my_a : 0.0f) * Rw;
@@ -1968,7 +1972,7 @@ __global__ __launch_bounds__(NT) void k_stats_rows(KArgs A) {
     const __attribute__((address_space(4))) KArgs* Ap =
         (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
-    stats_row<FASTLD, XM, EXT, true>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
+    stats_row<FASTLD, XM, EXT, kManyRows>(*(const KArgs*)Ap, row, U, pen_sh, (int)blockIdx.x);
     if (threadIdx.x == 0) next_row = next();
     __syncthreads();  // also: every wave is done with this row's shared memory
     row = next_row;
@@ -2002,7 +2006,7 @@ __global__ __launch_bounds__(NT) void k_split(KArgs A) {
   const __attribute__((address_space(4))) KArgs* Ap =
       (const __attribute__((address_space(4))) KArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(Ap));
-  stats_row<FASTLD, XM>(*(const KArgs*)Ap, row, U.stats, pen_sh, row);
+  stats_row<FASTLD, XM, false, kSplitRow>(*(const KArgs*)Ap, row, U.stats, pen_sh, row);
 }
 
 }  // namespace
