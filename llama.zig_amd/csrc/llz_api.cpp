@@ -456,9 +456,12 @@ static int sample_rows_impl(const float* d_logits, int64_t row_stride, int32_t r
   //   eight batches of the filters chain: 300 rows of 32000 30 to 64 against 48
   //   to 69, 512 of 64000 48 to 82 against 66 to 90, 4096 of 128256 457 to 470
   //   against 543 to 558; but 300 of 128256 60 to 101 against 72 to 89, 1024 of
-  //   128256 165 to 183 against 161 to 181).
+  //   128256 165 to 183 against 161 to 181); with a scale or a penalty, which
+  //   leave it two workgroups per CU, up to 32k logits (1024 of 64000 with a
+  //   penalty: 174 to 208 against 148 to 179).
   const bool typ_none = typical_on && cfg->top_p > 0.0f && cfg->top_p < 1.0f && cfg->typical_p >= cfg->top_p;
-  const bool pays = !typical_on && (vocab <= 65536 || rows / std::max(1, P.grid) >= 8);
+  const bool plain = (xf_src | xb) == 0u;
+  const bool pays = !typical_on && (vocab <= (plain ? 65536 : 32768) || (plain && rows / std::max(1, P.grid) >= 8));
   if (tok_only && cfg->min_p >= 0x1p-6f && (typ_none || pays) && P.grid < rows && rows > kMaxGrid &&
       workspace_bytes >= L.total && vocab <= kResidentMax && !(xf_src & kXfCap)) {
     Q.nund = (unsigned long long*)(ws + L.und);
