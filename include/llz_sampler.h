@@ -133,7 +133,8 @@ size_t llz_sample_workspace_bytes(int32_t rows, int32_t vocab, const llz_sampler
  *                  may be NULL when n_prev == 0.
  *   d_uniforms:    [rows] the value random.float(f32) would return at
  *                  sampler.zig:162 for that row.
- *   d_tokens:      [rows] sampled TokenID (sampler.zig's return value).
+ *   d_tokens:      [rows] sampled TokenID (sampler.zig's return value); greedy
+ *                  rows (temperature <= 0) write it as llz_argmax_rows does.
  *   d_consumed:    [rows] 1 when the row reached the draw (sampler.zig:162)
  *                  and so consumed its uniform, 0 on the early exits
  *                  (temperature <= 0, sum <= 0, empty kept set).  May be NULL.
