@@ -742,6 +742,13 @@ __device__ __noinline__ NormResult select_norm_fallback(const KArgs* A, int row,
   if (threadIdx.x == 0) shl.cand_count = 0;
   NormResult r;
   r.S = row_normaliser(X, P.n, P, shl, bank, r.m, m_known);
+  if (P.temperature > 3.402823466e38f) {
+    // an infinite temperature: a -inf logit's argument is -inf / inf = NaN,
+    // which the roundings above do not carry
+    bool neg = false;
+    for (int i = (int)threadIdx.x; i < P.n; i += kNT) neg = neg || X.at(i) == -kInf;
+    if (wg_max_u32<kNT>(neg ? 1u : 0u, shl.wg, bank) != 0u) r.S = __builtin_nanf("");
+  }
   r.bank = bank;
   return r;
 }

@@ -81,9 +81,12 @@ def test_long_rows_low_masks(n, offset, low, t, scale, exact):
 
 @pytest.mark.parametrize("n", [129028, 151937])
 def test_long_rows_infinite_temperature(n):
-    x = np.random.default_rng(n).normal(0.0, 2.0, size=(2, n)).astype(np.float32)
+    x = np.random.default_rng(n).normal(0.0, 2.0, size=(3, n)).astype(np.float32)
+    x[1, n // 2] = -np.inf  # (-inf - max) / inf: NaN, in the reference too
+    x[2, 3] = -np.inf
     for p in (FILTERS, DEFAULT):
-        _check(x, dataclasses.replace(p, temperature=float("inf")))
+        for exact in (False, True):
+            _check(x, dataclasses.replace(p, temperature=float("inf")), exact=exact)
 
 
 @pytest.mark.parametrize("exact", [False, True], ids=["token", "exact"])
@@ -106,7 +109,7 @@ def test_resident_rows_low_masks(n, offset, low, t, scale, exact):
            post=llz.LogitPost(0.0, scale) if scale != 1.0 else None, offset=offset, exact=exact)
 
 
-@pytest.mark.parametrize("n", [5, 2049, 4100, 129021, 129024])
+@pytest.mark.parametrize("n", [5, 1000, 2048, 2049, 4100, 129021, 129024])
 def test_resident_rows_infinite_temperature(n):
     x = np.random.default_rng(n).normal(0.0, 2.0, size=(3, n)).astype(np.float32)
     x[2, n // 2] = -np.inf  # (-inf - max) / inf: NaN, in the reference too
